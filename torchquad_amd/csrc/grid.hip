@@ -384,6 +384,9 @@ static int launch_grid(const tq_grid_desc* gd, const tq_integrand* f, const void
 // ---------------------------------------------------------------------------
 // Point writer (user integrands)
 // ---------------------------------------------------------------------------
+// Any grid: one point per thread, coordinates stored one by one.  Used for
+// more than 2^31 points, more axes than the staged writer's LDS holds and
+// unaligned outputs.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_grid_points(const T* domain, int d, int n, int rule,
                                                         const double* glx, long long P, T* pts) {
@@ -400,6 +403,95 @@ __global__ __launch_bounds__(kBlock) void k_grid_points(const T* domain, int d, 
             row[k] = (T)node_of(s_axis[k], j, n, rule, glx);
         }
     }
+}
+
+// Staged writer (write_stage): bound by the HBM writes of the points.  A
+// point costs one multiply-high per axis for its digits and, with NODES, a
+// read of the axis's node from an LDS table (else the node is formed where
+// it is used).
+constexpr size_t kNodeTableMax = 16 * 1024;
+
+template <typename T, bool NODES, int PPL>
+__global__ __launch_bounds__(kBlock) void k_grid_points_staged(const T* domain, int d, FastDiv by_n, int rule,
+                                                               const double* glx, uint32_t P, uint32_t chunks,
+                                                               T* pts) {
+    extern __shared__ __align__(16) unsigned char s_raw[];
+    __shared__ Axis s_axis[kMaxDimPoints];
+    const int n = (int)by_n.n;
+    for (int k = threadIdx.x; k < d; k += kBlock) s_axis[k] = make_axis(domain, k, n, rule);
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
+    constexpr int C = kWave * PPL;
+    T* slice = reinterpret_cast<T*>(s_raw) + (size_t)wave * C * d;
+    T* node = reinterpret_cast<T*>(s_raw) + (size_t)kWavesPerBlock * C * d;
+    if (NODES) {
+        for (int e = threadIdx.x; e < d * n; e += kBlock) {
+            const int k = (int)by_n.div((uint32_t)e);
+            node[e] = (T)node_of(s_axis[k], e - k * n, n, rule, glx);
+        }
+        __syncthreads();
+    }
+    const uint32_t stride = gridDim.x * kWavesPerBlock;
+    for (uint32_t c = blockIdx.x * kWavesPerBlock + wave; c < chunks; c += stride) {
+        const uint32_t first = c * C;
+        const uint32_t left = P - first;
+        const int points = left < (uint32_t)C ? (int)left : C;
+        uint32_t r[PPL];
+#pragma unroll
+        for (int i = 0; i < PPL; ++i) {
+            const int o = lane + kWave * i;
+            r[i] = first + (uint32_t)(o < points ? o : 0);  // lanes past the end repeat a point that exists
+        }
+        for (int k = d - 1; k >= 0; --k) {
+#pragma unroll
+            for (int i = 0; i < PPL; ++i) {
+                const uint32_t q = by_n.div(r[i]);
+                const int j = (int)(r[i] - q * by_n.n);
+                r[i] = q;
+                slice[(lane + kWave * i) * d + k] =
+                    NODES ? node[k * n + j] : (T)node_of(s_axis[k], j, n, rule, glx);
+            }
+        }
+        wave_lds_fence();
+        write_stage<T>(slice, pts, (long long)first, points, C, d);
+        wave_lds_fence();  // the slice is read before the next chunk overwrites it
+    }
+}
+
+template <typename T, int PPL>
+static void launch_points_staged(const tq_grid_desc* g, const void* domain, long long P, void* points,
+                                 hipStream_t st) {
+    const FastDiv by_n = make_fast_div((uint32_t)g->n);
+    const size_t nodes = (size_t)g->dim * g->n * sizeof(T);
+    const bool table = nodes <= kNodeTableMax;
+    const size_t lds = stage_bytes(g->dim, sizeof(T)) * kWavesPerBlock + (table ? nodes : 0);
+    const uint32_t chunks = (uint32_t)((P + kWave * PPL - 1) / (kWave * PPL));
+    // as many blocks as there is work for, at most 8 per CU: each builds the
+    // node table once and then walks its chunks
+    long long blocks = ((long long)chunks + kWavesPerBlock - 1) / kWavesPerBlock;
+    if (blocks > 2048) blocks = 2048;
+    if (table)
+        hipLaunchKernelGGL((k_grid_points_staged<T, true, PPL>), dim3((unsigned)blocks), dim3(kBlock), lds, st,
+                           (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points);
+    else
+        hipLaunchKernelGGL((k_grid_points_staged<T, false, PPL>), dim3((unsigned)blocks), dim3(kBlock), lds, st,
+                           (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points);
+}
+
+template <typename T>
+static int launch_points(const tq_grid_desc* g, const void* domain, long long P, void* points, hipStream_t st) {
+    if (P <= 0x7fffffffLL && stage_fits(g->dim, sizeof(T), points)) {
+        if (stage_ppl(g->dim, sizeof(T)) > 1)
+            launch_points_staged<T, 16 / (int)sizeof(T)>(g, domain, P, points, st);
+        else
+            launch_points_staged<T, 1>(g, domain, P, points, st);
+        return check_launch("k_grid_points_staged");
+    }
+    long long blocks = (P + kBlock - 1) / kBlock;
+    if (blocks > 65536) blocks = 65536;
+    hipLaunchKernelGGL((k_grid_points<T>), dim3((unsigned)blocks), dim3(kBlock), 0, st, (const T*)domain, g->dim,
+                       g->n, g->rule, g->gl_nodes, P, (T*)points);
+    return check_launch("k_grid_points");
 }
 
 template <typename T>
@@ -756,16 +848,8 @@ int tq_grid_points(const tq_grid_desc* g, const void* domain, void* points, void
     if (!domain || !points) return fail(TQ_E_NULL, "domain/points is NULL");
     long long P;
     ipow_checked(g->n, g->dim, 1LL << 62, &P);
-    long long blocks = (P + kBlock - 1) / kBlock;
-    if (blocks > 65536) blocks = 65536;
-    if (blocks < 1) blocks = 1;
-    if (g->dtype == TQ_F32)
-        hipLaunchKernelGGL((k_grid_points<float>), dim3((unsigned)blocks), dim3(kBlock), 0, as_stream(stream),
-                           (const float*)domain, g->dim, g->n, g->rule, g->gl_nodes, P, (float*)points);
-    else
-        hipLaunchKernelGGL((k_grid_points<double>), dim3((unsigned)blocks), dim3(kBlock), 0, as_stream(stream),
-                           (const double*)domain, g->dim, g->n, g->rule, g->gl_nodes, P, (double*)points);
-    return check_launch("k_grid_points");
+    if (g->dtype == TQ_F32) return launch_points<float>(g, domain, P, points, as_stream(stream));
+    return launch_points<double>(g, domain, P, points, as_stream(stream));
 }
 
 int tq_grid_h(const tq_grid_desc* g, const void* domain, void* h_out, void* stream) {

@@ -39,6 +39,67 @@ __device__ inline double block_sum(double v, double* smem /* [kWavesPerBlock] */
     return r;
 }
 
+// Division of r < 2^31 by a divisor n that is fixed for a launch, as a
+// multiply-high and a shift instead of the 30-odd instructions of an integer
+// division.  With l = ceil(log2 n) and m = ceil(2^(31+l) / n) < 2^32,
+// floor(r m / 2^(31+l)) = floor(r / n): the excess r (m n - 2^(31+l)) /
+// (n 2^(31+l)) is below r / 2^(31+l) < 2^-l <= 1 / n.
+struct FastDiv {
+    uint32_t n, m, sh;
+    __device__ inline uint32_t div(uint32_t r) const { return n == 1u ? r : __umulhi(r, m) >> sh; }
+};
+
+inline FastDiv make_fast_div(uint32_t n) {
+    FastDiv f{n, 1u, 0u};
+    if (n > 1u) {
+        uint32_t l = 0;
+        while ((1ull << l) < n) ++l;
+        f.sh = l - 1u;
+        f.m = (uint32_t)(((1ull << (31 + l)) + n - 1ull) / n);
+    }
+    return f;
+}
+
+// LDS writes of the calling wave become visible to all of its lanes.
+__device__ inline void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// Point writers ([P, d] row-major).  A lane that stored its point's d
+// coordinates itself would touch 64 separate d-element rows per store
+// instruction.  Instead each wave puts a chunk of 64 ppl points into its own
+// LDS slice and writes the slice out in 16-byte pieces, consecutive lanes at
+// consecutive addresses (5 axes, 6.9e7 FP32 points: 530 us with lane-strided
+// 4-byte stores and 64-bit index divisions, 237 us or 5.8 TB/s of writes so).
+constexpr size_t kStageMax = 40 * 1024;  // LDS of a block's slices
+
+// Points per lane and chunk: 16 bytes of each coordinate while four slices stay small, else one point.
+inline int stage_ppl(int d, int tsize) { return d <= 8 ? 16 / tsize : 1; }
+inline size_t stage_bytes(int d, int tsize) { return (size_t)kWave * stage_ppl(d, tsize) * d * tsize; }
+inline bool stage_fits(int d, int tsize, const void* out) {
+    return stage_bytes(d, tsize) * kWavesPerBlock <= kStageMax && ((uintptr_t)out & 15) == 0;
+}
+
+// Writes the wave's slice (`points` rows of d values) to out + first * d.  first is a multiple of
+// 64, so a slice starts 16-byte aligned when `out` does.
+template <typename T>
+__device__ inline void write_stage(const T* slice, T* out, long long first, int points, int full, int d) {
+    constexpr int V = 16 / (int)sizeof(T);
+    using V4 = __attribute__((ext_vector_type(4))) uint32_t;
+    const int lane = threadIdx.x & (kWave - 1);
+    T* dst = out + first * d;
+    if (points == full) {
+        const V4* s4 = reinterpret_cast<const V4*>(slice);
+        V4* d4 = reinterpret_cast<V4*>(dst);
+        const int nv = full * d / V;
+        for (int e = lane; e < nv; e += kWave) d4[e] = s4[e];
+    } else {
+        for (int e = lane; e < points * d; e += kWave) dst[e] = slice[e];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Philox-4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers: as
 // easy as 1, 2, 3", SC'11).  Ten rounds of two 32x32->64 multiplies with the
