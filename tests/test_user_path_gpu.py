@@ -68,3 +68,68 @@ def test_mc_points_staged(d, N, dtype, dev):
     assert torch.equal(pts, other.view(N, d))
     lo, hi = dom[:, 0], dom[:, 1]
     assert bool(((pts >= lo) & (pts <= hi)).all())
+
+
+# (dim, n, S): one value per load and four, rows that four values cross, one
+# axis longer than the weight table, every S class and its edges
+VALUES = [(1, 5, 1), (1, 257, 1), (1, 2049, 1), (1, 100001, 1), (2, 45, 1), (2, 49, 1), (3, 101, 1), (5, 9, 1),
+          (8, 5, 1), (2, 2501, 1), (3, 9, 2), (2, 33, 3), (4, 5, 31), (2, 65, 63), (1, 2305, 7), (1, 101, 64),
+          (2, 17, 65), (1, 10001, 200), (3, 13, 130), (1, 1, 1)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rule", ["trapezoid", "boole", "gauss_legendre", "unit"])
+@pytest.mark.parametrize("d,n,S", VALUES)
+def test_grid_reduce_sizes(d, n, S, rule, dtype, dev):
+    unit = rule == "unit"
+    if unit:
+        rule = "gauss_legendre"
+    if rule == "boole":
+        n = max(5, n - (n - 1) % 4)
+    if rule == "trapezoid":
+        n = max(2, n)
+    dom = _box(d, dtype, dev, n)
+    gl = gauss_legendre(n, device=dev) if rule == "gauss_legendre" else None
+    gen = torch.Generator(device=dev).manual_seed(d * 1000 + n + S)
+    vals = torch.rand((n**d, S), dtype=dtype, device=dev, generator=gen) - 0.25
+    got = _ops.grid_reduce(_ops.RULES[rule], d, n, dom, vals, unit_weights=unit, gl=gl)
+    # an unaligned copy takes one value per load
+    other = _unaligned(vals.numel(), dtype, dev)
+    other.copy_(vals.reshape(-1))
+    got2 = _ops.grid_reduce(_ops.RULES[rule], d, n, dom, other.view(n**d, S), unit_weights=unit, gl=gl)
+    b = dom.double().cpu().numpy()
+    if unit:
+        w, scale = np.ones(n), np.prod(0.5 * (b[:, 1] - b[:, 0]))
+    elif gl is not None:
+        w, scale = gl[1].cpu().numpy(), np.prod(0.5 * (b[:, 1] - b[:, 0]))
+    elif rule == "trapezoid":
+        w, scale = np.r_[1.0, np.full(n - 2, 2.0), 1.0], np.prod((b[:, 1] - b[:, 0]) / (n - 1) / 2.0)
+    else:
+        w, scale = np.full(n, 14.0), np.prod((b[:, 1] - b[:, 0]) / (n - 1) / 22.5)
+        w[1::2], w[2::4], w[0], w[-1] = 32.0, 12.0, 7.0, 7.0
+    W = torch.tensor(w, device=dev)
+    full = W
+    for _ in range(d - 1):
+        full = (full[:, None] * W[None, :]).reshape(-1)
+    ref = torch.sum(full[:, None] * vals.double(), dim=0) * scale
+    bar = float(torch.max(torch.sum(full[:, None].abs() * vals.double().abs(), dim=0))) * abs(scale)
+    # FP64 sums, one rounding of the result; N <= 6.3e6 terms of relative error 2^-53 each, at worst in one direction
+    tol = bar * (2.0**-24 if dtype == torch.float32 else 0.0) + bar * vals.shape[0] * 2.0**-53
+    assert float((got.double() - ref).abs().max()) <= tol
+    assert float((got2.double() - ref).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("N,S", [(1, 1), (255, 1), (1024, 1), (1025, 1), (3000001, 1), (1000, 2), (777, 63), (100, 64),
+                                 (4097, 65), (10, 1000)])
+def test_mc_reduce_sizes(N, S, dtype, dev):
+    dom = _box(3, dtype, dev, N)
+    gen = torch.Generator(device=dev).manual_seed(N + S)
+    vals = torch.rand((N, S), dtype=dtype, device=dev, generator=gen) - 0.25
+    other = _unaligned(vals.numel(), dtype, dev)
+    other.copy_(vals.reshape(-1))
+    vol = float(torch.prod(dom.double()[:, 1] - dom.double()[:, 0]))
+    ref = torch.mean(vals.double(), dim=0) * vol
+    tol = vol * ((2.0**-24 if dtype == torch.float32 else 0.0) + N * 2.0**-53)
+    for v in (vals, other.view(N, S)):
+        assert float((_ops.mc_reduce(v, dom).double() - ref).abs().max()) <= tol

@@ -17,6 +17,7 @@
 
 #include "tq_host.hpp"
 #include "tq_grid_tile.hpp"
+#include "tq_values.hpp"
 
 namespace tq {
 
@@ -505,117 +506,8 @@ __global__ void k_grid_h(const T* domain, int d, int n, int rule, const double* 
 }
 
 // ---------------------------------------------------------------------------
-// Weighted reduction of user values f[P, S]
-// Lanes enumerate (inner point over the last m axes, component s); the wave
-// walks the outer index with an odometer; reads are coalesced.
+// Weighted reduction of user values f[P, S] (kernels in tq_values.hpp)
 // ---------------------------------------------------------------------------
-struct ReduceGeom {
-    int d, n, m, rule;
-    long long S;
-    long long inner;       // n^m
-    long long lane_elems;  // inner*S
-    long long lane_waves;
-    long long outer;       // n^(d-m)
-    long long ipw;
-    long long chunks;
-    long long num_waves;
-    long long blocks;
-};
-
-static int make_reduce_geom(const tq_grid_desc* gd, long long S, ReduceGeom& R) {
-    const int d = gd->dim, n = gd->n;
-    R.d = d;
-    R.n = n;
-    R.rule = gd->rule;
-    R.S = S;
-    int m = d;
-    long long c = 1;
-    for (int k = 1; k <= d; ++k) {
-        c *= n;
-        if (c * S >= 64) {
-            m = k;
-            break;
-        }
-    }
-    if (m > d) m = d;
-    long long inner;
-    ipow_checked(n, m, 1LL << 62, &inner);
-    R.m = m;
-    R.inner = inner;
-    R.lane_elems = inner * S;
-    R.lane_waves = (R.lane_elems + kWave - 1) / kWave;
-    long long outer;
-    ipow_checked(n, d - m, 1LL << 62, &outer);
-    R.outer = outer;
-    const long long target_waves = 16384;
-    long long ipw = (outer * R.lane_waves + target_waves - 1) / target_waves;
-    if (ipw < 16) ipw = outer < 16 ? outer : 16;
-    if (ipw < 1) ipw = 1;
-    while (((outer + ipw - 1) / ipw) * R.lane_waves > (1LL << 30)) ipw *= 2;
-    R.ipw = ipw;
-    R.chunks = (outer + ipw - 1) / ipw;
-    R.num_waves = R.chunks * R.lane_waves;
-    R.blocks = (R.num_waves + kWavesPerBlock - 1) / kWavesPerBlock;
-    return TQ_OK;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_grid_reduce(ReduceGeom R, const T* fv, const double* glw,
-                                                        double* partials /* [blocks][S] */) {
-    __shared__ double s_acc[kBlock];
-    __shared__ long long s_comp[kBlock];
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const long long wave = (long long)blockIdx.x * kWavesPerBlock + (tid >> 6);
-    const int n = R.n, d = R.d, m = R.m, rule = R.rule;
-    double acc = 0.0;
-    long long comp = -1;
-    if (wave < R.num_waves) {
-        const long long lw = wave % R.lane_waves;
-        const long long chunk = wave / R.lane_waves;
-        const long long e = lw * kWave + lane;
-        if (e < R.lane_elems) {
-            comp = e % R.S;
-            long long rem = e / R.S;
-            double w_in = 1.0;
-            for (int k = d - 1; k >= d - m; --k) {
-                const int j = (int)(rem % n);
-                rem /= n;
-                w_in *= weight_of(rule, j, n, glw);
-            }
-            const long long o0 = chunk * R.ipw;
-            const long long o1 = (o0 + R.ipw < R.outer) ? (o0 + R.ipw) : R.outer;
-            int odig[kMaxDimPoints];
-            const int no = d - m;
-            {
-                long long r = o0;
-                for (int k = no - 1; k >= 0; --k) {
-                    odig[k] = (int)(r % n);
-                    r /= n;
-                }
-            }
-            const long long stride = R.lane_elems;
-            for (long long o = o0; o < o1; ++o) {
-                double w = w_in;
-                for (int k = 0; k < no; ++k) w *= weight_of(rule, odig[k], n, glw);
-                acc = fma(w, (double)fv[o * stride + e], acc);
-                for (int k = no - 1; k >= 0; --k) {
-                    if (++odig[k] < n) break;
-                    odig[k] = 0;
-                }
-            }
-        }
-    }
-    s_acc[tid] = acc;
-    s_comp[tid] = comp;
-    __syncthreads();
-    for (long long s = tid; s < R.S; s += blockDim.x) {
-        double v = 0.0;
-        for (int i = 0; i < (int)blockDim.x; ++i)
-            if (s_comp[i] == s) v += s_acc[i];
-        partials[(long long)blockIdx.x * R.S + s] = v;
-    }
-}
-
 // Scale of the weighted reduction: Newton-Cotes uses the caller's mesh
 // widths when given (hs[k]/c as _apply_composite_rule does), otherwise the
 // domain's; Gauss-Legendre uses (b-a)/2 per axis.
@@ -637,15 +529,18 @@ __device__ inline double reduce_scale(const T* domain, const T* hs, int d, int n
 }
 
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_grid_reduce_finalize(const double* partials, long long blocks,
-                                                                 long long S, const T* domain, const T* hs,
-                                                                 int unit, int d, int n, int rule, T* out) {
-    __shared__ double s_red[kWavesPerBlock];
-    const long long s = blockIdx.x;
-    double v = 0.0;
-    for (long long b = threadIdx.x; b < blocks; b += blockDim.x) v += partials[b * S + s];
-    v = block_sum(v, s_red);
-    if (threadIdx.x == 0) out[s] = (T)(v * reduce_scale(domain, hs, d, n, rule, unit));
+struct GridScale {
+    const T* domain;
+    const T* hs;
+    int d, n, rule, unit;
+    __device__ double operator()() const { return reduce_scale(domain, hs, d, n, rule, unit); }
+};
+
+// Plan of the reduction; unit weights: every point weighs 1.
+static int plan_reduce(const tq_grid_desc* g, long long S, int unit, ValuePlan& V) {
+    long long P;
+    ipow_checked(g->n, g->dim, 1LL << 62, &P);
+    return plan_values(unit ? 0 : g->dim, g->n, g->rule, g->gl_weights, P, S, g->dtype == TQ_F32 ? 4 : 8, V);
 }
 
 // grad_f[p, s] = grad_out[s] * scale * W(p)
@@ -870,9 +765,9 @@ int tq_grid_h(const tq_grid_desc* g, const void* domain, void* h_out, void* stre
 
 size_t tq_grid_reduce_workspace_size(const tq_grid_desc* g, int64_t S) {
     if (check_grid_desc(g, kMaxDimPoints) || S < 1) return 0;
-    ReduceGeom R;
-    make_reduce_geom(g, S, R);
-    return (size_t)(R.blocks * S) * sizeof(double);
+    ValuePlan V;  // the same partial count with and without unit weights
+    if (plan_reduce(g, S, 0, V)) return 0;
+    return values_workspace(V);
 }
 
 int tq_grid_reduce(const tq_grid_desc* g, const void* domain, const void* hs, int32_t unit_weights,
@@ -886,34 +781,20 @@ int tq_grid_reduce(const tq_grid_desc* g, const void* domain, const void* hs, in
     }
     if (S < 1) return fail(TQ_E_ARG, "S must be >= 1");
     if (!domain || !fvals || !out) return fail(TQ_E_NULL, "domain/fvals/out is NULL");
-    ReduceGeom R;
-    make_reduce_geom(g, S, R);
-    if (R.S > 65535) return fail(TQ_E_UNSUPPORTED, "more than 65535 integrand components");
-    const size_t need = (size_t)(R.blocks * S) * sizeof(double);
-    if (!workspace || workspace_bytes < need) return fail(TQ_E_WORKSPACE, "reduce workspace too small");
-    // unit weights: every point has weight 1 (the reduce kernel still runs the
-    // rule's pattern, so route through the Gauss-Legendre branch with ones).
-    if (unit_weights) R.rule = -1;
-    hipStream_t st = as_stream(stream);
+    if (S > 65535) return fail(TQ_E_UNSUPPORTED, "more than 65535 integrand components");
     const int unit = unit_weights ? 1 : 0;
-    if (g->dtype == TQ_F32) {
-        hipLaunchKernelGGL((k_grid_reduce<float>), dim3((unsigned)R.blocks), dim3(kBlock), 0, st, R,
-                           (const float*)fvals, g->gl_weights, (double*)workspace);
-        rc = check_launch("k_grid_reduce");
-        if (rc) return rc;
-        hipLaunchKernelGGL((k_grid_reduce_finalize<float>), dim3((unsigned)S), dim3(kBlock), 0, st,
-                           (const double*)workspace, R.blocks, (long long)S, (const float*)domain,
-                           (const float*)hs, unit, g->dim, g->n, g->rule, (float*)out);
-    } else {
-        hipLaunchKernelGGL((k_grid_reduce<double>), dim3((unsigned)R.blocks), dim3(kBlock), 0, st, R,
-                           (const double*)fvals, g->gl_weights, (double*)workspace);
-        rc = check_launch("k_grid_reduce");
-        if (rc) return rc;
-        hipLaunchKernelGGL((k_grid_reduce_finalize<double>), dim3((unsigned)S), dim3(kBlock), 0, st,
-                           (const double*)workspace, R.blocks, (long long)S, (const double*)domain,
-                           (const double*)hs, unit, g->dim, g->n, g->rule, (double*)out);
-    }
-    return check_launch("k_grid_reduce_finalize");
+    ValuePlan V;
+    rc = plan_reduce(g, S, unit, V);
+    if (rc) return rc;
+    if (!workspace || workspace_bytes < values_workspace(V)) return fail(TQ_E_WORKSPACE, "reduce workspace too small");
+    hipStream_t st = as_stream(stream);
+    if (g->dtype == TQ_F32)
+        return launch_values<float>(V, (const float*)fvals, (double*)workspace,
+                                    GridScale<float>{(const float*)domain, (const float*)hs, g->dim, g->n, g->rule, unit},
+                                    (float*)out, st);
+    return launch_values<double>(V, (const double*)fvals, (double*)workspace,
+                                 GridScale<double>{(const double*)domain, (const double*)hs, g->dim, g->n, g->rule, unit},
+                                 (double*)out, st);
 }
 
 int tq_grid_reduce_backward(const tq_grid_desc* g, const void* domain, const void* hs, int32_t unit_weights,

@@ -2,6 +2,7 @@
 // reduction of (sum f, sum f^2).  No sample ever touches HBM on the fused
 // path; the point writer produces the identical stream for user integrands.
 #include "tq_host.hpp"
+#include "tq_values.hpp"
 
 namespace tq {
 
@@ -193,53 +194,18 @@ __global__ __launch_bounds__(kBlock) void k_uniform(uint64_t seed, uint64_t offs
     }
 }
 
-// Column sums of f[N, S].  Narrow S: each thread keeps one fixed column
-// (block size is a multiple of S).  Wide S: one thread per column, rows
-// split over blockIdx.y.
+// Mean of user values f[N, S]: the kernels of tq_values.hpp with unit weights.
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_colsum_narrow(const T* fv, long long N, long long S,
-                                                          double* partials /* [blocks][S] */) {
-    __shared__ double s_acc[kBlock];
-    const long long bd = blockDim.x;
-    const long long total = N * S;
-    const long long stride = (long long)gridDim.x * bd;
-    double acc = 0.0;
-    for (long long e = (long long)blockIdx.x * bd + threadIdx.x; e < total; e += stride) acc += (double)fv[e];
-    s_acc[threadIdx.x] = acc;
-    __syncthreads();
-    if (threadIdx.x < S) {
-        double v = 0.0;
-        for (long long i = threadIdx.x; i < bd; i += S) v += s_acc[i];
-        partials[(long long)blockIdx.x * S + threadIdx.x] = v;
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_colsum_wide(const T* fv, long long N, long long S, long long rpb,
-                                                        double* partials /* [gridDim.y][S] */) {
-    const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= S) return;
-    const long long r0 = (long long)blockIdx.y * rpb;
-    const long long r1 = (r0 + rpb < N) ? (r0 + rpb) : N;
-    double acc = 0.0;
-    for (long long r = r0; r < r1; ++r) acc += (double)fv[r * S + s];
-    partials[(long long)blockIdx.y * S + s] = acc;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_colsum_finalize(const double* partials, long long nb, long long S,
-                                                            const T* domain, int d, long long N, T* out) {
-    __shared__ double s_red[kWavesPerBlock];
-    const long long s = blockIdx.x;
-    double v = 0.0;
-    for (long long b = threadIdx.x; b < nb; b += blockDim.x) v += partials[b * S + s];
-    v = block_sum(v, s_red);
-    if (threadIdx.x == 0) {
+struct MeanScale {
+    const T* domain;
+    int d;
+    long long N;
+    __device__ double operator()() const {
         double vol = 1.0;
         for (int k = 0; k < d; ++k) vol *= (double)domain[2 * k + 1] - (double)domain[2 * k];
-        out[s] = (T)(vol * v / (double)N);
+        return vol / (double)N;
     }
-}
+};
 
 static long long mc_spt(const tq_mc_desc* m) {
     if (m->samples_per_thread > 0) return m->samples_per_thread;
@@ -263,24 +229,6 @@ static int check_mc(const tq_mc_desc* m) {
     if (m->N < 1) return fail(TQ_E_ARG, "N must be >= 1");
     if (mc_blocks(m) > 0x7fffffffLL) return fail(TQ_E_ARG, "N too large for one launch; raise samples_per_thread");
     return TQ_OK;
-}
-
-static void colsum_shape(long long N, long long S, long long* nb, int* bd, long long* rpb) {
-    if (S < 64) {
-        *bd = (int)(kBlock - (kBlock % S));
-        long long b = (N * S + (long long)(*bd) * 16 - 1) / ((long long)(*bd) * 16);
-        if (b > 4096) b = 4096;
-        if (b < 1) b = 1;
-        *nb = b;
-        *rpb = 0;
-    } else {
-        *bd = kBlock;
-        long long ry = (N + 255) / 256;
-        if (ry > 1024) ry = 1024;
-        if (ry < 1) ry = 1;
-        *rpb = (N + ry - 1) / ry;
-        *nb = (N + *rpb - 1) / *rpb;
-    }
 }
 
 template <typename T>
@@ -314,24 +262,13 @@ static int launch_mc(const tq_mc_desc* m, const tq_integrand* f, const void* dom
 }
 
 template <typename T>
-static int launch_colsum(const void* fv, long long N, long long S, const void* domain, int d, void* ws,
-                         size_t wsb, void* out, hipStream_t st) {
-    long long nb, rpb;
-    int bd;
-    colsum_shape(N, S, &nb, &bd, &rpb);
-    if (!ws || wsb < (size_t)(nb * S) * sizeof(double)) return fail(TQ_E_WORKSPACE, "reduce workspace too small");
-    if (S < 64) {
-        hipLaunchKernelGGL((k_colsum_narrow<T>), dim3((unsigned)nb), dim3(bd), 0, st, (const T*)fv, N, S,
-                           (double*)ws);
-    } else {
-        dim3 grid((unsigned)((S + kBlock - 1) / kBlock), (unsigned)nb);
-        hipLaunchKernelGGL((k_colsum_wide<T>), grid, dim3(kBlock), 0, st, (const T*)fv, N, S, rpb, (double*)ws);
-    }
-    int rc = check_launch("k_colsum");
+static int launch_mean(const void* fv, long long N, long long S, const void* domain, int d, void* ws, size_t wsb,
+                       void* out, hipStream_t st) {
+    ValuePlan V;
+    const int rc = plan_values(0, 1, 0, nullptr, N, S, (int)sizeof(T), V);
     if (rc) return rc;
-    hipLaunchKernelGGL((k_colsum_finalize<T>), dim3((unsigned)S), dim3(kBlock), 0, st, (const double*)ws, nb, S,
-                       (const T*)domain, d, N, (T*)out);
-    return check_launch("k_colsum_finalize");
+    if (!ws || wsb < values_workspace(V)) return fail(TQ_E_WORKSPACE, "reduce workspace too small");
+    return launch_values<T>(V, (const T*)fv, (double*)ws, MeanScale<T>{(const T*)domain, d, N}, (T*)out, st);
 }
 
 }  // namespace tq
@@ -382,10 +319,13 @@ int tq_mc_points(const tq_mc_desc* m, const void* domain, void* points, void* st
 
 size_t tq_mc_reduce_workspace_size(int64_t N, int64_t S) {
     if (N < 1 || S < 1) return 0;
-    long long nb, rpb;
-    int bd;
-    colsum_shape(N, S, &nb, &bd, &rpb);
-    return (size_t)(nb * S) * sizeof(double);
+    size_t most = 0;  // the data type sets the span's rounding: room for either
+    for (int tsize = 4; tsize <= 8; tsize += 4) {
+        ValuePlan V;
+        if (plan_values(0, 1, 0, nullptr, N, S, tsize, V)) return 0;
+        if (values_workspace(V) > most) most = values_workspace(V);
+    }
+    return most;
 }
 
 int tq_mc_reduce(int32_t dtype, const void* fvals, int64_t N, int64_t S, const void* domain, int32_t dim,
@@ -395,8 +335,8 @@ int tq_mc_reduce(int32_t dtype, const void* fvals, int64_t N, int64_t S, const v
     if (dim < 1) return fail(TQ_E_ARG, "dim must be >= 1");
     if (!fvals || !domain || !out) return fail(TQ_E_NULL, "fvals/domain/out is NULL");
     if (dtype == TQ_F32)
-        return launch_colsum<float>(fvals, N, S, domain, dim, workspace, workspace_bytes, out, as_stream(stream));
-    return launch_colsum<double>(fvals, N, S, domain, dim, workspace, workspace_bytes, out, as_stream(stream));
+        return launch_mean<float>(fvals, N, S, domain, dim, workspace, workspace_bytes, out, as_stream(stream));
+    return launch_mean<double>(fvals, N, S, domain, dim, workspace, workspace_bytes, out, as_stream(stream));
 }
 
 int tq_uniform(uint64_t seed, uint64_t offset, int32_t dtype, int64_t rows, int32_t cols, void* out,
