@@ -121,6 +121,10 @@ int tq_grid_integrate_noalloc(const tq_grid_desc* g, const tq_integrand* f, cons
  * (integration_grid.py:98-99). */
 int tq_grid_points(const tq_grid_desc* g, const void* domain, void* points, void* stream);
 
+/* tq_grid_points that also writes tq_grid_h's mesh widths to h_out ([dim],
+ * NULL: not asked for) in the same launch. */
+int tq_grid_points_h(const tq_grid_desc* g, const void* domain, void* points, void* h_out, void* stream);
+
 /* h_d = x_1 - x_0 per axis (integration_grid.py:90-93), dtype, [dim]. */
 int tq_grid_h(const tq_grid_desc* g, const void* domain, void* h_out, void* stream);
 
@@ -142,6 +146,14 @@ int tq_grid_reduce(const tq_grid_desc* g, const void* domain, const void* hs, in
 int tq_grid_reduce_backward(const tq_grid_desc* g, const void* domain, const void* hs,
                             int32_t unit_weights, const void* grad_out, int64_t S, void* grad_f,
                             void* stream);
+
+/* Both gradients of tq_grid_reduce in one launch: grad_f[P, S] (NULL: not
+ * asked for) and, where the scale comes from the domain (hs NULL, unit
+ * weights or Gauss-Legendre), grad_domain[dim, 2] = -+ sum_s grad_out[s]
+ * out[s] / (b_k - a_k) (NULL: not asked for); out[S] is the forward result. */
+int tq_grid_reduce_vjp(const tq_grid_desc* g, const void* domain, const void* hs, int32_t unit_weights,
+                       const void* grad_out, const void* out, int64_t S, void* grad_f, void* grad_domain,
+                       void* stream);
 
 /* Backward of tq_grid_points: grad_domain[k, 0/1] = sum_p grad_points[p, k]
  * * d x_k(p) / d(a_k, b_k) (the derivative of linspace / of the

@@ -133,3 +133,99 @@ def test_mc_reduce_sizes(N, S, dtype, dev):
     tol = vol * ((2.0**-24 if dtype == torch.float32 else 0.0) + N * 2.0**-53)
     for v in (vals, other.view(N, S)):
         assert float((_ops.mc_reduce(v, dom).double() - ref).abs().max()) <= tol
+
+
+def _axis_weights(rule, n, gl):
+    if rule == "gauss_legendre":
+        return gl[1].cpu().numpy()
+    if rule == "trapezoid":
+        return np.r_[1.0, np.full(n - 2, 2.0), 1.0]
+    w = np.full(n, 14.0)
+    w[1::2], w[2::4], w[0], w[-1] = 32.0, 12.0, 7.0, 7.0
+    return w
+
+
+BACKWARD = [(1, 5, 1), (1, 257, 1), (1, 2049, 1), (1, 30001, 1), (2, 45, 1), (2, 49, 1), (3, 101, 1), (8, 5, 1),
+            (2, 301, 1), (2, 2, 1), (3, 9, 2), (2, 33, 3), (4, 5, 31), (1, 1001, 64), (2, 17, 65), (1, 101, 200)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rule", ["trapezoid", "boole", "gauss_legendre"])
+@pytest.mark.parametrize("d,n,S", BACKWARD)
+def test_grid_reduce_vjp_sizes(d, n, S, rule, dtype, dev):
+    if rule == "boole":
+        n = max(5, n - (n - 1) % 4)
+    dom = _box(d, dtype, dev, n)
+    gl = gauss_legendre(n, device=dev) if rule == "gauss_legendre" else None
+    code = _ops.RULES[rule]
+    gen = torch.Generator(device=dev).manual_seed(d * 1000 + n + S)
+    g = torch.rand(S, dtype=dtype, device=dev, generator=gen) - 0.25
+    out = torch.rand(S, dtype=dtype, device=dev, generator=gen) - 0.25
+    gf, gd = _ops.grid_reduce_vjp(code, d, n, dom, g, out, n**d, gl=gl)
+    b = dom.double()
+    width = b[:, 1] - b[:, 0]
+    w = torch.tensor(_axis_weights(rule, n, gl), device=dev)
+    c = {"gauss_legendre": 0.5, "trapezoid": 0.5 / (n - 1), "boole": 1.0 / 22.5 / (n - 1)}[rule]
+    W = torch.prod(width * c).reshape(1)
+    for _ in range(d):
+        W = (W[:, None] * w[None, :]).reshape(-1)
+    ref = W[:, None] * g.double()[None, :]
+    # a product of at most 2 d + 2 FP64 factors, rounded once to the data type
+    eps = (2.0**-24 if dtype == torch.float32 else 0.0) + (2 * d + 4) * 2.0**-53
+    assert bool(((gf.double() - ref).abs() <= eps * ref.abs()).all())
+    other = _unaligned(n**d * S, dtype, dev)
+    desc = _ops.grid_desc(code, d, n, dtype, gl)
+    _lib.call("tq_grid_reduce_backward", ctypes.byref(desc), _lib.ptr(dom), None, 0, _lib.ptr(g), S, _lib.ptr(other),
+              _lib.stream_ptr(dev))
+    assert bool(((other.view(n**d, S).double() - ref).abs() <= eps * ref.abs()).all())
+    gs = torch.sum(g.double() * out.double())
+    bar = float(torch.sum((g.double() * out.double()).abs()))
+    rd = torch.stack([-gs / width, gs / width], dim=1)
+    tol = bar / width.min() * (S * 2.0**-53) + rd.abs() * eps
+    assert bool(((gd.double() - rd).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rule", ["trapezoid", "gauss_legendre"])
+@pytest.mark.parametrize("d,n", [(1, 2), (1, 64), (1, 2049), (1, 40001), (2, 3), (2, 45), (2, 700), (3, 65), (4, 32),
+                                 (5, 9), (9, 3), (12, 2)])
+def test_grid_points_backward_sizes(d, n, rule, dtype, dev):
+    dom = _box(d, dtype, dev, n)
+    gl = gauss_legendre(n, device=dev) if rule == "gauss_legendre" else None
+    gen = torch.Generator(device=dev).manual_seed(d * 1000 + n)
+    gp = torch.rand((n**d, d), dtype=dtype, device=dev, generator=gen) - 0.25
+    got = _ops.grid_points_backward(_ops.RULES[rule], d, n, dom, gp, gl).double()
+    if gl is None:
+        t = torch.arange(n, dtype=torch.float64, device=dev) / (n - 1)
+    else:
+        t = 0.5 * (1.0 + gl[0])
+    g64 = gp.double().view(*([n] * d), d)
+    for k in range(d):
+        s = g64[..., k].sum(dim=[q for q in range(d) if q != k]) if d > 1 else g64[..., 0]
+        gb, ga = torch.sum(s * t), torch.sum(s * (1.0 - t))
+        bar = float(gp[:, k].double().abs().sum())
+        # FP64 sums of n^d terms, one rounding of the result
+        tol = bar * n**d * 2.0**-53 + float(max(ga.abs(), gb.abs())) * (2.0**-24 if dtype == torch.float32 else 0.0)
+        assert abs(float(got[k, 0] - ga)) <= tol and abs(float(got[k, 1] - gb)) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("name", ["Trapezoid", "Simpson", "Boole", "GaussLegendre"])
+def test_call_gradients_match_recorded_backward(name, dtype, dev):
+    """Gradients of a callable's integral with and without a recorded backward
+    (create_graph), for the values' and the domain's part."""
+    import torchquad_amd as tq
+
+    d, n = 2, 13
+    a = torch.tensor([1.3, 0.7], dtype=dtype, device=dev, requires_grad=True)
+    dom = _box(d, dtype, dev, 5).requires_grad_()
+
+    def value():
+        return getattr(tq, name)().integrate(lambda x: torch.exp(-torch.sum(a * x * x, dim=1)), d, N=n**d,
+                                             integration_domain=dom)
+
+    plain = torch.autograd.grad(value(), [a, dom])
+    kept = torch.autograd.grad(value(), [a, dom], create_graph=True)
+    eps = 2.0**-22 if dtype == torch.float32 else 2.0**-50
+    for p, q in zip(plain, kept):
+        assert float((p - q).abs().max()) <= eps * float(q.abs().max())

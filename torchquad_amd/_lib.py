@@ -127,10 +127,12 @@ SIGNATURES = {
         [ctypes.POINTER(GridDesc), ctypes.POINTER(Integrand), _P, _P, _P, _P],
     ),
     "tq_grid_points": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _P]),
+    "tq_grid_points_h": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _P, _P]),
     "tq_grid_h": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _P]),
     "tq_grid_reduce_workspace_size": (_SZ, [ctypes.POINTER(GridDesc), _I64]),
     "tq_grid_reduce": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _I32, _P, _I64, _P, _SZ, _P, _P]),
     "tq_grid_reduce_backward": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _I32, _P, _I64, _P, _P]),
+    "tq_grid_reduce_vjp": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _I32, _P, _P, _I64, _P, _P, _P]),
     "tq_grid_points_backward_workspace_size": (_SZ, [ctypes.POINTER(GridDesc)]),
     "tq_grid_points_backward": (ctypes.c_int, [ctypes.POINTER(GridDesc), _P, _P, _P, _SZ, _P, _P]),
     "tq_gauss_legendre": (ctypes.c_int, [_I32, _P, _P, _P]),

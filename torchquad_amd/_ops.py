@@ -98,6 +98,16 @@ def grid_points(rule, dim, n, domain, gl=None):
     return pts
 
 
+def grid_points_h(rule, dim, n, domain, gl=None):
+    """grid_points and grid_h from one launch."""
+    require_device(domain)
+    g = grid_desc(rule, dim, n, domain.dtype, gl)
+    pts = torch.empty((n**dim, dim), dtype=domain.dtype, device=domain.device)
+    h = torch.empty((dim,), dtype=domain.dtype, device=domain.device)
+    call("tq_grid_points_h", ctypes.byref(g), ptr(domain), ptr(pts), ptr(h), stream_ptr(domain.device))
+    return pts, h
+
+
 def grid_h(rule, dim, n, domain, gl=None):
     require_device(domain)
     g = grid_desc(rule, dim, n, domain.dtype, gl)
@@ -157,6 +167,37 @@ def grid_reduce_backward(rule, dim, n, domain, grad_out, npoints, hs=None, unit_
         stream_ptr(domain.device),
     )
     return grad_f
+
+
+def grid_reduce_vjp(rule, dim, n, domain, grad_out, out, npoints, hs=None, unit_weights=False, gl=None,
+                    need_values=True, need_domain=True):
+    """Gradients of grid_reduce for the values and the domain (a scale from the
+    domain: hs None, unit weights or Gauss-Legendre) in one launch; None for
+    the one that is not needed."""
+    require_device(domain)
+    grad_out = grad_out.contiguous().to(domain.dtype)
+    g = grid_desc(rule, dim, n, domain.dtype, gl)
+    grad_f = grad_domain = None
+    if need_values:
+        grad_f = torch.empty((npoints, *grad_out.shape), dtype=domain.dtype, device=domain.device)
+    if need_domain:
+        grad_domain = torch.empty((dim, 2), dtype=domain.dtype, device=domain.device)
+    if hs is not None:
+        hs = hs.detach().to(domain.dtype).contiguous()
+    call(
+        "tq_grid_reduce_vjp",
+        ctypes.byref(g),
+        ptr(domain),
+        ptr(hs),
+        1 if unit_weights else 0,
+        ptr(grad_out),
+        ptr(out),
+        grad_out.numel(),
+        ptr(grad_f),
+        ptr(grad_domain),
+        stream_ptr(domain.device),
+    )
+    return grad_f, grad_domain
 
 
 def grid_points_backward(rule, dim, n, domain, grad_points, gl=None):

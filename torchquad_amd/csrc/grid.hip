@@ -385,14 +385,25 @@ static int launch_grid(const tq_grid_desc* gd, const tq_integrand* f, const void
 // ---------------------------------------------------------------------------
 // Point writer (user integrands)
 // ---------------------------------------------------------------------------
+// h = x_1 - x_0 of an axis in the data type (integration_grid.py:90-93).
+template <typename T>
+__device__ inline T mesh_width(const Axis& ax, int n, int rule, const double* glx) {
+    const T x0 = (T)node_of(ax, 0, n, rule, glx);
+    const T x1 = (n > 1) ? (T)node_of(ax, 1, n, rule, glx) : x0;
+    return x1 - x0;
+}
+
 // Any grid: one point per thread, coordinates stored one by one.  Used for
 // more than 2^31 points, more axes than the staged writer's LDS holds and
 // unaligned outputs.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_grid_points(const T* domain, int d, int n, int rule,
-                                                        const double* glx, long long P, T* pts) {
+                                                        const double* glx, long long P, T* pts, T* h) {
     __shared__ Axis s_axis[kMaxDimPoints];
-    for (int k = threadIdx.x; k < d; k += blockDim.x) s_axis[k] = make_axis(domain, k, n, rule);
+    for (int k = threadIdx.x; k < d; k += blockDim.x) {
+        s_axis[k] = make_axis(domain, k, n, rule);
+        if (h && blockIdx.x == 0) h[k] = mesh_width<T>(s_axis[k], n, rule, glx);
+    }
     __syncthreads();
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += stride) {
@@ -415,11 +426,14 @@ constexpr size_t kNodeTableMax = 16 * 1024;
 template <typename T, bool NODES, int PPL>
 __global__ __launch_bounds__(kBlock) void k_grid_points_staged(const T* domain, int d, FastDiv by_n, int rule,
                                                                const double* glx, uint32_t P, uint32_t chunks,
-                                                               T* pts) {
+                                                               T* pts, T* h) {
     extern __shared__ __align__(16) unsigned char s_raw[];
     __shared__ Axis s_axis[kMaxDimPoints];
     const int n = (int)by_n.n;
-    for (int k = threadIdx.x; k < d; k += kBlock) s_axis[k] = make_axis(domain, k, n, rule);
+    for (int k = threadIdx.x; k < d; k += kBlock) {
+        s_axis[k] = make_axis(domain, k, n, rule);
+        if (h && blockIdx.x == 0) h[k] = mesh_width<T>(s_axis[k], n, rule, glx);
+    }
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
     constexpr int C = kWave * PPL;
@@ -460,7 +474,7 @@ __global__ __launch_bounds__(kBlock) void k_grid_points_staged(const T* domain, 
 }
 
 template <typename T, int PPL>
-static void launch_points_staged(const tq_grid_desc* g, const void* domain, long long P, void* points,
+static void launch_points_staged(const tq_grid_desc* g, const void* domain, long long P, void* points, void* h,
                                  hipStream_t st) {
     const FastDiv by_n = make_fast_div((uint32_t)g->n);
     const size_t nodes = (size_t)g->dim * g->n * sizeof(T);
@@ -473,25 +487,28 @@ static void launch_points_staged(const tq_grid_desc* g, const void* domain, long
     if (blocks > 2048) blocks = 2048;
     if (table)
         hipLaunchKernelGGL((k_grid_points_staged<T, true, PPL>), dim3((unsigned)blocks), dim3(kBlock), lds, st,
-                           (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points);
+                           (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points,
+                           (T*)h);
     else
         hipLaunchKernelGGL((k_grid_points_staged<T, false, PPL>), dim3((unsigned)blocks), dim3(kBlock), lds, st,
-                           (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points);
+                           (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points,
+                           (T*)h);
 }
 
 template <typename T>
-static int launch_points(const tq_grid_desc* g, const void* domain, long long P, void* points, hipStream_t st) {
+static int launch_points(const tq_grid_desc* g, const void* domain, long long P, void* points, void* h,
+                         hipStream_t st) {
     if (P <= 0x7fffffffLL && stage_fits(g->dim, sizeof(T), points)) {
         if (stage_ppl(g->dim, sizeof(T)) > 1)
-            launch_points_staged<T, 16 / (int)sizeof(T)>(g, domain, P, points, st);
+            launch_points_staged<T, 16 / (int)sizeof(T)>(g, domain, P, points, h, st);
         else
-            launch_points_staged<T, 1>(g, domain, P, points, st);
+            launch_points_staged<T, 1>(g, domain, P, points, h, st);
         return check_launch("k_grid_points_staged");
     }
     long long blocks = (P + kBlock - 1) / kBlock;
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL((k_grid_points<T>), dim3((unsigned)blocks), dim3(kBlock), 0, st, (const T*)domain, g->dim,
-                       g->n, g->rule, g->gl_nodes, P, (T*)points);
+                       g->n, g->rule, g->gl_nodes, P, (T*)points, (T*)h);
     return check_launch("k_grid_points");
 }
 
@@ -499,10 +516,7 @@ template <typename T>
 __global__ void k_grid_h(const T* domain, int d, int n, int rule, const double* glx, T* h) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= d) return;
-    const Axis ax = make_axis(domain, k, n, rule);
-    const T x0 = (T)node_of(ax, 0, n, rule, glx);
-    const T x1 = (n > 1) ? (T)node_of(ax, 1, n, rule, glx) : x0;
-    h[k] = x1 - x0;
+    h[k] = mesh_width<T>(make_axis(domain, k, n, rule), n, rule, glx);
 }
 
 // ---------------------------------------------------------------------------
@@ -543,77 +557,225 @@ static int plan_reduce(const tq_grid_desc* g, long long S, int unit, ValuePlan& 
     return plan_values(unit ? 0 : g->dim, g->n, g->rule, g->gl_weights, P, S, g->dtype == TQ_F32 ? 4 : 8, V);
 }
 
-// grad_f[p, s] = grad_out[s] * scale * W(p)
+// Backward of the weighted reduction: grad_f[p, s] = grad_out[s] * scale *
+// W(p), a stream of writes.  Waves write contiguous ranges of `span` values
+// (a multiple of 64 VEC), VEC per lane and store; a lane's values mostly
+// share their point, so its weight is formed when the point changes (1e6
+// values, d=4: 10.2 -> 7.6 us; [N, S] values were written one component at a
+// time with lanes S elements apart).  One
+// more block (when grad_domain is asked for) forms d/d domain, which only
+// the scale depends on: -+ sum_s grad_out[s] out[s] / (b_k - a_k).
+template <typename T, int VEC, int MODE>
+__global__ __launch_bounds__(kBlock) void k_grid_reduce_backward(PointWeights w, GridScale<T> scale, const T* grad_out,
+                                                                 FastDiv by_S, long long total, long long span,
+                                                                 T* grad_f, const T* out, T* grad_domain) {
+    extern __shared__ double s_w[];
+    __shared__ double s_scale, s_red[kWavesPerBlock];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int S = (int)by_S.n;
+    if (grad_domain && blockIdx.x == gridDim.x - 1) {
+        double v = 0.0;
+        for (int s = tid; s < S; s += kBlock) v = fma((double)grad_out[s], (double)out[s], v);
+        v = block_sum(v, s_red);
+        if (tid == 0) s_scale = v;
+        __syncthreads();
+        for (int k = tid; k < scale.d; k += kBlock) {
+            const double g = s_scale / ((double)scale.domain[2 * k + 1] - (double)scale.domain[2 * k]);
+            grad_domain[2 * k] = (T)(-g);
+            grad_domain[2 * k + 1] = (T)g;
+        }
+        return;
+    }
+    if (tid == 0) s_scale = scale();
+    const WeightTables tab = build_weights<MODE>(w, s_w);
+    __syncthreads();
+    const long long wave = (long long)blockIdx.x * kWavesPerBlock + __builtin_amdgcn_readfirstlane(tid >> 6);
+    const long long e0 = wave * span;
+    if (e0 >= total) return;
+    const uint32_t len = (uint32_t)(total - e0 < span ? total - e0 : span);
+    const long long pt0 = S == 1 ? e0 : e0 / S;
+    const uint32_t sub0 = S == 1 ? 0u : (uint32_t)(e0 - pt0 * S);
+    uint32_t row0 = 0, in0 = (uint32_t)pt0;
+    if (MODE != kUnitWeights && w.outer_axes > 0) {
+        row0 = (uint32_t)(pt0 / w.inner);
+        in0 = (uint32_t)(pt0 - (long long)row0 * w.inner);
+    }
+    const double sc = s_scale;
+    const double g0 = S == 1 ? (double)grad_out[0] : 0.0;
+    T* dst = grad_f + e0;
+    auto values = [&](uint32_t off, T* x, int count) {
+        if (S == 1) {
+            if (MODE == kUnitWeights || w.outer_axes == 0) {
+                for (int i = 0; i < count; ++i)
+                    x[i] = (T)(sc * point_weight<MODE>(w, tab, row0, in0, off + i) * g0);
+                return;
+            }
+            // one outer weight per row
+            const uint32_t p = in0 + off, r = w.by_inner.div(p);
+            uint32_t in = p - r * w.inner;
+            double wo = sc * outer_weight<MODE>(w, tab, row0 + r);
+            for (int i = 0; i < count; ++i, ++in) {
+                if (in == w.inner) {
+                    in = 0;
+                    wo = sc * outer_weight<MODE>(w, tab, row0 + r + 1);
+                }
+                x[i] = (T)(wo * inner_weight<MODE>(w, tab, in) * g0);
+            }
+            return;
+        }
+        uint32_t pt = by_S.div(sub0 + off), s = sub0 + off - pt * (uint32_t)S;
+        double wp = sc * point_weight<MODE>(w, tab, row0, in0, pt);
+        for (int i = 0; i < count; ++i, ++s) {
+            if (s == (uint32_t)S) {
+                s = 0;
+                ++pt;
+                wp = sc * point_weight<MODE>(w, tab, row0, in0, pt);
+            }
+            x[i] = (T)(wp * (double)grad_out[s]);
+        }
+    };
+    uint32_t off = 0;
+    constexpr uint32_t step = kWave * VEC;
+    for (; off + step <= len; off += step) {
+        T x[VEC];
+        values(off + lane * VEC, x, VEC);
+        if constexpr (VEC == 1) {
+            dst[off + lane] = x[0];
+        } else {
+            using V = __attribute__((ext_vector_type(VEC))) T;
+            V v;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) v[i] = x[i];
+            *reinterpret_cast<V*>(dst + off + lane * VEC) = v;
+        }
+    }
+    for (off += lane; off < len; off += kWave) values(off, dst + off, 1);
+}
+
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_grid_reduce_backward(const T* domain, const T* hs, int unit, int d,
-                                                                 int n, int rule, const double* glw,
-                                                                 const T* grad_out, long long S, long long P,
-                                                                 T* grad_f) {
-    const double scale = reduce_scale(domain, hs, d, n, rule, unit);
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += stride) {
-        double w = scale;
-        if (!unit) {
-            unsigned long long rem = (unsigned long long)p;
-            for (int k = d - 1; k >= 0; --k) {
-                const int j = (int)(rem % (unsigned long long)n);
-                rem /= (unsigned long long)n;
-                w *= weight_of(rule, j, n, glw);
+static int launch_reduce_backward(const tq_grid_desc* g, const void* domain, const void* hs, int unit,
+                                  const void* grad_out, long long S, void* grad_f, const void* out, void* grad_domain,
+                                  hipStream_t st) {
+    constexpr int VEC = 16 / (int)sizeof(T);
+    ValuePlan V;  // for the weights; the values' split below is over P * S elements
+    int rc = plan_reduce(g, 1, unit, V);
+    if (rc) return rc;
+    const long long total = V.P * S;
+    const GridScale<T> scale{(const T*)domain, (const T*)hs, g->dim, g->n, g->rule, unit};
+    long long span = (total + 8191) / 8192;
+    if (span < 1024) span = 1024;
+    span = (span + kWave * VEC - 1) / (kWave * VEC) * (kWave * VEC);
+    if (span > (1LL << 30)) return fail(TQ_E_ARG, "too many values for one launch");
+    const long long per_block = span * kWavesPerBlock;
+    const long long blocks = (grad_f ? (total + per_block - 1) / per_block : 0) + (grad_domain ? 1 : 0);
+    if (blocks == 0) return TQ_OK;
+    const bool vec = ((uintptr_t)grad_f & 15) == 0 &&
+                     (V.w.mode == kUnitWeights || S > 1 || V.w.inner >= (uint32_t)VEC);
+    const FastDiv by_S = make_fast_div((uint32_t)S);
+#define TQ_RB(VV, MODE)                                                                                             \
+    hipLaunchKernelGGL((k_grid_reduce_backward<T, VV, MODE>), dim3((unsigned)blocks), dim3(kBlock), V.lds, st, V.w, \
+                       scale, (const T*)grad_out, by_S, total, span, (T*)grad_f, (const T*)out, (T*)grad_domain)
+#define TQ_RBV(MODE)                     \
+    do {                                 \
+        if (vec) TQ_RB(VEC, MODE);       \
+        else TQ_RB(1, MODE);             \
+    } while (0)
+    if (V.w.mode == kUnitWeights) TQ_RBV(kUnitWeights);
+    else if (V.w.mode == kTableWeights) TQ_RBV(kTableWeights);
+    else TQ_RBV(kDirectWeights);
+#undef TQ_RBV
+#undef TQ_RB
+    return check_launch("k_grid_reduce_backward");
+}
+
+// Backward of the point writer over grad_points[P, d], a stream of reads.
+// A node is x = a (1 - t) + b t with t = j/(n-1), or (1 + r_j)/2 for
+// Gaussian rules, so d/da = sum g (1 - t) and d/db = sum g t: two sums per
+// axis.  64 / d points per wave and load, each lane on one axis, whose digit
+// of the point index takes two multiply-highs; t comes from an LDS table
+// when it fits.  With 64-bit divisions per element 1e6 points, d=4 took 28 us,
+// 11 us so (21 MB read; the rest is launch, table and block sums).
+constexpr int kNodeWeights = 2048;  // t values kept in LDS (16 KB)
+
+// t of node j
+__device__ inline double node_fraction(int j, int n, int rule, const double* glx) {
+    if (rule == TQ_RULE_GAUSS_LEGENDRE) return 0.5 * (1.0 + glx[j]);
+    return n > 1 ? (double)j / (double)(n - 1) : 0.0;
+}
+
+template <typename T, bool TABLE>
+__global__ __launch_bounds__(kBlock) void k_grid_points_backward(int d, int n, int rule, const double* glx,
+                                                                 long long P, long long span, const T* gp,
+                                                                 double* partials /* [blocks][d][2] */) {
+    __shared__ double s_t[TABLE ? kNodeWeights : 1];
+    __shared__ double s_a[kBlock], s_b[kBlock];
+    if (TABLE) {
+        for (int j = threadIdx.x; j < n; j += kBlock) s_t[j] = node_fraction(j, n, rule, glx);
+        __syncthreads();
+    }
+    const int lane = threadIdx.x & (kWave - 1);
+    const int step = kWave / d, po = lane / d, k = lane - po * d;
+    const long long wave = (long long)blockIdx.x * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long p0 = wave * span, p1 = p0 + span < P ? p0 + span : P;
+    double acc = 0.0, acc_t = 0.0;
+    if (po < step && p0 < p1) {
+        // digit of axis k: (p / n^(d-1-k)) mod n.  It repeats every n^(d-k) points, so the walk keeps p
+        // modulo that period (when it is below 2^31) and divides 32-bit numbers.
+        long long stride = 1;
+        for (int q = k + 1; q < d; ++q) stride *= n;
+        const bool small = stride <= 0x3fffffffLL / n;
+        const long long period = stride * n;
+        long long p = p0 + po;
+        uint32_t r = small ? (uint32_t)(p % period) : 0u;
+        const uint32_t st32 = small ? (uint32_t)stride : 1u;
+        // multiply-high constants of this lane's stride (tq FastDiv)
+        uint32_t m = 1u, sh = 0u;
+        if (st32 > 1u) {
+            const int l = 32 - __builtin_clz(st32 - 1u);
+            sh = (uint32_t)l - 1u;
+            m = (uint32_t)(((1ull << (31 + l)) + st32 - 1ull) / st32);
+        }
+        const uint32_t per32 = small ? (uint32_t)period : 0xffffffffu;
+        // one step may pass several periods of a short axis
+        const uint32_t adv = small ? (uint32_t)step % per32 : 0u;
+        const T* src = gp + p0 * d + lane;
+        const long long row = (long long)step * d;
+        constexpr int U = 4;
+        // t of this lane's axis at point q; then the walk's digit state moves one step on
+        auto fraction = [&](long long q) {
+            const int j = small ? (int)(st32 == 1u ? r : __umulhi(r, m) >> sh) : (int)((q / stride) % n);
+            r += adv;
+            if (r >= per32) r -= per32;
+            return TABLE ? s_t[j] : node_fraction(j, n, rule, glx);
+        };
+        for (; p + (long long)(U - 1) * step < p1; p += (long long)U * step, src += U * row) {
+            T x[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u] = src[u * row];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const double g = (double)x[u];
+                acc += g;
+                acc_t = fma(g, fraction(p + (long long)u * step), acc_t);
             }
         }
-        for (long long s = 0; s < S; ++s) grad_f[p * S + s] = (T)(w * (double)grad_out[s]);
-    }
-}
-
-// d x_k / d a_k and d x_k / d b_k of node j on axis k.
-__device__ inline void node_grad(int j, int n, int rule, const double* glx, double* da, double* db) {
-    if (rule == TQ_RULE_GAUSS_LEGENDRE) {
-        const double r = glx[j];
-        *da = 0.5 * (1.0 - r);
-        *db = 0.5 * (1.0 + r);
-    } else {
-        const double t = (n > 1) ? (double)j / (double)(n - 1) : 0.0;
-        *da = 1.0 - t;
-        *db = t;
-    }
-}
-
-// Column-fixed threads over grad_points[P, d]: block size is a multiple of d.
-struct Strides {
-    long long s[kMaxDimPoints];
-};
-
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_grid_points_backward(int d, int n, int rule, const double* glx,
-                                                                 Strides strides, long long P,
-                                                                 const T* gp, double* partials /* [blocks][d][2] */) {
-    __shared__ double s_a[kBlock], s_b[kBlock];
-    const long long bd = blockDim.x;
-    const long long total = P * d;
-    const long long stride = (long long)gridDim.x * bd;
-    double acc_a = 0.0, acc_b = 0.0;
-    const long long e0 = (long long)blockIdx.x * bd + threadIdx.x;
-    const int k = (int)(e0 % d);
-    const long long st = strides.s[k];
-    for (long long e = e0; e < total; e += stride) {
-        const long long p = e / d;
-        const int j = (int)((p / st) % n);
-        double da, db;
-        node_grad(j, n, rule, glx, &da, &db);
-        const double g = (double)gp[e];
-        acc_a = fma(g, da, acc_a);
-        acc_b = fma(g, db, acc_b);
-    }
-    s_a[threadIdx.x] = acc_a;
-    s_b[threadIdx.x] = acc_b;
-    __syncthreads();
-    if (threadIdx.x < d) {
-        double va = 0.0, vb = 0.0;
-        for (long long i = threadIdx.x; i < bd; i += d) {
-            va += s_a[i];
-            vb += s_b[i];
+        for (; p < p1; p += step, src += row) {
+            const double g = (double)*src;
+            acc += g;
+            acc_t = fma(g, fraction(p), acc_t);
         }
-        partials[((long long)blockIdx.x * d + threadIdx.x) * 2] = va;
+    }
+    s_a[threadIdx.x] = acc;
+    s_b[threadIdx.x] = acc_t;
+    __syncthreads();
+    if ((int)threadIdx.x < d) {
+        double va = 0.0, vb = 0.0;
+        for (int q = 0; q < kWavesPerBlock; ++q)
+            for (int i = threadIdx.x; i < step * d; i += d) {
+                va += s_a[q * kWave + i];
+                vb += s_b[q * kWave + i];
+            }
+        partials[((long long)blockIdx.x * d + threadIdx.x) * 2] = va - vb;
         partials[((long long)blockIdx.x * d + threadIdx.x) * 2 + 1] = vb;
     }
 }
@@ -629,12 +791,13 @@ __global__ __launch_bounds__(kBlock) void k_grid_points_backward_finalize(const 
     if (threadIdx.x == 0) grad_domain[e] = (T)v;
 }
 
-static void points_backward_shape(int d, long long P, int* bd, long long* nb) {
-    *bd = kBlock - (kBlock % d);
-    long long b = (P * d + (long long)(*bd) * 32 - 1) / ((long long)(*bd) * 32);
-    if (b > 2048) b = 2048;
-    if (b < 1) b = 1;
-    *nb = b;
+// Points per wave: at most about 4096 waves, at least 2048 values each.
+static void points_backward_shape(int d, long long P, long long* span, long long* nb) {
+    const long long least = (2048 + d - 1) / d;
+    long long s = (P + 4095) / 4096;
+    if (s < least) s = least;
+    *span = s;
+    *nb = (P + s * kWavesPerBlock - 1) / (s * kWavesPerBlock);
 }
 
 // ---------------------------------------------------------------------------
@@ -735,7 +898,7 @@ int tq_grid_integrate_noalloc(const tq_grid_desc* g, const tq_integrand* f, cons
     return launch_grid<double>(g, f, domain, ws, need, out, out_f64, as_stream(stream));
 }
 
-int tq_grid_points(const tq_grid_desc* g, const void* domain, void* points, void* stream) {
+int tq_grid_points_h(const tq_grid_desc* g, const void* domain, void* points, void* h_out, void* stream) {
     int rc = check_grid_desc(g, kMaxDimPoints);
     if (rc) return rc;
     rc = check_gl_tables(g);
@@ -743,8 +906,12 @@ int tq_grid_points(const tq_grid_desc* g, const void* domain, void* points, void
     if (!domain || !points) return fail(TQ_E_NULL, "domain/points is NULL");
     long long P;
     ipow_checked(g->n, g->dim, 1LL << 62, &P);
-    if (g->dtype == TQ_F32) return launch_points<float>(g, domain, P, points, as_stream(stream));
-    return launch_points<double>(g, domain, P, points, as_stream(stream));
+    if (g->dtype == TQ_F32) return launch_points<float>(g, domain, P, points, h_out, as_stream(stream));
+    return launch_points<double>(g, domain, P, points, h_out, as_stream(stream));
+}
+
+int tq_grid_points(const tq_grid_desc* g, const void* domain, void* points, void* stream) {
+    return tq_grid_points_h(g, domain, points, nullptr, stream);
 }
 
 int tq_grid_h(const tq_grid_desc* g, const void* domain, void* h_out, void* stream) {
@@ -797,41 +964,66 @@ int tq_grid_reduce(const tq_grid_desc* g, const void* domain, const void* hs, in
                                  (double*)out, st);
 }
 
-int tq_grid_reduce_backward(const tq_grid_desc* g, const void* domain, const void* hs, int32_t unit_weights,
-                            const void* grad_out, int64_t S, void* grad_f, void* stream) {
+int tq_grid_reduce_vjp(const tq_grid_desc* g, const void* domain, const void* hs, int32_t unit_weights,
+                       const void* grad_out, const void* out, int64_t S, void* grad_f, void* grad_domain,
+                       void* stream) {
     int rc = check_grid_desc(g, kMaxDimPoints);
     if (rc) return rc;
     if (!unit_weights) {
         rc = check_gl_tables(g);
         if (rc) return rc;
     }
-    if (S < 1) return fail(TQ_E_ARG, "S must be >= 1");
-    if (!domain || !grad_out || !grad_f) return fail(TQ_E_NULL, "domain/grad_out/grad_f is NULL");
-    long long P;
-    ipow_checked(g->n, g->dim, 1LL << 62, &P);
-    long long blocks = (P + kBlock - 1) / kBlock;
-    if (blocks > 65536) blocks = 65536;
+    if (S < 1 || S > 0x3fffffff) return fail(TQ_E_ARG, "S out of range");
+    if (!domain || !grad_out || (!grad_f && !grad_domain)) return fail(TQ_E_NULL, "domain/grad_out/grad_f is NULL");
+    if (grad_domain && !out) return fail(TQ_E_NULL, "grad_domain needs the forward result");
     const int unit = unit_weights ? 1 : 0;
+    if (grad_domain && hs && !unit && g->rule != TQ_RULE_GAUSS_LEGENDRE)
+        return fail(TQ_E_ARG, "with mesh widths the result does not depend on the domain");
     if (g->dtype == TQ_F32)
-        hipLaunchKernelGGL((k_grid_reduce_backward<float>), dim3((unsigned)blocks), dim3(kBlock), 0,
-                           as_stream(stream), (const float*)domain, (const float*)hs, unit, g->dim, g->n, g->rule,
-                           g->gl_weights, (const float*)grad_out, (long long)S, P, (float*)grad_f);
-    else
-        hipLaunchKernelGGL((k_grid_reduce_backward<double>), dim3((unsigned)blocks), dim3(kBlock), 0,
-                           as_stream(stream), (const double*)domain, (const double*)hs, unit, g->dim, g->n,
-                           g->rule, g->gl_weights, (const double*)grad_out, (long long)S, P, (double*)grad_f);
-    return check_launch("k_grid_reduce_backward");
+        return launch_reduce_backward<float>(g, domain, hs, unit, grad_out, S, grad_f, out, grad_domain,
+                                             as_stream(stream));
+    return launch_reduce_backward<double>(g, domain, hs, unit, grad_out, S, grad_f, out, grad_domain,
+                                          as_stream(stream));
+}
+
+int tq_grid_reduce_backward(const tq_grid_desc* g, const void* domain, const void* hs, int32_t unit_weights,
+                            const void* grad_out, int64_t S, void* grad_f, void* stream) {
+    if (!grad_f) return fail(TQ_E_NULL, "domain/grad_out/grad_f is NULL");
+    return tq_grid_reduce_vjp(g, domain, hs, unit_weights, grad_out, nullptr, S, grad_f, nullptr, stream);
 }
 
 size_t tq_grid_points_backward_workspace_size(const tq_grid_desc* g) {
     if (check_grid_desc(g, kMaxDimPoints)) return 0;
-    long long P;
+    long long P, span, nb;
     ipow_checked(g->n, g->dim, 1LL << 62, &P);
-    int bd;
-    long long nb;
-    points_backward_shape(g->dim, P, &bd, &nb);
+    points_backward_shape(g->dim, P, &span, &nb);
     return (size_t)(nb * g->dim * 2) * sizeof(double);
 }
+
+}  // extern "C"
+
+template <typename T>
+static int launch_points_backward(const tq_grid_desc* g, const void* grad_points, void* ws, size_t ws_bytes,
+                                  void* grad_domain, hipStream_t s) {
+    long long P, span, nb;
+    ipow_checked(g->n, g->dim, 1LL << 62, &P);
+    points_backward_shape(g->dim, P, &span, &nb);
+    if (!ws || ws_bytes < (size_t)(nb * g->dim * 2) * sizeof(double))
+        return fail(TQ_E_WORKSPACE, "points backward workspace too small");
+    if (g->n <= kNodeWeights)
+        hipLaunchKernelGGL((k_grid_points_backward<T, true>), dim3((unsigned)nb), dim3(kBlock), 0, s, g->dim, g->n,
+                           g->rule, g->gl_nodes, P, span, (const T*)grad_points, (double*)ws);
+    else
+        hipLaunchKernelGGL((k_grid_points_backward<T, false>), dim3((unsigned)nb), dim3(kBlock), 0, s, g->dim, g->n,
+                           g->rule, g->gl_nodes, P, span, (const T*)grad_points, (double*)ws);
+    const int rc = check_launch("k_grid_points_backward");
+    if (rc) return rc;
+    hipLaunchKernelGGL((k_grid_points_backward_finalize<T>), dim3(g->dim * 2), dim3(kBlock), 0, s, (const double*)ws,
+                       nb, g->dim, (T*)grad_domain);
+    return check_launch("k_grid_points_backward_finalize");
+}
+
+extern "C" {
 
 int tq_grid_points_backward(const tq_grid_desc* g, const void* domain, const void* grad_points, void* workspace,
                             size_t workspace_bytes, void* grad_domain, void* stream) {
@@ -840,38 +1032,10 @@ int tq_grid_points_backward(const tq_grid_desc* g, const void* domain, const voi
     rc = check_gl_tables(g);
     if (rc) return rc;
     if (!domain || !grad_points || !grad_domain) return fail(TQ_E_NULL, "domain/grad_points/grad_domain is NULL");
-    long long P;
-    ipow_checked(g->n, g->dim, 1LL << 62, &P);
-    int bd;
-    long long nb;
-    points_backward_shape(g->dim, P, &bd, &nb);
-    const size_t need = (size_t)(nb * g->dim * 2) * sizeof(double);
-    if (!workspace || workspace_bytes < need) return fail(TQ_E_WORKSPACE, "points backward workspace too small");
-    Strides strides;
-    long long st = 1;
-    for (int k = g->dim - 1; k >= 0; --k) {
-        strides.s[k] = st;
-        st *= g->n;
-    }
-    hipStream_t s = as_stream(stream);
-    if (g->dtype == TQ_F32) {
-        hipLaunchKernelGGL((k_grid_points_backward<float>), dim3((unsigned)nb), dim3(bd), 0, s, g->dim, g->n,
-                           g->rule, g->gl_nodes, strides, P, (const float*)grad_points,
-                           (double*)workspace);
-        rc = check_launch("k_grid_points_backward");
-        if (rc) return rc;
-        hipLaunchKernelGGL((k_grid_points_backward_finalize<float>), dim3(g->dim * 2), dim3(kBlock), 0, s,
-                           (const double*)workspace, nb, g->dim, (float*)grad_domain);
-    } else {
-        hipLaunchKernelGGL((k_grid_points_backward<double>), dim3((unsigned)nb), dim3(bd), 0, s, g->dim, g->n,
-                           g->rule, g->gl_nodes, strides, P, (const double*)grad_points,
-                           (double*)workspace);
-        rc = check_launch("k_grid_points_backward");
-        if (rc) return rc;
-        hipLaunchKernelGGL((k_grid_points_backward_finalize<double>), dim3(g->dim * 2), dim3(kBlock), 0, s,
-                           (const double*)workspace, nb, g->dim, (double*)grad_domain);
-    }
-    return check_launch("k_grid_points_backward_finalize");
+    if (g->dtype == TQ_F32)
+        return launch_points_backward<float>(g, grad_points, workspace, workspace_bytes, grad_domain,
+                                             as_stream(stream));
+    return launch_points_backward<double>(g, grad_points, workspace, workspace_bytes, grad_domain, as_stream(stream));
 }
 
 }  // extern "C"

@@ -50,6 +50,15 @@ class _GridReduceFn(torch.autograd.Function):
         rule, dim, n, unit, gl, npoints, vdtype, has_hs = ctx.meta
         hs = hs_saved if has_hs else None
         grad_values = grad_domain = grad_hs = None
+        if not torch.is_grad_enabled() and not has_hs:
+            # plain backward (no graph of it is recorded) with the scale taken from the domain
+            grad_values, grad_domain = _ops.grid_reduce_vjp(
+                rule, dim, n, domain.detach(), grad_out, out, npoints, None, unit, gl,
+                ctx.needs_input_grad[0], ctx.needs_input_grad[1],
+            )
+            if grad_values is not None:
+                grad_values = grad_values.to(vdtype)
+            return grad_values, grad_domain, None, None, None, None, None, None
         if ctx.needs_input_grad[0]:
             grad_values = _ops.grid_reduce_backward(
                 rule, dim, n, domain.detach(), grad_out, npoints, hs, unit, gl
@@ -153,7 +162,15 @@ class GridIntegrator(BaseIntegrator):
         if self._tq_standard():
             # user callable: HIP points -> fn -> HIP weighted reduction with the
             # rule's own weights (no [N] weight tensor is built)
-            grid_points, hs, n_per_dim = self.calculate_grid(N, domain)
+            if type(self).calculate_grid is GridIntegrator.calculate_grid:
+                # Gaussian rules scale by the domain, and so do Newton-Cotes rules whose domain carries
+                # a gradient (h = width / (n - 1) there too): neither forms the mesh widths
+                gauss = self._tq_rule == _ops.RULES["gauss_legendre"]
+                grid = IntegrationGrid(self._adjust_N(dim=dim, N=N), domain, self._grid_func,
+                                       _with_h=not (gauss or _needs_grad(domain)))
+                grid_points, hs, n_per_dim = grid.points, grid.h, grid._N
+            else:
+                grid_points, hs, n_per_dim = self.calculate_grid(N, domain)
             logger.debug("Evaluating integrand on the grid.")
             function_values, num_points = self.evaluate_integrand(fn, grid_points)
             self._nr_of_fevals = num_points

@@ -68,7 +68,9 @@ class IntegrationGrid:
     _dim = None
     _runtime = None
 
-    def __init__(self, N, integration_domain, grid_func=grid_func, disable_integration_domain_check=False):
+    def __init__(self, N, integration_domain, grid_func=grid_func, disable_integration_domain_check=False,
+                 _with_h=True):
+        # _with_h False: h stays None on the standard grids (for callers that scale by the domain)
         start = perf_counter()
         self._check_inputs(N, integration_domain, disable_integration_domain_check)
         if not isinstance(integration_domain, torch.Tensor):
@@ -98,8 +100,12 @@ class IntegrationGrid:
             else:
                 rule = _ops.RULES["gauss_legendre"]
                 gl = gl_provider(self._N, dom.device)
-            self.h = standard_h(rule, self._dim, self._N, dom, gl)
-            self.points = standard_points(rule, self._dim, self._N, dom, gl)
+            if _with_h and not (requires_grad and torch.is_grad_enabled()):
+                self.points, self.h = _ops.grid_points_h(rule, self._dim, self._N, dom, gl)
+            else:
+                if _with_h:
+                    self.h = standard_h(rule, self._dim, self._N, dom, gl)
+                self.points = standard_points(rule, self._dim, self._N, dom, gl)
         else:
             grid_1d = [
                 grid_func(integration_domain[d], self._N, requires_grad=requires_grad, backend="torch")
