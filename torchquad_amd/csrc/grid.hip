@@ -1,4 +1,8 @@
-// Tensor-product grid rules (Trapezoid, Simpson, Boole, Gauss-Legendre).
+// Tensor-product grid rules (Trapezoid, Simpson, Boole, Gauss-Legendre):
+// the point-by-point fused kernel, which integrals of one or two axes and of
+// axes too long for grid_product.hip's tables take (that kernel needs every
+// axis's factors in FP64 first, which pays from three axes on: trapezoid d=2
+// n=1000 9.7 us here, 13 us there), and the kernels of user integrands.
 //
 // Index space.  The n^d grid points (ij order, last axis fastest, as
 // IntegrationGrid.points in integration_grid.py:98-99) are split into
@@ -16,6 +20,7 @@
 #include <mutex>
 
 #include "tq_host.hpp"
+#include "tq_grid_launch.hpp"
 #include "tq_grid_tile.hpp"
 #include "tq_values.hpp"
 
@@ -29,25 +34,12 @@ struct GridArgs {
     const T* domain;
     const double* glx;
     const double* glw;
-    double* partials;
-    unsigned int* done;  // blocks finished; zero between launches
+    BlockSums sums;
     T* out;
     double* out64;
     double c0;
     Params<T> p;
 };
-
-// Workspace of the fused kernel: completion counters in the first
-// kWsHeader bytes (zero before the first launch, and every launch leaves
-// them zero), then one FP64 partial per workgroup.  Workgroup b counts into
-// group counter b % kDoneGroups; the last workgroup of each group counts
-// into the top counter, whose last arrival sums the partials.  One counter
-// for all workgroups serialised their atomics at about 15 ns each (10112
-// workgroups: 148 us for 3.9e7 evaluations).
-constexpr int kDoneGroups = 16;
-constexpr int kDoneStride = 64;  // words between counters (256 bytes; 4 KB measured the same)
-constexpr int kDoneTop = kDoneGroups * kDoneStride;
-constexpr size_t kWsHeader = ((size_t)(kDoneTop + 1) * sizeof(unsigned int) + 255) & ~(size_t)255;
 
 static int check_grid_desc(const tq_grid_desc* g, int max_dim) {
     if (!g) return fail(TQ_E_NULL, "grid descriptor is NULL");
@@ -81,15 +73,8 @@ static int check_gl_tables(const tq_grid_desc* g) {
     return TQ_OK;
 }
 
-// LDS for a merged (two-axis) loop table in the fused kernel; any cap of at
-// least 1024 entries gives the same launch size (see kMergeMaxN).
-constexpr size_t kFusedMergeLds = 40 * 1024;
-
-inline long long fused_merge_cap(int fam, int tsize) {
-    const long long cap = (long long)(kFusedMergeLds / ((size_t)tab_stride(fam) * tsize));
-    return cap > 1024 ? cap : 1024;
-}
-
+// merge_cap 1024: the plan that workspaces are sized by (at least as many
+// workgroups as any launch takes).
 static int make_geom(const tq_grid_desc* gd, GridGeom& G, long long merge_cap = 1024) {
     return plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, 16384, G, merge_cap);
 }
@@ -98,19 +83,12 @@ static int make_geom(const tq_grid_desc* gd, GridGeom& G, long long merge_cap = 
 // Fused kernel
 // ---------------------------------------------------------------------------
 // Dynamic LDS of the fused kernel: [row weights: L*n FP64][loop table:
-// S*nl T][row contributions: slots*L*n T] (the row parts only when ROWTAB),
-// then for a two-axis loop, 8-byte aligned, the loop axes' table weights (2n FP64: weights or their keys)
-// and nodes (2n T) from which the table is built.
-template <typename T, int FAM>
-__host__ __device__ inline size_t fused_pair_offset(const GridGeom& G, bool rowtab) {
-    constexpr int S = TabStride<FAM>::v;
-    size_t b = (size_t)S * G.nl * sizeof(T);
-    if (rowtab) b += (size_t)G.L * G.n * (sizeof(double) + StateSlots<FAM>::v * sizeof(T));
-    return (b + 7) & ~(size_t)7;
-}
+// S*nl T][row contributions: slots*L*n T] (the row parts only when ROWTAB).
 template <typename T, int FAM>
 inline size_t fused_lds_bytes(const GridGeom& G, bool rowtab) {
-    return fused_pair_offset<T, FAM>(G, rowtab) + (G.q == 2 ? (size_t)2 * G.n * (sizeof(double) + sizeof(T)) : 0);
+    size_t b = (size_t)TabStride<FAM>::v * G.nl * sizeof(T);
+    if (rowtab) b += (size_t)G.L * G.n * (sizeof(double) + StateSlots<FAM>::v * sizeof(T));
+    return b;
 }
 constexpr size_t kFusedLdsMax = 48 * 1024;
 
@@ -131,22 +109,8 @@ __global__ __launch_bounds__(BW * kWave) void k_grid_fused(GridArgs<T> A) {
     T* s_tab = reinterpret_cast<T*>(smem_raw + (ROWTAB ? (size_t)L * n * sizeof(double) : 0));
     T* s_rt = s_tab + (size_t)TabStride<FAM>::v * g.nl;
     if (TABLE) {
-        // Two loop axes: their 2n nodes and weights first, so that each of
-        // the n^2 entries costs two folds and a product instead of a
-        // division for its indices and two node and weight evaluations.
-        const bool pair = g.q == 2;
-        double* s_pw = reinterpret_cast<double*>(smem_raw + fused_pair_offset<T, FAM>(g, ROWTAB));
-        T* s_px = reinterpret_cast<T*>(s_pw + 2 * n);
-        if (pair) {
-            for (int e = tid; e < 2 * n; e += NT) {
-                const int j = e < n ? e : e - n;
-                s_px[e] = (T)node_of(s_axis[e < n ? L : L + 1], j, n, rule, A.glx);
-                s_pw[e] = table_weight<T, FAM>(weight_of(rule, j, n, A.glw));
-            }
-        } else {
-            for (int j = tid; j < g.nl; j += NT)
-                loop_table_entry<T, FAM>(s_tab, j, s_axis, L, 1, n, rule, A.glx, A.glw, A.p);
-        }
+        for (int j = tid; j < g.nl; j += NT)
+            loop_table_entry<T, FAM>(s_tab, j, s_axis, L, 1, n, rule, A.glx, A.glw, A.p);
         if (ROWTAB)
             for (int e = tid; e < L * n; e += NT) {
                 const int k = e / n;
@@ -154,22 +118,6 @@ __global__ __launch_bounds__(BW * kWave) void k_grid_fused(GridArgs<T> A) {
                                         A.p);
             }
         __syncthreads();
-        if (pair) {
-            const AxisC<T> c1 = axis_c(A.p, L), c2 = axis_c(A.p, L + 1);
-            // entry j = j1 n + j2, stepped by NT without a division per entry
-            int j1 = tid / n, j2 = tid - j1 * n;
-            const int s1 = NT / n, s2 = NT - s1 * n;
-            for (int j = tid; j < g.nl; j += NT) {
-                pair_table_entry<T, FAM>(s_tab, j, s_px[j1], s_px[n + j2], s_pw[j1], s_pw[n + j2], c1, c2, A.p);
-                j1 += s1;
-                j2 += s2;
-                if (j2 >= n) {
-                    j2 -= n;
-                    ++j1;
-                }
-            }
-            __syncthreads();
-        }
     }
     // readfirstlane: the wave index is uniform, so the tile loop runs on SGPRs
     const long long wave = (long long)blockIdx.x * BW + __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -184,41 +132,8 @@ __global__ __launch_bounds__(BW * kWave) void k_grid_fused(GridArgs<T> A) {
         acc = grid_tile<T, FAM, TABLE, ROWTAB>(d, n, g.nl, g.m, L, rule, g.lane_count, A.p, s_axis, s_tab, A.glx,
                                                A.glw, lw, t0, t1, s_rt, s_rw);
     }
-    const double bs = block_sum(acc, s_red);
-    // The last block to finish sums every block's partial in a fixed order
-    // (independent of which block is last) and applies the per-axis scale:
-    // partial store, device-scope release, counter; the last block acquires
-    // before reading the partials and resets the counter for the next launch.
-    // Release writes this workgroup's partial back to device scope (no L2
-    // invalidate, which a full fence in every workgroup would add); only
-    // the last workgroup acquires.
-    // Counting goes through kDoneGroups group counters: the last arrival of
-    // a group acquires its group's partials and releases them on to the top
-    // counter, so the final block sees every partial.
-    __shared__ bool s_last;
-    if (tid == 0) {
-        A.partials[blockIdx.x] = bs;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const unsigned nb = gridDim.x, grp = blockIdx.x % kDoneGroups;
-        const unsigned members = (nb - 1 - grp) / kDoneGroups + 1;  // blocks b < nb with b % kDoneGroups == grp
-        unsigned int* gc = A.done + grp * kDoneStride;
-        bool last = false;
-        if (__hip_atomic_fetch_add(gc, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == members - 1) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            __hip_atomic_store(gc, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            const unsigned groups = nb < (unsigned)kDoneGroups ? nb : (unsigned)kDoneGroups;
-            last = __hip_atomic_fetch_add(A.done + kDoneTop, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                   groups - 1;
-        }
-        s_last = last;
-    }
-    __syncthreads();
-    if (!s_last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    double v = 0.0;
-    for (unsigned i = tid; i < gridDim.x; i += NT) v += A.partials[i];
-    v = block_sum(v, s_red);
+    double v;
+    if (!sum_over_blocks(acc, A.sums, s_red, &v)) return;
     if (tid == 0) {
         double scale = A.c0;
         for (int k = 0; k < d; ++k)
@@ -226,7 +141,6 @@ __global__ __launch_bounds__(BW * kWave) void k_grid_fused(GridArgs<T> A) {
         const double r = v * scale;
         if (A.out) *A.out = (T)r;
         if (A.out64) *A.out64 = r;
-        __hip_atomic_store(A.done + kDoneTop, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -347,17 +261,23 @@ template <typename T>
 static int launch_grid(const tq_grid_desc* gd, const tq_integrand* f, const void* domain,
                        void* ws, size_t ws_bytes, void* out, double* out64, hipStream_t st) {
     GridGeom G;
-    int rc = make_geom(gd, G, fused_merge_cap(f->family, (int)sizeof(T)));
+    int rc = make_geom(gd, G);
     if (rc) return rc;
     const size_t need = kWsHeader + (size_t)G.blocks * sizeof(double);
     if (!ws || ws_bytes < need) return fail(TQ_E_WORKSPACE, "grid workspace too small");
+    bool taken = false;
+    rc = launch_grid_product<T>(gd, f, domain, ws, ws_bytes, out, out64, st, &taken);
+    if (rc || taken) return rc;
+    // one loop axis: the integrals that could merge two take the product kernel
+    rc = make_geom(gd, G, 0);
+    if (rc) return rc;
+    if (ws_bytes < kWsHeader + (size_t)G.blocks * sizeof(double)) return fail(TQ_E_WORKSPACE, "grid workspace too small");
     GridArgs<T> A;
     A.g = G;
     A.domain = (const T*)domain;
     A.glx = gd->gl_nodes;
     A.glw = gd->gl_weights;
-    A.done = (unsigned int*)ws;
-    A.partials = (double*)((unsigned char*)ws + kWsHeader);
+    A.sums = block_sums(ws);
     A.out = (T*)out;
     A.out64 = out64;
     A.c0 = f->c0;

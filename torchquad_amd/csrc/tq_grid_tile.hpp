@@ -73,6 +73,17 @@ __device__ __host__ inline double axis_scale(double a, double b, int n, int rule
     }
 }
 
+// axis_scale from an axis's map: the spacing (Newton-Cotes) or half width is
+// already there, so no second division is waited for.
+__device__ inline double axis_scale_of(const Axis& ax, int rule) {
+    switch (rule) {
+        case TQ_RULE_TRAPEZOID: return ax.h * 0.5;
+        case TQ_RULE_SIMPSON: return ax.h * (1.0 / 3.0);
+        case TQ_RULE_BOOLE: return ax.h * (1.0 / 22.5);
+        default: return ax.a;
+    }
+}
+
 // Loop LDS table: entry j holds the loop's contribution to the integrand
 // state at its point j (fold_c(zero, c_L, x_j) for one loop axis, both axes
 // folded for two), then the point's weight; per point the tile loop only
