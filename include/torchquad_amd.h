@@ -241,27 +241,30 @@ typedef struct tq_batch_tile {
 } tq_batch_tile;
 
 /* Host-side plan sizes: bytes of the device descriptor array and tile count
- * for tiles of about tile_points points. */
+ * for tiles of about tile_points points (16 times as many where a workgroup
+ * takes a tile). */
 int tq_batch_plan_sizes(const tq_batch_item* items, int64_t count, int32_t dtype, int64_t tile_points,
                         int64_t* desc_bytes, int64_t* n_tiles);
 /* Host-side plan: descriptors (desc_out, host memory of desc_bytes), tiles
  * ordered by kernel class and, within a class, longest integral first, each
  * integral's tiles contiguous; tile_begin[i] / tile_count[i] for integral i.
  * class_offsets (optional, [5]): tiles [class_offsets[c], class_offsets[c+1])
- * belong to class c -- 0: one-axis integrals; multi-axis ones with 1: loop
- * and row-axis tables within 4 KB of LDS per wave (or no loop axis), 2:
- * within 8 KB, 3: larger (general kernel). */
+ * belong to class c -- 0: one-axis integrals; multi-axis ones whose factor
+ * tables take 1: up to 26 KB of LDS, 2: up to 60 KB, 3: more (general
+ * kernel).  In classes 1 and 2 a tile's lane groups and items are those of
+ * the product kernel's split of the axes (items: groups of four loop points). */
 int tq_batch_plan(const tq_batch_item* items, int64_t count, int32_t dtype, int64_t tile_points, void* desc_out,
                   tq_batch_tile* tiles_out, int64_t* tile_begin, int64_t* tile_count, int64_t* class_offsets);
-/* Runs a plan whose arrays were copied to the device: one kernel per
- * non-empty class, one wave per tile in the plan's order (longest integrals
- * first, so the hardware dispatcher hands out the large tiles first), then
- * out[i] (dtype) / out64[i] = integral i.  With more than one non-empty
- * class the classes run concurrently on two library-owned streams forked
- * from `stream` and joined back into it with events (under graph capture
- * the run becomes a forked subgraph).  tile_partials: [n_tiles];
- * class_offsets: host [5] from tq_batch_plan, or NULL to run every tile on
- * a general kernel that carries both the one-axis and multi-axis code.  gl_nodes / gl_weights: every Gauss-Legendre item's
+/* Runs a plan whose arrays were copied to the device, tiles in the plan's
+ * order (longest integrals first, so the hardware dispatcher hands out the
+ * large tiles first): classes 0 and 1 in one launch (one wave and one
+ * workgroup per tile), class 2 (one workgroup) and class 3 (one wave) in one
+ * each where they have tiles; then out[i] (dtype) / out64[i] = integral i.
+ * When both of the former and of the latter have tiles, classes 2 and 3 run
+ * on a library-owned stream forked from `stream` and joined back into it with
+ * events (under graph capture the run becomes a forked subgraph).
+ * tile_partials: [n_tiles]; class_offsets: host [5] from tq_batch_plan, or
+ * NULL to hand every tile to two kernels of which each takes its own.  gl_nodes / gl_weights: every Gauss-Legendre item's
  * table at its gl_offset, gl_len entries each; gl_pairs32 (optional, F32
  * batches only, else ignored): the same tables as interleaved FP32 (node,
  * weight) pairs, pair k at [2 (gl_offset + k)], read by one-axis items

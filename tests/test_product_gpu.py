@@ -160,3 +160,48 @@ def test_product_custom_weights(dev):
         per_axis = np.sum(wn * np.exp(-((r - 0.25) ** 2)))
         scale = np.sum(np.abs(wn) * np.exp(-((r - 0.25) ** 2))) ** 3
         assert abs(got - per_axis**3) <= bar * scale
+
+
+def _batch_item(rule, fam, d, n, seed):
+    fn, factors = _make(fam, d, seed)
+    return {"rule": rule, "fn": fn, "dim": d, "n": n, "domain": [[-0.75, 1.25], [-1.0, 0.5]] * (d // 2)
+            + [[-0.75, 1.25]] * (d % 2)}, factors
+
+
+# (dim, n): two axes, table classes (26 and 60 KB), axes too long for them, one and two loop axes (n = 32, 33),
+# more lane groups than tiles, more tiles than lane groups, no full lane group, rows
+BATCH = [(2, 2), (2, 33), (2, 129), (2, 701), (2, 2301), (3, 2), (3, 21), (3, 32), (3, 33), (3, 101), (4, 5), (4, 31),
+         (5, 9), (6, 10), (7, 3), (8, 5)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("rule", ["trapezoid", "simpson", "gauss_legendre"])
+@pytest.mark.parametrize("tile_points", [64, 8192, 1 << 20])
+def test_batch_product_sizes(tile_points, rule, dtype, dev, parity):
+    """Every family at every size in one batch, with classes and (the same
+    tiles on the general kernel) without."""
+    from torchquad_amd import _lib
+    from torchquad_amd.batch import Batch
+
+    specs = []
+    for d, n in BATCH:
+        if tile_points == 64 and n**d > 2e5:
+            continue  # tens of thousands of tiles say nothing new
+        if rule == "simpson" and n % 2 == 0:
+            n += 1
+        for fam in FAMILIES:
+            specs.append((fam, d, n, *_batch_item(rule, fam, d, n, 31 * d + n)))
+    b = Batch([s[3] for s in specs], dtype=dtype, device=dev, tile_points=tile_points)
+    out64 = b.run()[1].clone()
+    alone = torch.empty_like(out64)
+    _lib.call("tq_batch_run", b.dt, _lib.ptr(b.desc), b.count, _lib.ptr(b.tiles), b.n_tiles, _lib.ptr(b.tile_begin),
+              _lib.ptr(b.tile_count), _lib.ptr(b.gl_x), _lib.ptr(b.gl_w), _lib.ptr(b.gl_p32),
+              b.gl_x.numel() if b.gl_x is not None else 0, _lib.ptr(b.tile_part), None, _lib.ptr(alone), None,
+              _lib.stream_ptr(dev))
+    bar = 1e-6 if dtype == torch.float32 else 1e-12
+    for i, (fam, d, n, item, factors) in enumerate(specs):
+        gl = gauss_legendre(n, device=dev) if rule == "gauss_legendre" else None
+        ref, scale = _reference(fam, item["fn"], factors, rule, item["domain"], n, gl)
+        for v in (float(out64[i]), float(alone[i])):
+            parity.record(abs(v - ref) / scale, bar)
+            assert abs(v - ref) <= bar * scale, (fam, d, n, v, ref)

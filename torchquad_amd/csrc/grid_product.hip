@@ -1,15 +1,22 @@
 // The fused grid kernel of integrals with at least two axes whose factor
 // tables fit in LDS (tq_product.hpp says how values become products).
 //
-// Index space: the last m axes are spread over lanes, K combinations per
-// lane (64 K per wave); the loop runs over one or two axes whose combined
-// factors form an LDS table; the leading axes are rows, their factors merged
-// into the lane's states once per row.  A wave owns one group of 64 K lane
-// combinations and a contiguous range of (row, group of four loop points).
+// Index space (ProductSplit): lanes hold K combinations of the last axes, the
+// loop runs over one or two axes whose combined factors form an LDS table,
+// and the leading axes are rows, their factors merged into the states once
+// per row.  A wave owns one group of 64 lane slots and a contiguous range of
+// (row, group of four loop points).
 #include "tq_grid_launch.hpp"
 #include "tq_product.hpp"
 
 namespace tq {
+
+struct ProductGeom {
+    ProductSplit s;
+    int rule, K;
+    long long ipw;  // items per wave
+    long long num_waves, blocks;
+};
 
 template <typename T>
 struct ProductArgs {
@@ -35,107 +42,31 @@ constexpr int product_waves_per_simd(int fam, int tsize) {
 
 template <typename T, int FAM, int K>
 __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, sizeof(T))) void k_grid_product(ProductArgs<T> A) {
-    using F = Factor<FAM, T>;
-    constexpr int C = F::C, nt = kProductWaves * kWave;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ Axis s_axis[TQ_MAX_DIM];
-    __shared__ int s_top[TQ_MAX_DIM], s_exp[TQ_MAX_DIM];
+    __shared__ int s_exp[TQ_MAX_DIM];
     __shared__ double s_red[kProductWaves], s_scale[TQ_MAX_DIM];
     const ProductGeom& g = A.g;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int d = g.d, n = g.n, L = g.L, total = d * n, entries = g.groups * kGroup;
+    const int tid = threadIdx.x, d = g.s.d;
     if (tid < d) {
-        const Axis a = make_axis(A.domain, tid, n, g.rule);
+        const Axis a = make_axis(A.domain, tid, g.s.n, g.rule);
         s_axis[tid] = a;
         s_scale[tid] = axis_scale_of(a, g.rule);
     }
     __syncthreads();
-    T* axis = reinterpret_cast<T*>(smem_raw);
-    unsigned char* second = smem_raw + (((size_t)C * total * sizeof(T) + 15) & ~(size_t)15);
-    T* tab = reinterpret_cast<T*>(second);
-    build_axis_factors<FAM, T>(d, n, g.rule, s_axis, A.glx, A.glw, A.p, g.by_n, axis,
-                               reinterpret_cast<double*>(second), s_top, s_exp);
-    // Loop table, over the FP64 copies (they are done with).  Four entries
-    // per thread and trip: their reads go out together.
-    for (int e0 = tid; e0 < entries; e0 += 4 * nt) {
-        F f[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = e0 + i * nt;
-            f[i] = F::one(false);
-            if (e < g.nl) {
-                if (g.q == 2) {
-                    const int j1 = (int)g.by_n.div((uint32_t)e);
-                    f[i] = F::merge(axis_factor<FAM, T>(axis, total, L * n + j1),
-                                    axis_factor<FAM, T>(axis, total, (L + 1) * n + e - j1 * n));
-                } else {
-                    f[i] = axis_factor<FAM, T>(axis, total, L * n + e);
-                }
-                f[i] = f[i].dual();
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int c = 0; c < C; ++c)
-                if (e0 + i * nt < entries) tab[c * entries + e0 + i * nt] = f[i].v[c];
-    }
-    __syncthreads();
+    const ProductTables<T> tab = build_product_tables<FAM, T>(g.s, g.rule, s_axis, A.glx, A.glw, A.p, smem_raw, s_exp);
 
     double acc = 0.0;
     const long long wave = (long long)blockIdx.x * kProductWaves + __builtin_amdgcn_readfirstlane(tid >> 6);
     if (wave < g.num_waves) {
-        const unsigned uw = (unsigned)wave, ulg = (unsigned)g.lane_groups;
+        const unsigned uw = (unsigned)wave, ulg = (unsigned)g.s.lane_groups;
         const unsigned chunk = uw / ulg;
         const int lg = (int)(uw - chunk * ulg);
         const long long t0 = (long long)chunk * g.ipw;
-        const long long t1 = t0 + g.ipw < g.items ? t0 + g.ipw : g.items;
-        // the lane's K states over the lane axes; lanes past the last combination carry zeros
-        F own[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const int slot = (lg * K + k) * kWave + lane;
-            const bool on = slot < g.lane_count;
-            uint32_t r = on ? (uint32_t)slot : 0u;
-            own[k] = F::one(on);
-            for (int a = d - 1; a >= d - g.m; --a) {
-                const uint32_t q = g.by_n.div(r);
-                own[k] = F::merge(own[k], axis_factor<FAM, T>(axis, total, a * n + (int)(r - q * g.by_n.n)));
-                r = q;
-            }
-        }
-        if (L == 0) {
-            acc = sum_entries<FAM, T, K>(own, tab, entries, (int)t0, (int)t1);
-        } else {
-            // row odometer: lane k of `dig` holds the digit of row axis k
-            long long row = t0 / g.groups;
-            int gi = (int)(t0 - row * g.groups);
-            int dig = 0;
-            for (int k = L - 1; k >= 0; --k) {
-                const long long q = row / n;
-                dig = lane == k ? (int)(row - q * n) : dig;
-                row = q;
-            }
-            for (long long t = t0; t < t1;) {
-                F rf = F::one(true);
-                for (int k = 0; k < L; ++k)
-                    rf = F::merge(rf, axis_factor<FAM, T>(axis, total, k * n + __builtin_amdgcn_readlane(dig, k)));
-                F s[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) s[k] = F::merge(own[k], rf);
-                const int left = g.groups - gi;
-                const int ge = t1 - t < left ? gi + (int)(t1 - t) : g.groups;
-                acc += sum_entries<FAM, T, K>(s, tab, entries, gi, ge);
-                t += ge - gi;
-                gi = 0;
-                for (int k = L - 1; k >= 0; --k) {
-                    const int dk = __builtin_amdgcn_readlane(dig, k) + 1;
-                    const bool wrap = dk >= n;
-                    dig = lane == k ? (wrap ? 0 : dk) : dig;
-                    if (!wrap) break;
-                }
-            }
-        }
+        const long long t1 = t0 + g.ipw < g.s.items ? t0 + g.ipw : g.s.items;
+        Factor<FAM, T> own[K];
+        lane_states<FAM, T, K>(g.s, tab, lg * kWave + (tid & (kWave - 1)), own);
+        acc = sum_items<FAM, T, K>(g.s, tab, own, t0, t1);
     }
     double v;
     if (!sum_over_blocks(acc, A.sums, s_red, &v)) return;
@@ -144,7 +75,7 @@ __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, 
         int exponent = 0;
         for (int k = 0; k < d; ++k) {
             scale *= s_scale[k];
-            exponent += s_exp[k];
+            exponent += exp_or_zero(s_exp[k]);
         }
         const double r = ldexp(v, exponent) * scale;
         if (A.out) *A.out = (T)r;
@@ -152,19 +83,16 @@ __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, 
     }
 }
 
-// LDS of a merged (two-axis) loop table, and of all tables.
+// LDS of a two-axis loop table, of a two-axis outer table, and of all tables.
 constexpr size_t kProductLoopLds = 40 * 1024;
+constexpr size_t kProductOuterLds = 20 * 1024;
 constexpr size_t kProductLdsMax = 60 * 1024;
 
 // Plan; false: the grid does not take this kernel.
-static bool plan_product(const tq_grid_desc* gd, int C, int tsize, int cus, ProductGeom& G) {
+static bool plan_product(const tq_grid_desc* gd, int C, int tsize, ProductGeom& G) {
     const int d = gd->dim, n = gd->n;
-    if (d < 3 || n < 2) return false;
-    G.d = d;
-    G.n = n;
+    if (d < 3) return false;
     G.rule = gd->rule;
-    G.by_n = make_fast_div((uint32_t)n);
-    if ((size_t)C * d * n * (sizeof(double) + tsize) > kProductLdsMax) return false;
     double P = 1.0;
     for (int k = 0; k < d; ++k) P *= n;
     // States per lane (they share the LDS reads of the loop entries) where
@@ -174,43 +102,10 @@ static bool plan_product(const tq_grid_desc* gd, int C, int tsize, int cus, Prod
     const int kmax = tsize == 4 ? 8 : 4;
     G.K = 1;
     while (G.K < kmax && P >= (double)(4 * G.K * G.K) * (1 << 21)) G.K *= 2;
-    // Loop axes: two when their table fits and a lane axis remains, so the
-    // per-row work (state merges, FP64 flush) comes once per n^2 points.
-    G.q = (d >= 3 && (size_t)C * ((size_t)n * n + kGroup) * tsize <= kProductLoopLds) ? 2 : 1;
-    // Lane axes: the fewest that fill 95 % of the 64 K slots of their waves,
-    // else the best filling count.
-    const int mmax = d - G.q;
-    int m = 1;
-    if (gd->lane_axes > 0) {
-        m = gd->lane_axes < d ? gd->lane_axes : d - 1;
-        if (m > mmax) G.q = 1;
-    } else {
-        double best = -1.0, c = 1.0;
-        for (int k = 1; k <= mmax; ++k) {
-            c *= n;
-            if (c > (double)(1 << 30)) break;
-            const double slots = (double)kWave * G.K;
-            const double fill = c / (std::ceil(c / slots) * slots);
-            if (fill > best) {
-                best = fill;
-                m = k;
-            }
-            if (fill >= 0.95) break;
-        }
-    }
-    G.m = m;
-    G.L = d - m - G.q;
-    long long lc;
-    if (ipow_checked(n, m, 1LL << 30, &lc) != 0) return false;
-    G.lane_count = (int)lc;
-    G.lane_groups = (int)((lc + kWave * G.K - 1) / (kWave * G.K));
-    G.nl = G.q == 2 ? n * n : n;
-    G.groups = (G.nl + kGroup - 1) / kGroup;
-    if (product_lds_bytes(G, C, tsize) > kProductLdsMax) return false;
-    long long rows;
-    if (ipow_checked(n, G.L, (1LL << 62) / G.groups, &rows) != 0) return false;
-    G.items = rows * G.groups;
-    return true;
+    const long long entry = (long long)C * tsize;
+    const int lane_axes = gd->lane_axes > 0 ? (gd->lane_axes < d ? gd->lane_axes : d - 1) : 0;
+    return split_product_axes(d, n, G.K, C, tsize, (long long)kProductLoopLds / entry,
+                              G.K > 1 ? (long long)kProductOuterLds / entry : 0, lane_axes, kProductLdsMax, G.s);
 }
 
 // Splits the items over waves and the waves over blocks: one fill of the
@@ -228,23 +123,23 @@ static void split_product(ProductGeom& G, long long items_per_wave, int waves_pe
     long long ipw = items_per_wave > 0 ? (items_per_wave + kGroup - 1) / kGroup : 0;
     if (ipw <= 0) {
         const long long waves = 4LL * cus * waves_per_simd;
-        long long per = waves / G.lane_groups;
+        long long per = waves / G.s.lane_groups;
         if (per < 1) per = 1;
-        ipw = (G.items + per - 1) / per;
+        ipw = (G.s.items + per - 1) / per;
         if (ipw < kLeastItems) ipw = kLeastItems;
     }
-    if (ipw > G.items) ipw = G.items;
+    if (ipw > G.s.items) ipw = G.s.items;
     for (;; ipw *= 2) {
         G.ipw = ipw;
-        G.num_waves = ((G.items + ipw - 1) / ipw) * (long long)G.lane_groups;
+        G.num_waves = ((G.s.items + ipw - 1) / ipw) * (long long)G.s.lane_groups;
         G.blocks = (G.num_waves + kProductWaves - 1) / kProductWaves;
-        if (G.blocks <= max_blocks || ipw >= G.items) return;
+        if (G.blocks <= max_blocks || ipw >= G.s.items) return;
     }
 }
 
 template <typename T, int FAM>
 static int launch_family(ProductGeom& G, ProductArgs<T>& A, hipStream_t st) {
-    const size_t lds = product_lds_bytes(G, family_comps(FAM), (int)sizeof(T));
+    const size_t lds = product_lds_bytes(G.s, family_comps(FAM), (int)sizeof(T));
     A.g = G;
     const dim3 grid((unsigned)G.blocks), block(kProductWaves * kWave);
     switch (G.K) {
@@ -264,8 +159,8 @@ int launch_grid_product(const tq_grid_desc* gd, const tq_integrand* f, const voi
     *taken = false;
     ProductGeom G;
     const int cus = device_cus();
-    if (cus <= 0 || !plan_product(gd, family_comps(f->family), (int)sizeof(T), cus, G)) return TQ_OK;
-    const bool many = family_comps(f->family) * G.d * G.n > kManyFactors;
+    if (cus <= 0 || !plan_product(gd, family_comps(f->family), (int)sizeof(T), G)) return TQ_OK;
+    const bool many = family_comps(f->family) * G.s.d * G.s.n > kManyFactors;
     split_product(G, gd->items_per_wave, many ? 2 : product_waves_per_simd(f->family, (int)sizeof(T)), cus,
                   (long long)((ws_bytes - kWsHeader) / sizeof(double)));
     if (kWsHeader + (size_t)G.blocks * sizeof(double) > ws_bytes || G.num_waves > 0x7fffffffLL) return TQ_OK;

@@ -237,24 +237,79 @@ __device__ inline void row_table_entry(T* rt, double* rw, int k, int j, const Ax
 // the axes between the row and lane axes: one axis, nl = n, or two, nl = n^2,
 // which needs the table).  Returns the lane's weighted sum.  `ax` holds the
 // per-axis maps, `tab` the loop table (loop_table_entry) when TABLE.
-// Code paths a grid_tile instantiation carries: one-axis integrals (m == 0),
-// multi-axis ones (m > 0), or both.  The batched kernels run the two kinds in
-// separate launches, each without the other's code and live registers; an
-// integral sent to an instantiation without its path yields NaN.
-constexpr int kPathsOneAxis = 1;
+// Code paths a grid_tile instantiation carries: one-axis integrals (m == 0)
+// of Newton-Cotes and of Gauss-Legendre rules, multi-axis ones (m > 0).  The
+// batched kernels run the kinds in separate launches, each without the
+// others' code and live registers; an integral sent to an instantiation
+// without its path yields NaN.
+constexpr int kPathsNewtonCotes = 1;
 constexpr int kPathsMultiAxis = 2;
-constexpr int kPathsAll = 3;
+constexpr int kPathsGauss = 4;
+constexpr int kPathsOneAxis = kPathsNewtonCotes | kPathsGauss;
+constexpr int kPathsAll = kPathsOneAxis | kPathsMultiAxis;
+
+// Rows [t_begin, t_end) of a one-axis Gauss-Legendre integral whose folded
+// table (grid_tile's GL_FOLD) is given as FP32 (node, weight) pairs: one
+// 8-byte load per two points.  FP32 results only; node and weight carry 2^-24
+// relative rounding, far inside the FP32 tolerance.  Bound by the reads: four
+// rows' loads are issued together.
+template <int FAM>
+__device__ inline double gl_pair_rows(int n, const Params<float>& p, const Axis& a0, const float* pairs32,
+                                      long long t_begin, long long t_end) {
+    using F = Family<FAM, float>;
+    const int lane = threadIdx.x & (kWave - 1);
+    const float2* pairs = reinterpret_cast<const float2*>(pairs32);
+    const float sa = (float)a0.a, sh = (float)a0.h;
+    const State<float> s0 = F::start(p);
+    const AxisC<float> ac0 = axis_c(p, 0);
+    const int h = (n + 1) >> 1;  // nodes 0 .. h-1; for odd n node h-1 is the middle one, counted once
+    const long long last = (h - 1) / kWave;  // row of node h-1: the only one with lanes past it or a middle node
+    double acc = 0.0;
+    for (long long tb = t_begin; tb < t_end; tb += kFlush) {
+        const long long te = (tb + kFlush < t_end) ? (tb + kFlush) : t_end;
+        const long long tf = te < last ? te : last;  // whole rows
+        float fa = 0.0f;
+        auto value = [&](float x) { return F::finish(F::fold_c(s0, ac0, x, p), p); };
+        auto add = [&](float2 e) {
+            fa = fmaf(e.y, value(fmaf(sa, e.x, sh)), fa);
+            fa = fmaf(e.y, value(fmaf(-sa, e.x, sh)), fa);
+        };
+        // (one row where the sine's argument reduction would be repeated eightfold: 132 registers)
+        constexpr int U = FAM == TQ_FAM_SIN_SUM ? 1 : 4;
+        long long t = tb;
+        for (; t + U <= tf; t += U) {
+            const float2* row = pairs + t * kWave;
+            float2 e[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) e[u] = row[u * kWave + lane];
+#pragma unroll
+            for (int u = 0; u < U; ++u) add(e[u]);
+        }
+        for (; t < tf; ++t) add(pairs[t * kWave + lane]);
+        if (t < te) {
+            const int k = (int)(last * kWave) + lane;
+            float2 e = pairs[k < h ? k : h - 1];
+            const float w1 = (k < h) ? e.y : 0.0f;
+            const float w2 = (k < h && 2 * k + 1 != n) ? e.y : 0.0f;
+            fa = fmaf(w1, value(fmaf(sa, e.x, sh)), fa);
+            fa = fmaf(w2, value(fmaf(-sa, e.x, sh)), fa);
+        }
+        acc += (double)fa;
+    }
+    return acc;
+}
 
 template <typename T, int FAM, bool TABLE, bool ROWTAB = false, bool GL_FOLD = true, int PATHS = kPathsAll>
 __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule, int lane_count, const Params<T>& p,
                                    const Axis* ax, const T* tab, const double* glx, const double* glw, int lw,
                                    long long t_begin, long long t_end, const T* rt = nullptr,
-                                   const double* rw = nullptr, const float* gl_pairs32 = nullptr) {
+                                   const double* rw = nullptr) {
     using F = Family<FAM, T>;
     const int lane = threadIdx.x & (kWave - 1);
     double acc = 0.0;
     if constexpr ((PATHS & kPathsOneAxis) != 0) {
-        if (m == 0 && GL_FOLD && rule == TQ_RULE_GAUSS_LEGENDRE) {
+        if ((PATHS & kPathsGauss) == 0 && rule == TQ_RULE_GAUSS_LEGENDRE) return __longlong_as_double(0x7ff8000000000000ll);
+        if ((PATHS & kPathsGauss) != 0 && m == 0 && GL_FOLD && rule == TQ_RULE_GAUSS_LEGENDRE) {
             const State<T> s0 = F::start(p);
             const AxisC<T> ac0 = axis_c(p, 0);
             const Axis a0 = ax[0];
@@ -262,36 +317,17 @@ __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule,
             for (long long tb = t_begin; tb < t_end; tb += kFlush) {
                 const long long te = (tb + kFlush < t_end) ? (tb + kFlush) : t_end;
                 T fa = T(0);
-                if (gl_pairs32) {
-                    // FP32 (node, weight) pairs: one 8-byte load per two points
-                    // (FP32 results only; the node and weight carry 2^-24
-                    // relative rounding, far inside the FP32 tolerance)
-                    const float2* pairs = reinterpret_cast<const float2*>(gl_pairs32);
-                    const float sa = (float)a0.a, sh = (float)a0.h;
-    #pragma unroll 2
-                    for (long long t = tb; t < te; ++t) {
-                        const int k = (int)(t * kWave) + lane;
-                        const float2 e = pairs[k < h ? k : h - 1];
-                        const T w1 = (k < h) ? (T)e.y : T(0);
-                        const T w2 = (k < h && 2 * k + 1 != n) ? (T)e.y : T(0);
-                        const T x1 = (T)fmaf(sa, e.x, sh);
-                        const T x2 = (T)fmaf(-sa, e.x, sh);
-                        fa = fma(w1, F::finish(F::fold_c(s0, ac0, x1, p), p), fa);
-                        fa = fma(w2, F::finish(F::fold_c(s0, ac0, x2, p), p), fa);
-                    }
-                } else {
-    #pragma unroll 2
-                    for (long long t = tb; t < te; ++t) {
-                        const int k = (int)(t * kWave) + lane;
-                        const int kk = k < h ? k : h - 1;
-                        const double xn = glx[kk], wk = glw[kk];
-                        const T w1 = (k < h) ? (T)wk : T(0);
-                        const T w2 = (k < h && 2 * k + 1 != n) ? (T)wk : T(0);
-                        const T x1 = (T)fma(a0.a, xn, a0.h);
-                        const T x2 = (T)fma(-a0.a, xn, a0.h);
-                        fa = fma(w1, F::finish(F::fold_c(s0, ac0, x1, p), p), fa);
-                        fa = fma(w2, F::finish(F::fold_c(s0, ac0, x2, p), p), fa);
-                    }
+#pragma unroll 2
+                for (long long t = tb; t < te; ++t) {
+                    const int k = (int)(t * kWave) + lane;
+                    const int kk = k < h ? k : h - 1;
+                    const double xn = glx[kk], wk = glw[kk];
+                    const T w1 = (k < h) ? (T)wk : T(0);
+                    const T w2 = (k < h && 2 * k + 1 != n) ? (T)wk : T(0);
+                    const T x1 = (T)fma(a0.a, xn, a0.h);
+                    const T x2 = (T)fma(-a0.a, xn, a0.h);
+                    fa = fma(w1, F::finish(F::fold_c(s0, ac0, x1, p), p), fa);
+                    fa = fma(w2, F::finish(F::fold_c(s0, ac0, x2, p), p), fa);
                 }
                 acc += (double)fa;
             }
@@ -322,7 +358,7 @@ __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule,
                 acc += edge_item(t_end_item);
                 ie = t_end_item;
             }
-            if (rule == TQ_RULE_GAUSS_LEGENDRE) {
+            if ((PATHS & kPathsGauss) != 0 && rule == TQ_RULE_GAUSS_LEGENDRE) {
                 for (long long tb = ib; tb < ie; tb += kFlush) {
                     const long long te = (tb + kFlush < ie) ? (tb + kFlush) : ie;
                     T fa = T(0);
@@ -338,16 +374,21 @@ __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule,
                 // Newton-Cotes interior weights repeat with period 4 in the node
                 // index, and 64 t + lane = lane (mod 4): one weight per lane.
                 const double w_lane = weight_of(rule, kWave + lane, 0x7fffffff, glw);
+                const double row_step = kWave * a0.h;
                 for (long long tb = ib; tb < ie; tb += kFlush) {
                     const long long te = (tb + kFlush < ie) ? (tb + kFlush) : ie;
-                    double kd = (double)(tb * kWave + lane);
+                    // four rows per trip: one FP64 product for their nodes, then an addition each
                     T fa = T(0);
-    #pragma unroll 4
-                    for (long long t = tb; t < te; ++t) {
-                        const T x = (T)fma(kd, a0.h, a0.a);
-                        kd += (double)kWave;
-                        fa += F::finish(F::fold_c(s0, ac0, x, p), p);
+                    long long t = tb;
+                    constexpr int U = FAM == TQ_FAM_SIN_SUM ? 1 : 4;
+                    for (; t + U <= te; t += U) {
+                        const double x0 = fma((double)(t * kWave + lane), a0.h, a0.a);
+#pragma unroll
+                        for (int u = 0; u < U; ++u)
+                            fa += F::finish(F::fold_c(s0, ac0, (T)(u ? x0 + u * row_step : x0), p), p);
                     }
+                    for (; t < te; ++t)
+                        fa += F::finish(F::fold_c(s0, ac0, (T)fma((double)(t * kWave + lane), a0.h, a0.a), p), p);
                     acc += w_lane * (double)fa;
                 }
             }

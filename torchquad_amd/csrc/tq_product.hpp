@@ -120,118 +120,75 @@ __device__ inline int mag_exp(double v) {
 }
 __device__ inline int exp_or_zero(int e) { return e == -0x7fffffff ? 0 : e; }
 
-// Largest value of the wave's lanes, in every lane (DPP, no LDS).
-__device__ inline int wave_max(int v) {
-    auto step = [&](int o) { v = o > v ? o : v; };
-    step(__builtin_amdgcn_update_dpp(v, v, 0x111, 0xF, 0xF, false));  // row_shr 1, 2, 4, 8
-    step(__builtin_amdgcn_update_dpp(v, v, 0x112, 0xF, 0xF, false));
-    step(__builtin_amdgcn_update_dpp(v, v, 0x114, 0xF, 0xF, false));
-    step(__builtin_amdgcn_update_dpp(v, v, 0x118, 0xF, 0xF, false));
-    step(__builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));  // row_bcast15 into rows 1 and 3
-    step(__builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));  // row_bcast31 into rows 2 and 3
-    return __builtin_amdgcn_readlane(v, kWave - 1);
-}
-
-// The integer above an exponent, or the smallest int for NaN.
-__device__ inline int exp_ceil(double x) { return x == x ? (int)ceil(x) : -0x7fffffff; }
-
-// Weighted factor of node j on axis k; top: the axis's largest exponent (exponential families).  Returns the
-// exponent of the value that the axis is scaled by.
+// Exponent that a node's weighted factor does not exceed by more than one,
+// without evaluating the factor: the power of two that its axis is scaled by
+// is the largest of these.
 template <int FAM, typename T>
-__device__ inline int weighted_factor(int k, T x, double ex, int top, double w, const Params<T>& p, double* v) {
+__device__ inline int factor_scale(int k, T x, double w, double ex, const Params<T>& p) {
+    const int m = mag_exp(w);
+    if (m == -0x7fffffff) return m;
     if constexpr (family_exponential(FAM)) {
-        v[0] = w * exp2(ex - (double)exp_or_zero(top));
-        return mag_exp(v[0]);
+        return ex == ex ? m + (int)ceil(ex) : -0x7fffffff;
+    } else if constexpr (FAM == TQ_FAM_PRODUCT_PEAK) {
+        const double t = (double)x - (double)p.u[k];
+        const int e = mag_exp(fma(t, t, (double)p.b[k]));
+        return e == -0x7fffffff ? e : m - e + 1;
     } else {
-        factor_comps<FAM, T>(k, x, w, p, v);
-        return mag_exp(FAM == TQ_FAM_PRODUCT_PEAK ? v[0] : w);
+        return m;
     }
 }
 
 // Axis tables of a whole block: component c of axis k's node j goes to
 // axis[c * d * n + k * n + j], the power of two taken out of axis k to
-// s_exp[k].  Axes of up to 128 nodes: one wave per axis, two nodes per lane,
-// in registers.  Longer ones: the block walks all nodes, with 8-byte copies
-// of the entries in `tmp` until they are scaled (s_top: [d] ints).  Ends with
-// a barrier.
-constexpr int kWaveAxis = 2 * kWave;
-
+// s_exp[k].  The d n nodes are spread over the block's threads; the scales
+// come from a first pass over them that evaluates no transcendental (an
+// earlier form, one wave per axis with the factors in registers, left most
+// lanes idle on short axes and evaluated long ones up to three times).  Ends
+// with a barrier.
 template <int FAM, typename T>
 __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax, const double* glx,
-                                          const double* glw, const Params<T>& p, FastDiv by_n, T* axis, double* tmp,
-                                          int* s_top, int* s_exp) {
+                                          const double* glw, const Params<T>& p, FastDiv by_n, T* axis, int* s_exp) {
     constexpr int C = family_comps(FAM);
-    constexpr bool EXP = family_exponential(FAM);
     const int tid = threadIdx.x, nt = blockDim.x, total = d * n;
-    if (n <= kWaveAxis) {
-        const int lane = tid & (kWave - 1), waves = nt >> 6;
-        for (int k = __builtin_amdgcn_readfirstlane(tid >> 6); k < d; k += waves) {
-            double ex[2] = {0.0, 0.0}, w[2], v[2][C];
-            T x[2];
-            int top = -0x7fffffff, m = -0x7fffffff;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if (i * kWave >= n) continue;
-                const int j = lane + i * kWave, jc = j < n ? j : n - 1;  // lanes past the end repeat the last node
-                x[i] = (T)node_of(ax[k], jc, n, rule, glx);
-                w[i] = weight_of(rule, jc, n, glw);
-                if constexpr (EXP) {
-                    ex[i] = factor_exponent<FAM, T>(k, x[i], p);
-                    const int e = exp_ceil(ex[i]);
-                    top = e > top ? e : top;
-                }
-            }
-            if (EXP) top = wave_max(top);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                if (i * kWave >= n) continue;
-                const int e = weighted_factor<FAM, T>(k, x[i], ex[i], top, w[i], p, v[i]);
-                m = e > m ? e : m;
-            }
-            m = exp_or_zero(wave_max(m));
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int j = lane + i * kWave;
-                if (j < n)
-#pragma unroll
-                    for (int c = 0; c < C; ++c) axis[c * total + k * n + j] = (T)ldexp(v[i][c], -m);
-            }
-            if (lane == 0) s_exp[k] = m + (EXP ? exp_or_zero(top) : 0);
-        }
-        __syncthreads();
-        return;
-    }
-    if (tid < d) {
-        s_top[tid] = -0x7fffffff;
-        s_exp[tid] = -0x7fffffff;
-    }
+    constexpr bool EXP = family_exponential(FAM);
+    if (tid < d) s_exp[tid] = -0x7fffffff;
     __syncthreads();
-    if (EXP) {
-        for (int e = tid; e < total; e += nt) {
-            const int k = (int)by_n.div((uint32_t)e), j = e - k * n;
-            tmp[e] = factor_exponent<FAM, T>(k, (T)node_of(ax[k], j, n, rule, glx), p);
-            atomicMax(&s_top[k], exp_ceil(tmp[e]));
-        }
-        __syncthreads();
-    }
-    for (int e = tid; e < total; e += nt) {
-        const int k = (int)by_n.div((uint32_t)e), j = e - k * n;
+    struct Node {
+        int k;
+        T x;
+        double w, ex;
+    };
+    auto node = [&](int e) {
+        Node v;
+        v.k = (int)by_n.div((uint32_t)e);
+        const int j = e - v.k * n;
+        v.x = (T)node_of(ax[v.k], j, n, rule, glx);
+        v.w = weight_of(rule, j, n, glw);
+        v.ex = 0.0;
+        if constexpr (EXP) v.ex = factor_exponent<FAM, T>(v.k, v.x, p);
+        return v;
+    };
+    auto scale = [&](const Node& v) { atomicMax(&s_exp[v.k], factor_scale<FAM, T>(v.k, v.x, v.w, v.ex, p)); };
+    auto store = [&](const Node& nd, int e) {
+        const int m = exp_or_zero(s_exp[nd.k]);
         double v[C];
-        const T x = EXP ? T(0) : (T)node_of(ax[k], j, n, rule, glx);
-        const int m = weighted_factor<FAM, T>(k, x, EXP ? tmp[e] : 0.0, EXP ? s_top[k] : 0,
-                                              weight_of(rule, j, n, glw), p, v);
+        if constexpr (EXP) {
+            v[0] = nd.w * exp2(nd.ex - (double)m);
+        } else {
+            factor_comps<FAM, T>(nd.k, nd.x, nd.w, p, v);
 #pragma unroll
-        for (int c = 0; c < C; ++c) tmp[c * total + e] = v[c];
-        atomicMax(&s_exp[k], m);
-    }
-    __syncthreads();
-    for (int e = tid; e < total; e += nt) {
-        const int m = exp_or_zero(s_exp[by_n.div((uint32_t)e)]);
+            for (int c = 0; c < C; ++c) v[c] = ldexp(v[c], -m);
+        }
 #pragma unroll
-        for (int c = 0; c < C; ++c) axis[c * total + e] = (T)ldexp(tmp[c * total + e], -m);
-    }
+        for (int c = 0; c < C; ++c) axis[c * total + e] = (T)v[c];
+    };
+    // the thread's first node is kept over the barrier, later ones are formed again
+    Node first = node(tid < total ? tid : total - 1);
+    if (tid < total) scale(first);
+    for (int e = tid + nt; e < total; e += nt) scale(node(e));
     __syncthreads();
-    if (tid < d) s_exp[tid] = exp_or_zero(s_exp[tid]) + (EXP ? exp_or_zero(s_top[tid]) : 0);
+    if (tid < total) store(first, tid);
+    for (int e = tid + nt; e < total; e += nt) store(node(e), e);
     __syncthreads();
 }
 
@@ -299,26 +256,214 @@ __device__ inline double sum_entries(const Factor<FAM, T>* s, const T* tab, int 
     return acc;
 }
 
-// ---- planning --------------------------------------------------------------
-struct ProductGeom {
-    int d, n, m, q, L;  // row axes [0, L), loop axes [L, L + q), lane axes [d - m, d)
-    int rule, K;
+// Table of the combined factors of axes A .. A + q - 1 (q = 2: entry
+// j1 n + j2), `count` of them, zeros from there to `entries`; DUAL: in the
+// form that meets a state.  Four entries per thread and trip: their reads go
+// out together.  The caller's next barrier publishes it.
+template <int FAM, typename T, bool DUAL>
+__device__ inline void build_table(const T* axis, int total, int n, int A, int q, int count, int entries, FastDiv by_n,
+                                   T* tab) {
+    using F = Factor<FAM, T>;
+    const int nt = blockDim.x;
+    for (int e0 = threadIdx.x; e0 < entries; e0 += 4 * nt) {
+        F f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = e0 + i * nt;
+            f[i] = F::one(false);
+            if (e < count) {
+                if (q == 2) {
+                    const int j1 = (int)by_n.div((uint32_t)e);
+                    f[i] = F::merge(axis_factor<FAM, T>(axis, total, A * n + j1),
+                                    axis_factor<FAM, T>(axis, total, (A + 1) * n + e - j1 * n));
+                } else {
+                    f[i] = axis_factor<FAM, T>(axis, total, A * n + e);
+                }
+                if (DUAL) f[i] = f[i].dual();
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < F::C; ++c)
+                if (e0 + i * nt < entries) tab[c * entries + e0 + i * nt] = f[i].v[c];
+    }
+}
+
+// How an integral's axes are split: row axes [0, L), loop axes [L, L + q),
+// lane axes [L + q, d).  The outer one or two lane axes (`outer` of them, N
+// combinations) are cut into K parts of H: a lane holds one combination of
+// the inner lane axes and K of the outer ones, f, f + H, f + 2 H, ..., so its
+// states share everything but one table entry.  (Spreading the K states over
+// consecutive combinations cost digits for every state and axis: an eighth of
+// the instructions of an 8192-integral batch.)
+struct ProductSplit {
+    int d, n, L, q;
+    int outer, inner;   // lane axes: outer (1 or 2) and inner ones
+    int N, H;           // outer combinations, and per state
     int nl, groups;     // loop points n^q and their groups of four
-    int lane_count;     // n^m
-    int lane_groups;    // ceil(n^m / (64 K))
+    int slots;          // H * n^inner
+    int lane_groups;    // ceil(slots / 64)
     FastDiv by_n;
     long long items;    // rows * groups
-    long long ipw;      // items per wave
-    long long num_waves, blocks;
 };
 
-inline size_t product_axis_bytes(const ProductGeom& G, int C, int tsize) {
-    return ((size_t)C * G.d * G.n * tsize + 15) & ~(size_t)15;
+// LDS tables of a split: every axis's factors, the loop table, and the outer
+// table when two axes are combined there.
+template <typename T>
+struct ProductTables {
+    T* axis;
+    T* loop;
+    T* outer;  // component c of outer combination f: outer[c * outer_stride + f]
+    int outer_stride;
+};
+
+inline size_t round16(size_t b) { return (b + 15) & ~(size_t)15; }
+inline size_t product_lds_bytes(const ProductSplit& S, int C, int tsize) {
+    return round16((size_t)C * S.d * S.n * tsize) + round16((size_t)C * S.groups * kGroup * tsize) +
+           (S.outer == 2 ? (size_t)C * S.N * tsize : 0);
 }
-inline size_t product_lds_bytes(const ProductGeom& G, int C, int tsize) {
-    const size_t tmp = G.n > kWaveAxis ? (size_t)C * G.d * G.n * sizeof(double) : 0;
-    const size_t loop = (size_t)C * G.groups * kGroup * tsize;
-    return product_axis_bytes(G, C, tsize) + (tmp > loop ? tmp : loop);
+
+// Builds them (all threads of the block; ends with a barrier).
+template <int FAM, typename T>
+__device__ inline ProductTables<T> build_product_tables(const ProductSplit& S, int rule, const Axis* ax,
+                                                        const double* glx, const double* glw, const Params<T>& p,
+                                                        unsigned char* lds, int* s_exp) {
+    constexpr int C = family_comps(FAM);
+    const int total = S.d * S.n, entries = S.groups * kGroup;
+    ProductTables<T> t;
+    t.axis = reinterpret_cast<T*>(lds);
+    const size_t a = ((size_t)C * total * sizeof(T) + 15) & ~(size_t)15;
+    t.loop = reinterpret_cast<T*>(lds + a);
+    build_axis_factors<FAM, T>(S.d, S.n, rule, ax, glx, glw, p, S.by_n, t.axis, s_exp);
+    build_table<FAM, T, true>(t.axis, total, S.n, S.L, S.q, S.nl, entries, S.by_n, t.loop);
+    if (S.outer == 2) {
+        t.outer = reinterpret_cast<T*>(lds + a + (((size_t)C * entries * sizeof(T) + 15) & ~(size_t)15));
+        t.outer_stride = S.N;
+        build_table<FAM, T, false>(t.axis, total, S.n, S.L + S.q, 2, S.N, S.N, S.by_n, t.outer);
+    } else {
+        t.outer = t.axis + (S.L + S.q) * S.n;
+        t.outer_stride = total;
+    }
+    __syncthreads();
+    return t;
+}
+
+// The K states of lane slot `slot`; zeros where there is no combination.
+template <int FAM, typename T, int K>
+__device__ inline void lane_states(const ProductSplit& S, const ProductTables<T>& t, int slot, Factor<FAM, T>* own) {
+    using F = Factor<FAM, T>;
+    const bool on = slot < S.slots;
+    uint32_t r = on ? (uint32_t)slot : 0u;
+    F common = F::one(true);
+    for (int a = S.d - 1; a >= S.d - S.inner; --a) {
+        const uint32_t q = S.by_n.div(r);
+        common = F::merge(common, axis_factor<FAM, T>(t.axis, S.d * S.n, a * S.n + (int)(r - q * S.by_n.n)));
+        r = q;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const int f = (int)r + k * S.H;
+        const bool has = on && f < S.N;
+        F o = axis_factor<FAM, T>(t.outer, t.outer_stride, has ? f : 0);
+        o = F::merge(common, o);
+#pragma unroll
+        for (int c = 0; c < F::C; ++c) own[k].v[c] = has ? o.v[c] : T(0);
+    }
+}
+
+// Sum over the wave-uniform items [t0, t1) of the K states' values: item t is
+// group t mod `groups` of the loop table on row t / groups, whose factor (of
+// the axes [0, L)) is merged into the states.
+template <int FAM, typename T, int K>
+__device__ inline double sum_items(const ProductSplit& S, const ProductTables<T>& t, const Factor<FAM, T>* own,
+                                   long long t0, long long t1) {
+    using F = Factor<FAM, T>;
+    const int lane = threadIdx.x & (kWave - 1), n = S.n, L = S.L, groups = S.groups, entries = groups * kGroup;
+    if (L == 0) return sum_entries<FAM, T, K>(own, t.loop, entries, (int)t0, (int)t1);
+    // row odometer: lane k of `dig` holds the digit of row axis k
+    long long row = t0 / groups;
+    int gi = (int)(t0 - row * groups);
+    int dig = 0;
+    for (int k = L - 1; k >= 0; --k) {
+        const long long q = row / n;
+        dig = lane == k ? (int)(row - q * n) : dig;
+        row = q;
+    }
+    double acc = 0.0;
+    for (long long at = t0; at < t1;) {
+        F rf = F::one(true);
+        for (int k = 0; k < L; ++k)
+            rf = F::merge(rf, axis_factor<FAM, T>(t.axis, S.d * n, k * n + __builtin_amdgcn_readlane(dig, k)));
+        F s[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) s[k] = F::merge(own[k], rf);
+        const int left = groups - gi;
+        const int ge = t1 - at < left ? gi + (int)(t1 - at) : groups;
+        acc += sum_entries<FAM, T, K>(s, t.loop, entries, gi, ge);
+        at += ge - gi;
+        gi = 0;
+        for (int k = L - 1; k >= 0; --k) {
+            const int dk = __builtin_amdgcn_readlane(dig, k) + 1;
+            const bool wrap = dk >= n;
+            dig = lane == k ? (wrap ? 0 : dk) : dig;
+            if (!wrap) break;
+        }
+    }
+    return acc;
+}
+
+// The split of a d-axis integral with K states per lane that has the least
+// work, counted in instructions per wave: the multiply-adds of the (padded)
+// groups, the states' set-up once per lane group, and the merges, digits and
+// flush once per row.  max_entries: longest loop table; max_outer: longest
+// combined outer table; lane_axes > 0 fixes the number of lane axes.  False:
+// no split fits lds_max bytes of tables.
+inline bool split_product_axes(int d, int n, int K, int C, int tsize, long long max_entries, long long max_outer,
+                               int lane_axes, size_t lds_max, ProductSplit& S) {
+    if (d < 2 || n < 2) return false;
+    double best = -1.0;
+    for (int q = 1; q <= 2 && q < d; ++q) {
+        const double nl = q == 2 ? (double)n * n : (double)n, groups = std::ceil(nl / kGroup);
+        if (groups * kGroup > (double)max_entries) break;
+        for (int m = 1; m <= d - q; ++m) {
+            if (lane_axes > 0 && m != lane_axes) continue;
+            for (int outer = 1; outer <= 2 && outer <= m; ++outer) {
+                const double N = outer == 2 ? (double)n * n : (double)n;
+                if (outer == 2 && N > (double)max_outer) break;
+                const double H = std::ceil(N / K), slots = H * std::pow((double)n, m - outer);
+                if (slots > (double)(1 << 30)) break;
+                const int L = d - q - m;
+                const double rows = std::pow((double)n, L);
+                const double row = groups * kGroup * K * C + (L > 0 ? 30 + 8 * L + 2 * K * C : 0) +
+                                   std::ceil(groups / (kFlush / kGroup)) * 8;
+                const double init = 20 + 12 * (m - outer) + K * (5 + 3 * C);
+                const double work = std::ceil(slots / kWave) * (init + std::round(rows) * row);
+                if (best >= 0.0 && work >= best) continue;
+                ProductSplit X;
+                X.d = d;
+                X.n = n;
+                X.L = L;
+                X.q = q;
+                X.outer = outer;
+                X.inner = m - outer;
+                X.N = (int)N;
+                X.H = (int)H;
+                X.nl = (int)nl;
+                X.groups = (int)groups;
+                if (product_lds_bytes(X, C, tsize) > lds_max) continue;
+                X.slots = (int)slots;
+                X.lane_groups = (int)std::ceil(slots / kWave);
+                long long r;
+                if (ipow_checked(n, L, (1LL << 62) / X.groups, &r) != 0) continue;
+                X.items = r * X.groups;
+                best = work;
+                S = X;
+            }
+        }
+    }
+    S.by_n = make_fast_div((uint32_t)n);
+    return best >= 0.0;
 }
 
 }  // namespace tq
