@@ -58,7 +58,7 @@ __device__ __forceinline__ double batch_tile_general(const BatchDev<T>& D, const
     if (table) {
         const int lane = threadIdx.x & (kWave - 1);
         for (int j = lane; j < D.nl; j += kWave)
-            loop_table_entry<T, FAM>(tab, j, ax, D.L, D.q, D.n, D.rule, glx, glw, D.p);
+            loop_table_entry<T, FAM>(tab, j, ax, D.L, D.n, D.rule, glx, glw, D.p);
     }
     // make this wave's LDS writes visible to all of its lanes
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

@@ -16,11 +16,9 @@
 //   dI/dlo_k = (dI/dbeta_k - dI/dalpha_k)/2,  dI/dhi_k = (dI/dbeta_k + dI/dalpha_k)/2.
 // The backward kernel walks the same tiles as the forward one and forms
 // these sums per point in FP32 (flushed to FP64 at least every 128 points).
-#include "tq_grid_tile.hpp"
+#include "tq_sweep.hpp"
 
 namespace tq {
-
-constexpr int kSweepMaxD = 8;
 
 struct SweepGeom {
     GridGeom g;
@@ -32,61 +30,15 @@ struct SweepGeom {
 // loop-axis table, 1 + 3 dim block sums) is spread over many points.
 constexpr long long kSweepWaves = 16384;
 
-// The backward tile walks one loop axis.  The forward kernel may loop over
-// two (tables up to kSweepMergeCap entries) with the same lane axes, so both
-// plans have the same waves and the backward's workspace covers both.
-constexpr long long kSweepMergeCap = 1024;
-
-static int sweep_geom(const tq_grid_desc* gd, long long B, SweepGeom& S, long long merge_cap = 0) {
+// General kernels: one loop axis, walked the same way forward and backward.
+static int sweep_geom(const tq_grid_desc* gd, long long B, SweepGeom& S) {
     const long long per_integral = B > 0 ? (kSweepWaves + B - 1) / B : kSweepWaves;
     // the backward's one-axis rows walk every node, so the forward does too
-    int rc = plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, per_integral, S.g, merge_cap,
-                       false, false);
+    int rc = plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, per_integral, S.g, 0, false,
+                       false);
     if (rc) return rc;
     S.blocks_x = (S.g.num_waves + kWavesPerBlock - 1) / kWavesPerBlock;
     return TQ_OK;
-}
-
-// Parameters of integral b in the family's Params layout (as make_params
-// builds them for one integrand): Gaussian peak a[b][d], u[b][d]; product
-// peak a[b][d], u[b][d] (b_k = a_k^-2); oscillatory c[b][d] in a and w[b]
-// in u (FP32 phase in revolutions, FP64 in radians).
-template <typename T, int FAM>
-__device__ inline void load_sweep_params(int d, int n, int rule, long long b, const T* a, const T* u, const T* dom,
-                                         Params<T>* p, Axis* ax) {
-    const double sl2e = 1.2011224087864498;  // sqrt(log2 e), as in make_params
-    const int tid = threadIdx.x;
-    if (tid < TQ_MAX_DIM) {
-        T pa = T(0), pb = T(0), pu = T(0);
-        if (tid < d) {
-            const double ak = (double)a[b * d + tid];
-            if (FAM == TQ_FAM_GAUSSIAN_PEAK) {
-                const double uk = (double)u[b * d + tid];
-                pa = (T)(ak * sl2e);
-                pb = (T)(-ak * uk * sl2e);
-                pu = (T)uk;
-            } else if (FAM == TQ_FAM_PRODUCT_PEAK) {
-                pa = (T)ak;
-                pb = (T)(ak != 0.0 ? 1.0 / (ak * ak) : 0.0);
-                pu = u[b * d + tid];
-            } else {  // oscillatory
-                pa = (T)(sizeof(T) == 4 ? ak / (2.0 * M_PI) : ak);
-            }
-            ax[tid] = make_axis(dom + b * 2 * d, tid, n, rule);
-        }
-        p->a[tid] = pa;
-        p->b[tid] = pb;
-        p->u[tid] = pu;
-    }
-    if (tid == 0) {
-        p->c0 = T(1);
-        p->c1 = p->c3 = T(0);
-        p->c2 = T(0);
-        if (FAM == TQ_FAM_OSCILLATORY) {
-            const double w = (double)u[b];
-            p->c2 = (T)(sizeof(T) == 4 ? w : 2.0 * M_PI * w);
-        }
-    }
 }
 
 constexpr int kSweepRowTab = 1024;  // row-axis table entries (L*n) kept in LDS
@@ -105,12 +57,10 @@ static_assert(StateSlots<TQ_FAM_GAUSSIAN_PEAK>::v == 1 && StateSlots<TQ_FAM_PROD
                   StateSlots<TQ_FAM_OSCILLATORY>::v == 1,
               "sweep families keep one state slot");
 
-// BW waves per block: 16 with a two-axis loop (one block per integral
-// builds the n^2-entry table once), else 4.
-template <typename T, int FAM, bool TABLE, bool ROWTAB, int BW>
-__global__ __launch_bounds__(BW * kWave) void k_sweep_fwd(SweepGeom S, const T* a, const T* u, const T* dom,
+template <typename T, int FAM, bool TABLE, bool ROWTAB>
+__global__ __launch_bounds__(kBlock) void k_sweep_fwd(SweepGeom S, const T* a, const T* u, const T* dom,
                                                          const double* glx, const double* glw, double* partials) {
-    constexpr int NT = BW * kWave;
+    constexpr int NT = kBlock, BW = kWavesPerBlock;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ Params<T> s_p;
     __shared__ Axis s_axis[TQ_MAX_DIM];
@@ -123,12 +73,8 @@ __global__ __launch_bounds__(BW * kWave) void k_sweep_fwd(SweepGeom S, const T* 
     load_sweep_params<T, FAM>(g.d, g.n, g.rule, b, a, u, dom, &s_p, s_axis);
     __syncthreads();
     if (TABLE) {
-        if (g.q == 2 && g.n <= 32)
-            pair_table_wave<T, FAM>(s_tab, s_axis, g.L, g.n, g.rule, glx, glw, s_p,
-                                    __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kWave, NT);
-        else
-            for (int j = threadIdx.x; j < g.nl; j += NT)
-                loop_table_entry<T, FAM>(s_tab, j, s_axis, g.L, g.q, g.n, g.rule, glx, glw, s_p);
+        for (int j = threadIdx.x; j < g.nl; j += NT)
+            loop_table_entry<T, FAM>(s_tab, j, s_axis, g.L, g.n, g.rule, glx, glw, s_p);
         if (ROWTAB)
             for (int e = threadIdx.x; e < g.L * g.n; e += NT) {
                 const int k = e / g.n;
@@ -151,12 +97,6 @@ __global__ __launch_bounds__(BW * kWave) void k_sweep_fwd(SweepGeom S, const T* 
     if (threadIdx.x == 0) partials[b * gridDim.x + blockIdx.x] = bs;
 }
 
-// normalised node coordinate r in [-1, 1]
-__device__ inline double node_r(int j, int n, int rule, const double* glx) {
-    if (rule == TQ_RULE_GAUSS_LEGENDRE) return glx[j];
-    return (n > 1) ? 2.0 * (double)j / (double)(n - 1) - 1.0 : 0.0;
-}
-
 // One loop-axis table entry of the backward kernel: exponent term
 // -(a x + b)^2 + log2(w) in log2 units (the node weight folded into the
 // exponent, so w f is one exp2) and the normalised node r.  The loop axis's
@@ -168,17 +108,6 @@ template <typename T>
 struct alignas(2 * sizeof(T)) BwdEntry {
     T term, r;
 };
-
-// x = alpha r + beta on an axis (r the normalised node of node_r).
-__device__ inline void loop_axis_affine(const Axis& ax, int n, int rule, double* alpha, double* beta) {
-    if (rule == TQ_RULE_GAUSS_LEGENDRE) {
-        *alpha = ax.a;
-        *beta = ax.h;
-    } else {
-        *alpha = 0.5 * (ax.b - ax.a);
-        *beta = 0.5 * (ax.b + ax.a);
-    }
-}
 
 // Backward tile for D axes: flat walk of the tile's points (lane axes per
 // lane, the rest decoded per row).  Only the loop axis is accumulated per
@@ -971,8 +900,6 @@ __global__ __launch_bounds__(kBlock) void k_sweep_bwd_finalize_fam(const double*
     }
 }
 
-static int sweep_values(int family, int D) { return family == TQ_FAM_OSCILLATORY ? 2 + D : 1 + 3 * D; }
-
 static int check_family(int family) {
     if (family != TQ_FAM_GAUSSIAN_PEAK && family != TQ_FAM_OSCILLATORY && family != TQ_FAM_PRODUCT_PEAK)
         return fail(TQ_E_UNSUPPORTED, "sweeps support the Gaussian peak, oscillatory and product peak families");
@@ -994,35 +921,39 @@ static int check_sweep(const tq_grid_desc* g, int64_t B) {
     return TQ_OK;
 }
 
-template <typename T, int FAM, bool TABLE, bool ROWTAB, int BW>
+template <typename T, int FAM, bool TABLE, bool ROWTAB>
 static void launch_fwd_kernel(const SweepGeom& S, int64_t B, const void* a, const void* u, const void* dom,
                               const tq_grid_desc* gd, void* ws, size_t shmem, unsigned gx, hipStream_t s) {
-    hipLaunchKernelGGL((k_sweep_fwd<T, FAM, TABLE, ROWTAB, BW>), dim3(gx, (unsigned)B), dim3(BW * kWave), shmem, s,
-                       S, (const T*)a, (const T*)u, (const T*)dom, gd->gl_nodes, gd->gl_weights, (double*)ws);
+    hipLaunchKernelGGL((k_sweep_fwd<T, FAM, TABLE, ROWTAB>), dim3(gx, (unsigned)B), dim3(kBlock), shmem, s, S,
+                       (const T*)a, (const T*)u, (const T*)dom, gd->gl_nodes, gd->gl_weights, (double*)ws);
 }
 
 template <typename T, int FAM>
 static int launch_sweep_fwd(const tq_grid_desc* gd, int64_t B, const void* a, const void* u, const void* dom,
                             void* ws, size_t wsb, void* out, double* out64, hipStream_t s) {
+    long long gx = sweep_product_blocks(gd, B);
+    const bool product = gx > 0;
     SweepGeom S;
-    int rc = sweep_geom(gd, B, S, kSweepMergeCap);
-    if (rc) return rc;
-    if (!ws || wsb < (size_t)(S.blocks_x * B) * sizeof(double)) return fail(TQ_E_WORKSPACE, "sweep workspace too small");
-    if (S.blocks_x > 0x7fffffff) return fail(TQ_E_ARG, "too many blocks");
-    const bool wide = S.g.q == 2;
-    const int bw = wide ? 16 : kWavesPerBlock;
-    const unsigned gx = (unsigned)((S.g.num_waves + bw - 1) / bw);
-    if (S.g.use_table && S.g.L >= 1 && (long long)S.g.L * S.g.n <= kSweepRowTab) {
-        const size_t sh = sweep_fwd_lds<T, FAM>(S.g, true, true);
-        if (wide) launch_fwd_kernel<T, FAM, true, true, 16>(S, B, a, u, dom, gd, ws, sh, gx, s);
-        else launch_fwd_kernel<T, FAM, true, true, kWavesPerBlock>(S, B, a, u, dom, gd, ws, sh, gx, s);
-    } else if (S.g.use_table) {
-        const size_t sh = sweep_fwd_lds<T, FAM>(S.g, true, false);
-        if (wide) launch_fwd_kernel<T, FAM, true, false, 16>(S, B, a, u, dom, gd, ws, sh, gx, s);
-        else launch_fwd_kernel<T, FAM, true, false, kWavesPerBlock>(S, B, a, u, dom, gd, ws, sh, gx, s);
-    } else {
-        launch_fwd_kernel<T, FAM, false, false, kWavesPerBlock>(S, B, a, u, dom, gd, ws, 0, gx, s);
+    int rc = TQ_OK;
+    if (!product) {
+        rc = sweep_geom(gd, B, S);
+        if (rc) return rc;
+        gx = S.blocks_x;
     }
+    if (!ws || wsb < (size_t)(gx * B) * sizeof(double)) return fail(TQ_E_WORKSPACE, "sweep workspace too small");
+    if (gx > 0x7fffffff) return fail(TQ_E_ARG, "too many blocks");
+    if (product) {
+        rc = launch_sweep_product_fwd<T, FAM>(gd, B, a, u, dom, (double*)ws, gx, s);
+    } else if (S.g.use_table && S.g.L >= 1 && (long long)S.g.L * S.g.n <= kSweepRowTab) {
+        launch_fwd_kernel<T, FAM, true, true>(S, B, a, u, dom, gd, ws, sweep_fwd_lds<T, FAM>(S.g, true, true),
+                                              (unsigned)gx, s);
+    } else if (S.g.use_table) {
+        launch_fwd_kernel<T, FAM, true, false>(S, B, a, u, dom, gd, ws, sweep_fwd_lds<T, FAM>(S.g, true, false),
+                                               (unsigned)gx, s);
+    } else {
+        launch_fwd_kernel<T, FAM, false, false>(S, B, a, u, dom, gd, ws, 0, (unsigned)gx, s);
+    }
+    if (rc) return rc;
     rc = check_launch("k_sweep_fwd");
     if (rc) return rc;
     const long long fb = (B + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -1059,32 +990,46 @@ template <typename T, int FAM>
 static int launch_sweep_bwd(const tq_grid_desc* gd, int64_t B, const void* a, const void* u, const void* dom,
                             const void* grad_out, void* ws, size_t wsb, void* ga, void* gu, void* gdom,
                             hipStream_t s) {
-    SweepGeom S;
-    int rc = sweep_geom(gd, B, S);
-    if (rc) return rc;
+    long long gx = FAM == TQ_FAM_OSCILLATORY ? 0 : sweep_product_blocks(gd, B);
+    const bool product = gx > 0;
     const int D = gd->dim;
-    if (!ws || wsb < (size_t)(S.blocks_x * B * sweep_values(FAM, D)) * sizeof(double))
+    SweepGeom S;
+    int rc = TQ_OK;
+    if (!product) {
+        rc = sweep_geom(gd, B, S);
+        if (rc) return rc;
+        gx = S.blocks_x;
+    }
+    if (!ws || wsb < (size_t)(gx * B * sweep_values(FAM, D)) * sizeof(double))
         return fail(TQ_E_WORKSPACE, "sweep workspace too small");
-    switch (D) {
-        case 1: rc = launch_bwd_d<T, FAM, 1>(S, B, a, u, dom, gd, ws, s); break;
-        case 2: rc = launch_bwd_d<T, FAM, 2>(S, B, a, u, dom, gd, ws, s); break;
-        case 3: rc = launch_bwd_d<T, FAM, 3>(S, B, a, u, dom, gd, ws, s); break;
-        case 4: rc = launch_bwd_d<T, FAM, 4>(S, B, a, u, dom, gd, ws, s); break;
-        case 5: rc = launch_bwd_d<T, FAM, 5>(S, B, a, u, dom, gd, ws, s); break;
-        case 6: rc = launch_bwd_d<T, FAM, 6>(S, B, a, u, dom, gd, ws, s); break;
-        case 7: rc = launch_bwd_d<T, FAM, 7>(S, B, a, u, dom, gd, ws, s); break;
-        default: rc = launch_bwd_d<T, FAM, 8>(S, B, a, u, dom, gd, ws, s); break;
+    if constexpr (FAM != TQ_FAM_OSCILLATORY) {
+        if (product) {
+            rc = launch_sweep_product_bwd<T, FAM>(gd, B, a, u, dom, (double*)ws, gx, s);
+            if (rc) return rc;
+        }
+    }
+    if (!product) {
+        switch (D) {
+            case 1: rc = launch_bwd_d<T, FAM, 1>(S, B, a, u, dom, gd, ws, s); break;
+            case 2: rc = launch_bwd_d<T, FAM, 2>(S, B, a, u, dom, gd, ws, s); break;
+            case 3: rc = launch_bwd_d<T, FAM, 3>(S, B, a, u, dom, gd, ws, s); break;
+            case 4: rc = launch_bwd_d<T, FAM, 4>(S, B, a, u, dom, gd, ws, s); break;
+            case 5: rc = launch_bwd_d<T, FAM, 5>(S, B, a, u, dom, gd, ws, s); break;
+            case 6: rc = launch_bwd_d<T, FAM, 6>(S, B, a, u, dom, gd, ws, s); break;
+            case 7: rc = launch_bwd_d<T, FAM, 7>(S, B, a, u, dom, gd, ws, s); break;
+            default: rc = launch_bwd_d<T, FAM, 8>(S, B, a, u, dom, gd, ws, s); break;
+        }
     }
     if (rc) return rc;
     const long long fb = (B + kWavesPerBlock - 1) / kWavesPerBlock;
     if constexpr (FAM == TQ_FAM_GAUSSIAN_PEAK) {
         hipLaunchKernelGGL((k_sweep_bwd_finalize<T>), dim3((unsigned)fb), dim3(kBlock), 0, s, (const double*)ws,
-                           S.blocks_x, (long long)B, D, (const T*)a, (const T*)dom, gd->n, gd->rule,
+                           gx, (long long)B, D, (const T*)a, (const T*)dom, gd->n, gd->rule,
                            (const T*)grad_out, (T*)ga, (T*)gu, (T*)gdom);
     } else {
         hipLaunchKernelGGL((k_sweep_bwd_finalize_fam<T, FAM>), dim3((unsigned)fb), dim3(kBlock), 0, s,
-                           (const double*)ws, S.blocks_x, (long long)B, D, (const T*)a, (const T*)dom, gd->n,
-                           gd->rule, (const T*)grad_out, (T*)ga, (T*)gu, (T*)gdom);
+                           (const double*)ws, gx, (long long)B, D, (const T*)a, (const T*)dom, gd->n, gd->rule,
+                           (const T*)grad_out, (T*)ga, (T*)gu, (T*)gdom);
     }
     return check_launch("k_sweep_bwd_finalize");
 }
@@ -1107,8 +1052,10 @@ size_t tq_sweep_workspace_size(const tq_grid_desc* g, int64_t B) {
     if (check_sweep(g, B)) return 0;
     SweepGeom S;
     if (sweep_geom(g, B, S)) return 0;
+    long long blocks = sweep_product_blocks(g, B);
+    if (S.blocks_x > blocks) blocks = S.blocks_x;  // the oscillatory backward
     // the largest partial layout of the sweep families (1 + 3 dim values)
-    return (size_t)(S.blocks_x * B * (1 + 3 * g->dim)) * sizeof(double);
+    return (size_t)(blocks * B * (1 + 3 * g->dim)) * sizeof(double);
 }
 
 int tq_sweep_forward(const tq_grid_desc* g, int32_t family, int64_t B, const void* a, const void* u,

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(BW * kWave) void k_grid_fused(GridArgs<T> A) {
     T* s_rt = s_tab + (size_t)TabStride<FAM>::v * g.nl;
     if (TABLE) {
         for (int j = tid; j < g.nl; j += NT)
-            loop_table_entry<T, FAM>(s_tab, j, s_axis, L, 1, n, rule, A.glx, A.glw, A.p);
+            loop_table_entry<T, FAM>(s_tab, j, s_axis, L, n, rule, A.glx, A.glw, A.p);
         if (ROWTAB)
             for (int e = tid; e < L * n; e += NT) {
                 const int k = e / n;

@@ -273,10 +273,8 @@ struct Family<TQ_FAM_GAUSSIAN_PEAK, T> {
     }
     __device__ static inline State<T> merge(State<T> a, State<T> b) { return {a.s0 + b.s0, T(0)}; }
     __device__ static inline T finish(State<T> s, const Params<T>&) { return tq_exp2(s.s0); }
-    // the weight inside the state: w 2^s = 2^(s + log2 w); the key of a
-    // product of weights is the sum of their keys
+    // the weight inside the state: w 2^s = 2^(s + log2 w)
     __device__ static inline double weight_key(double w) { return log2(w); }
-    __device__ static inline double combine_keys(double a, double b) { return a + b; }
     __device__ static inline T fold_key(T s0, double key) { return (T)((double)s0 + key); }
 };
 
@@ -309,7 +307,6 @@ struct Family<TQ_FAM_PRODUCT_PEAK, T> {
     __device__ static inline T finish(State<T> s, const Params<T>&) { return tq_rcp(s.s0); }
     // the weight inside the state: w / s = 1 / (s (1 / w))
     __device__ static inline double weight_key(double w) { return 1.0 / w; }
-    __device__ static inline double combine_keys(double a, double b) { return a * b; }
     __device__ static inline T fold_key(T s0, double key) { return (T)((double)s0 * key); }
 };
 
@@ -325,7 +322,6 @@ struct Family<TQ_FAM_EXP_LINEAR, T> {
     __device__ static inline State<T> merge(State<T> a, State<T> b) { return {a.s0 + b.s0, T(0)}; }
     __device__ static inline T finish(State<T> s, const Params<T>&) { return tq_exp2(s.s0); }
     __device__ static inline double weight_key(double w) { return log2(w); }
-    __device__ static inline double combine_keys(double a, double b) { return a + b; }
     __device__ static inline T fold_key(T s0, double key) { return (T)((double)s0 + key); }
 };
 

@@ -84,9 +84,8 @@ __device__ inline double axis_scale_of(const Axis& ax, int rule) {
     }
 }
 
-// Loop LDS table: entry j holds the loop's contribution to the integrand
-// state at its point j (fold_c(zero, c_L, x_j) for one loop axis, both axes
-// folded for two), then the point's weight; per point the tile loop only
+// Loop LDS table: entry j holds the loop axis's contribution to the integrand
+// state at its node j (fold_c(zero, c_L, x_j)), then the node's weight; per point the tile loop only
 // merges it into the row/lane state.  Families with a two-component state
 // take three slots per entry.
 //
@@ -118,18 +117,12 @@ __host__ __device__ inline bool folds_weight(int fam) {
 __host__ __device__ inline int tab_stride(int fam) { return state_slots(fam) + (folds_weight(fam) ? 0 : 1); }
 
 // A table build's FP64 value of a weight: the weight, or its key when the
-// family folds it into the state; the value of a product of weights.
+// family folds it into the state.
 template <typename T, int FAM>
 __device__ inline double table_weight(double w) {
     if constexpr (FoldsWeight<FAM>::v) return Family<FAM, T>::weight_key(w);
     else return w;
 }
-template <typename T, int FAM>
-__device__ inline double combine_weights(double a, double b) {
-    if constexpr (FoldsWeight<FAM>::v) return Family<FAM, T>::combine_keys(a, b);
-    else return a * b;
-}
-
 // Stores table entry j from its state and the table_weight value w.
 template <typename T, int FAM>
 __device__ inline void store_table_entry(T* tab, int j, const State<T>& s, double w) {
@@ -143,71 +136,13 @@ __device__ inline void store_table_entry(T* tab, int j, const State<T>& s, doubl
     }
 }
 
-// Loop-table entry j when the loop runs over q consecutive axes L .. L+q-1
-// (q = 1 or 2; for q = 2, j = j1 n + j2 with j1 on axis L): the axes'
-// contributions folded together, then the product of their weights.
+// Loop-table entry of node j on the loop axis L.
 template <typename T, int FAM>
-__device__ inline void loop_table_entry(T* tab, int j, const Axis* ax, int L, int q, int n, int rule,
-                                        const double* glx, const double* glw, const Params<T>& p) {
+__device__ inline void loop_table_entry(T* tab, int j, const Axis* ax, int L, int n, int rule, const double* glx,
+                                        const double* glw, const Params<T>& p) {
     using F = Family<FAM, T>;
-    const int j1 = q == 2 ? j / n : j;
-    State<T> s = F::fold_c(F::zero(), axis_c(p, L), (T)node_of(ax[L], j1, n, rule, glx), p);
-    double w = weight_of(rule, j1, n, glw);
-    if (q == 2) {
-        const int j2 = j - j1 * n;
-        s = F::fold_c(s, axis_c(p, L + 1), (T)node_of(ax[L + 1], j2, n, rule, glx), p);
-        w *= weight_of(rule, j2, n, glw);
-    }
-    store_table_entry<T, FAM>(tab, j, s, table_weight<T, FAM>(w));
-}
-
-// Two-axis loop-table entry j = j1 n + j2 from the nodes of its two axes
-// (x1 on axis L, x2 on axis L + 1, already rounded to T as loop_table_entry
-// rounds node_of) and their table_weight values: the same folds as
-// loop_table_entry with q = 2, while the nodes and weights (or weight keys)
-// are formed once per axis instead of once per entry.
-template <typename T, int FAM>
-__device__ inline void pair_table_entry(T* tab, int j, T x1, T x2, double w1, double w2, const AxisC<T>& c1,
-                                        const AxisC<T>& c2, const Params<T>& p) {
-    using F = Family<FAM, T>;
-    State<T> s = F::fold_c(F::zero(), c1, x1, p);
-    s = F::fold_c(s, c2, x2, p);
-    store_table_entry<T, FAM>(tab, j, s, combine_weights<T, FAM>(w1, w2));
-}
-
-// Two-axis loop table (axes L and L + 1, n <= 32) built by whole waves: the
-// calling wave stores entries first + lane, first + stride + lane, ... (one
-// wave: first 0, stride 64; the waves of a block: first 64 w, stride 64 BW).
-// Lane l < 32 forms node l of axis L and lane 32 + l node l of axis L + 1,
-// and each entry takes its two nodes and weights from those lanes
-// (ds_bpermute).  Every lane runs every trip, so the lanes read from are
-// active; only entries j < n^2 are stored.
-template <typename T, int FAM>
-__device__ inline void pair_table_wave(T* tab, const Axis* ax, int L, int n, int rule, const double* glx,
-                                       const double* glw, const Params<T>& p, int first = 0, int stride = kWave) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int jn = lane & 31;
-    const bool has = jn < n;
-    const int js = has ? jn : 0;  // in-range index for the lanes past n
-    const T xn = (T)node_of(ax[lane < 32 ? L : L + 1], js, n, rule, glx);
-    const double wn = table_weight<T, FAM>(weight_of(rule, js, n, glw));
-    const T xa = has ? xn : T(0);
-    const double wa = has ? wn : 0.0;
-    const AxisC<T> c1 = axis_c(p, L), c2 = axis_c(p, L + 1);
-    const int nl = n * n;
-    int j1 = (first + lane) / n, j2 = first + lane - j1 * n;
-    const int s1 = stride / n, s2 = stride - s1 * n;
-    for (int jb = first; jb < nl; jb += stride) {
-        const T x1 = __shfl(xa, j1 & 31), x2 = __shfl(xa, 32 + j2);
-        const double w1 = __shfl(wa, j1 & 31), w2 = __shfl(wa, 32 + j2);
-        if (jb + lane < nl) pair_table_entry<T, FAM>(tab, jb + lane, x1, x2, w1, w2, c1, c2, p);
-        j1 += s1;
-        j2 += s2;
-        if (j2 >= n) {
-            j2 -= n;
-            ++j1;
-        }
-    }
+    const State<T> s = F::fold_c(F::zero(), axis_c(p, L), (T)node_of(ax[L], j, n, rule, glx), p);
+    store_table_entry<T, FAM>(tab, j, s, table_weight<T, FAM>(weight_of(rule, j, n, glw)));
 }
 
 // Row-axis tables (ROWTAB): for the row axes k < L, entry k*n + j holds the
@@ -233,9 +168,8 @@ __device__ inline void row_table_entry(T* rt, double* rw, int k, int j, const Ax
 // n - 1 - k (x_{n-1-k} = -x_k, w_{n-1-k} = w_k), so each table load serves
 // two points.  Otherwise the lanes of the calling wave
 // take lane combinations lw*64 .. lw*64+63 of the last m axes, the wave walks
-// loop items [t_begin, t_end) (row axes [0, L) x a loop of nl points over
-// the axes between the row and lane axes: one axis, nl = n, or two, nl = n^2,
-// which needs the table).  Returns the lane's weighted sum.  `ax` holds the
+// loop items [t_begin, t_end) (row axes [0, L) x a loop of nl = n points over
+// the axis between the row and lane axes).  Returns the lane's weighted sum.  `ax` holds the
 // per-axis maps, `tab` the loop table (loop_table_entry) when TABLE.
 // Code paths a grid_tile instantiation carries: one-axis integrals (m == 0)
 // of Newton-Cotes and of Gauss-Legendre rules, multi-axis ones (m > 0).  The
@@ -546,13 +480,13 @@ constexpr int kMergeMaxN = 32;
 
 // Splits the n^d index space of one integral (see grid_tile).  lane_axes /
 // items_per_wave override the automatic choice (0 = automatic).  When
-// merge_cap > 0, n^2 <= merge_cap (the caller's loop-table capacity) and
-// there are at least two axes between the row axes and the lane axes, the
-// loop runs over the last two non-lane axes (n^2 points per row, one table
-// entry per point pair), so a short axis does not pay the per-row cost
-// every n points.  trade_lane_axis = false keeps the lane axes (and so the
-// launch size) of the unmerged plan.  gl_fold: a one-axis (m == 0)
-// Gauss-Legendre plan covers half the table (grid_tile's GL_FOLD).
+// merge_cap > 0 and n^2 <= merge_cap, the loop is planned over the last two
+// non-lane axes: no kernel walks such a plan (those integrals take the factor
+// tables of tq_product.hpp), but the sizes of the plain path's workspace, and
+// so the grids that fit a given one, are those of this plan.
+// trade_lane_axis = false keeps the lane axes of the unmerged plan.  gl_fold:
+// a one-axis (m == 0) Gauss-Legendre plan covers half the table (grid_tile's
+// GL_FOLD).
 inline int plan_geom(int d, int n, int rule, int lane_axes, long long items_per_wave, long long target_waves,
                      GridGeom& G, long long merge_cap = 0, bool trade_lane_axis = true, bool gl_fold = true) {
     G.d = d;

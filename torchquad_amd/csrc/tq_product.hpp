@@ -318,8 +318,8 @@ struct ProductTables {
     int outer_stride;
 };
 
-inline size_t round16(size_t b) { return (b + 15) & ~(size_t)15; }
-inline size_t product_lds_bytes(const ProductSplit& S, int C, int tsize) {
+__host__ __device__ inline size_t round16(size_t b) { return (b + 15) & ~(size_t)15; }
+__host__ __device__ inline size_t product_lds_bytes(const ProductSplit& S, int C, int tsize) {
     return round16((size_t)C * S.d * S.n * tsize) + round16((size_t)C * S.groups * kGroup * tsize) +
            (S.outer == 2 ? (size_t)C * S.N * tsize : 0);
 }
@@ -417,13 +417,13 @@ __device__ inline double sum_items(const ProductSplit& S, const ProductTables<T>
 // work, counted in instructions per wave: the multiply-adds of the (padded)
 // groups, the states' set-up once per lane group, and the merges, digits and
 // flush once per row.  max_entries: longest loop table; max_outer: longest
-// combined outer table; lane_axes > 0 fixes the number of lane axes.  False:
-// no split fits lds_max bytes of tables.
+// combined outer table; lane_axes > 0 fixes the number of lane axes; max_q:
+// loop axes at most.  False: no split fits lds_max bytes of tables.
 inline bool split_product_axes(int d, int n, int K, int C, int tsize, long long max_entries, long long max_outer,
-                               int lane_axes, size_t lds_max, ProductSplit& S) {
+                               int lane_axes, size_t lds_max, ProductSplit& S, int max_q = 2) {
     if (d < 2 || n < 2) return false;
     double best = -1.0;
-    for (int q = 1; q <= 2 && q < d; ++q) {
+    for (int q = 1; q <= max_q && q < d; ++q) {
         const double nl = q == 2 ? (double)n * n : (double)n, groups = std::ceil(nl / kGroup);
         if (groups * kGroup > (double)max_entries) break;
         for (int m = 1; m <= d - q; ++m) {
