@@ -20,43 +20,87 @@ struct McArgs {
     Params<T> p;
 };
 
-// MAXD: compile-time bound on the dimension (4, 8 or 16), so the unrolled
-// per-coordinate work is not predicated over 16 coordinates for d <= 8.
-template <typename T, int FAM, int MAXD>
-__global__ __launch_bounds__(kBlock) void k_mc(McArgs<T> A) {
-    __shared__ double s_red[kWavesPerBlock];
-    const int d = A.d;
-    T lo[MAXD], sz[MAXD];
+// x[k] = lo + size u[k] of one sample.  FOLD (FP32): u[k] stays the integer
+// u 2^24 and the size carries the 2^-24: the same product, one multiply per
+// coordinate less.
+template <int D, bool FOLD>
+__device__ inline void mc_point(uint64_t seed, uint32_t c_lo, uint32_t c_hi, const float* lo, const float* sz,
+                                float* x) {
 #pragma unroll
-    for (int k = 0; k < MAXD; ++k) {
-        if (k < d) {
-            lo[k] = A.domain[2 * k];
-            sz[k] = A.domain[2 * k + 1] - A.domain[2 * k];
-        } else {
-            lo[k] = T(0);
-            sz[k] = T(0);
-        }
+    for (int k = 0; k < D; k += 4) {
+        const u32x4 r = philox_block(seed, c_lo, c_hi, (uint32_t)(k / 4));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (k + i < D) x[k + i] = fmaf(FOLD ? (float)(r.v[i] >> 8) : u01f(r.v[i]), sz[k + i], lo[k + i]);
     }
-    const uint64_t base = A.offset_dev ? *A.offset_dev : A.offset;
-    const long long gt = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long s0 = gt * A.spt;
-    const long long s1 = (s0 + A.spt < A.N) ? (s0 + A.spt) : A.N;
-    double acc = 0.0, acc2 = 0.0;
-    for (long long sb = s0; sb < s1; sb += kMcFlush) {
-        const long long se = (sb + kMcFlush < s1) ? (sb + kMcFlush) : s1;
-        T fa = T(0), fa2 = T(0);
-        for (long long s = sb; s < se; ++s) {
-            T x[MAXD];
-            Uniform<T>::template draw<MAXD>(A.seed, base + (uint64_t)s, d, x);
+}
+template <int D, bool FOLD>
+__device__ inline void mc_point(uint64_t seed, uint32_t c_lo, uint32_t c_hi, const double* lo, const double* sz,
+                                double* x) {
 #pragma unroll
-            for (int k = 0; k < MAXD; ++k)
-                if (k < d) x[k] = fma(x[k], sz[k], lo[k]);
-            const T f = eval_point<FAM, T, MAXD>(x, d, A.p);
+    for (int k = 0; k < D; k += 2) {
+        const u32x4 r = philox_block(seed, c_lo, c_hi, (uint32_t)(k / 2));
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (k + i < D) x[k + i] = fma(u01d(r.v[2 * i], r.v[2 * i + 1]), sz[k + i], lo[k + i]);
+    }
+}
+
+// The samples s0 .. s1-1 of a thread, in runs of one high counter word: the
+// Philox products of that word leave the loop.
+template <typename T, int FAM, int D, bool FOLD>
+__device__ inline void mc_samples(const McArgs<T>& A, const T* lo, const T* sz, long long s0, long long s1,
+                                  double& acc, double& acc2) {
+    const uint64_t base = A.offset_dev ? *A.offset_dev : A.offset;
+    while (s0 < s1) {
+        const uint64_t c = base + (uint64_t)s0;
+        const uint32_t c_lo = (uint32_t)c, c_hi = (uint32_t)(c >> 32);
+        const uint32_t left = 0u - c_lo;  // samples to the next high word, 0: all 2^32
+        int n = s1 - s0 < kMcFlush ? (int)(s1 - s0) : kMcFlush;
+        if (left && left < (uint32_t)n) n = (int)left;
+        T fa = T(0), fa2 = T(0);
+        for (int i = 0; i < n; ++i) {
+            T x[D];
+            mc_point<D, FOLD>(A.seed, c_lo + (uint32_t)i, c_hi, lo, sz, x);
+            const T f = eval_point<FAM, T, D>(x, D, A.p);
             fa += f;
             fa2 = fma(f, f, fa2);
         }
         acc += (double)fa;
         acc2 += (double)fa2;
+        s0 += n;
+    }
+}
+
+// D is exact (a bound of 4, 8 or 16 with run-time predicates cost two selects
+// per coordinate).  Bound by the vector unit: 36 Philox multiplies at about 7
+// cycles a wave and some 100 other operations per sample at d = 8.
+// Oscillatory, d = 8, FP32, 1e8 samples: 400 us before, 285 us now (3-input xors, exact D, the high
+// word's products and the 2^-24 out of the loop).
+template <typename T, int FAM, int D>
+__global__ __launch_bounds__(kBlock) void k_mc(McArgs<T> A) {
+    __shared__ double s_red[kWavesPerBlock];
+    T lo[D], sz[D];
+    bool fold = sizeof(T) == 4;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        lo[k] = A.domain[2 * k];
+        sz[k] = A.domain[2 * k + 1] - A.domain[2 * k];
+        // the scaled size is exact unless it leaves the normal range
+        if constexpr (sizeof(T) == 4) fold = fold && sz[k] * 0x1.0p-24f * 0x1.0p24f == sz[k];
+    }
+    const long long gt = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long s0 = gt * A.spt;
+    const long long s1 = (s0 + A.spt < A.N) ? (s0 + A.spt) : A.N;
+    double acc = 0.0, acc2 = 0.0;
+    if constexpr (sizeof(T) == 8) {
+        mc_samples<T, FAM, D, false>(A, lo, sz, s0, s1, acc, acc2);
+    } else if (fold) {
+#pragma unroll
+        for (int k = 0; k < D; ++k) sz[k] *= T(0x1.0p-24f);
+        mc_samples<T, FAM, D, true>(A, lo, sz, s0, s1, acc, acc2);
+    } else {
+        mc_samples<T, FAM, D, false>(A, lo, sz, s0, s1, acc, acc2);
     }
     const double b1 = block_sum(acc, s_red);
     const double b2 = block_sum(acc2, s_red);
@@ -231,6 +275,14 @@ static int check_mc(const tq_mc_desc* m) {
     return TQ_OK;
 }
 
+template <typename T, int FAM, int D = TQ_MAX_DIM>
+static void launch_mc_dim(const McArgs<T>& A, long long nb, hipStream_t st) {
+    if constexpr (D > 1) {
+        if (A.d < D) return launch_mc_dim<T, FAM, D - 1>(A, nb, st);
+    }
+    hipLaunchKernelGGL((k_mc<T, FAM, D>), dim3((unsigned)nb), dim3(kBlock), 0, st, A);
+}
+
 template <typename T>
 static int launch_mc(const tq_mc_desc* m, const tq_integrand* f, const void* domain, void* ws, size_t wsb,
                      void* out, double* stats, hipStream_t st, const uint64_t* offset_dev = nullptr) {
@@ -246,14 +298,7 @@ static int launch_mc(const tq_mc_desc* m, const tq_integrand* f, const void* dom
     A.domain = (const T*)domain;
     A.partials = (double*)ws;
     A.p = make_params<T>(*f);
-    TQ_DISPATCH_FAMILY(f->family, {
-        if (m->dim <= 4)
-            hipLaunchKernelGGL((k_mc<T, FAM, 4>), dim3((unsigned)nb), dim3(kBlock), 0, st, A);
-        else if (m->dim <= 8)
-            hipLaunchKernelGGL((k_mc<T, FAM, 8>), dim3((unsigned)nb), dim3(kBlock), 0, st, A);
-        else
-            hipLaunchKernelGGL((k_mc<T, FAM, TQ_MAX_DIM>), dim3((unsigned)nb), dim3(kBlock), 0, st, A);
-    });
+    TQ_DISPATCH_FAMILY(f->family, (launch_mc_dim<T, FAM>(A, nb, st)););
     int rc = check_launch("k_mc");
     if (rc) return rc;
     hipLaunchKernelGGL((k_mc_finalize<T>), dim3(1), dim3(1024), 0, st, (const double*)ws, nb, (const T*)domain,

@@ -109,6 +109,16 @@ struct u32x4 {
     uint32_t v[4];
 };
 
+// a ^ b ^ c of a round in one instruction: written with ^, the compiler makes
+// two (40 fewer per FP32 sample of eight coordinates).
+__device__ __host__ inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
+}
+
 __device__ __host__ inline u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
     const uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
@@ -119,9 +129,9 @@ __device__ __host__ inline u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1
         const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
         const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
         u32x4 n;
-        n.v[0] = hi1 ^ c.v[1] ^ k0;
+        n.v[0] = xor3(hi1, c.v[1], k0);
         n.v[1] = lo1;
-        n.v[2] = hi0 ^ c.v[3] ^ k1;
+        n.v[2] = xor3(hi0, c.v[3], k1);
         n.v[3] = lo0;
         c = n;
         k0 += W0;
@@ -132,13 +142,16 @@ __device__ __host__ inline u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1
 
 // The library's sample stream: sample s, block b of four 32-bit words uses
 // counter (lo32(s), hi32(s), b, 0) under key (lo32(seed), hi32(seed)).
-__device__ inline u32x4 philox_block(uint64_t seed, uint64_t s, uint32_t b) {
+__device__ inline u32x4 philox_block(uint64_t seed, uint32_t lo, uint32_t hi, uint32_t b) {
     u32x4 c;
-    c.v[0] = (uint32_t)s;
-    c.v[1] = (uint32_t)(s >> 32);
+    c.v[0] = lo;
+    c.v[1] = hi;
     c.v[2] = b;
     c.v[3] = 0u;
     return philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+}
+__device__ inline u32x4 philox_block(uint64_t seed, uint64_t s, uint32_t b) {
+    return philox_block(seed, (uint32_t)s, (uint32_t)(s >> 32), b);
 }
 
 // 32-bit word -> float in [0,1) with 24 random bits.
