@@ -365,7 +365,9 @@ __device__ inline unsigned long long f64_sig(double v) {
 // pass 1 for one (bin, value): count and largest exponent
 __device__ inline void hist_pass1(const HistSlots& h, int bin, double v) {
     atomicAdd(&h.cnt[bin], 1u);
-    if (v != 0.0) atomicMax(&h.exp[bin], f64_exp(v));
+    // the exponent only grows: an older value read here costs an atomic, never a wrong bin
+    const uint32_t e = v != 0.0 ? f64_exp(v) : 0u;
+    if (e > __hip_atomic_load(&h.exp[bin], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) atomicMax(&h.exp[bin], e);
 }
 
 // pass 2 for one (bin, value), after every pass 1 of the block
@@ -441,13 +443,36 @@ __device__ inline double uniform_coord<double>(uint64_t seed, uint64_t s, int k,
     return (k & 1) ? u01d(blk.v[2], blk.v[3]) : u01d(blk.v[0], blk.v[1]);
 }
 
-// MAXD: compile-time bound on the dimension; the fused launches use 8 for
-// d <= 8 so the unrolled per-axis work is not predicated over 16 axes.
-template <typename T, int FAM, int MODE, bool LDS_HIST, int MAXD = TQ_MAX_DIM>
+// Inclusive maximum over the lanes of a wave, values >= 0.
+template <int CTRL, int ROWS>
+__device__ inline int max_step(int v) {
+    const int o = __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+    return o > v ? o : v;
+}
+__device__ inline int wave_max_scan(int v) {
+    v = max_step<0x111, 0xF>(v);
+    v = max_step<0x112, 0xF>(v);
+    v = max_step<0x114, 0xF>(v);
+    v = max_step<0x118, 0xF>(v);
+    v = max_step<0x142, 0xA>(v);
+    return max_step<0x143, 0xC>(v);
+}
+
+// MIND, MAXD: compile-time bounds on the dimension (axes below MIND carry no
+// predicate).  Bound by the vector unit and the latency of the LDS gathers and
+// atomics: d = 6, FP32, 1.66e6 samples take 34 us, of which the vector unit
+// works 20 and LDS 9 (42 us with one class for d <= 8, a binary search per
+// sample and an unconditional exponent atomic per axis); more waves at fewer
+// registers spilled and lost 2 us.  Points: 16 axes unrolled four times took
+// 256 registers; classes and one run per block, 16.8 -> 7.2 us for 2000 FP64
+// samples at d = 4.
+template <typename T, int FAM, int MODE, bool LDS_HIST, int MIND, int MAXD>
 __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
     static_assert(MAXD % 2 == 0, "bin ids are packed in pairs");
-    using F = Family<FAM, T>;
     __shared__ int s_off[kOffLds];  // cube offsets relative to the block's first sample, clamped
+    uint16_t* s_cube = reinterpret_cast<uint16_t*>(s_off);  // fused: where a cube starts its index, else 0
+    static_assert(sizeof(int) * kOffLds >= sizeof(uint16_t) * kSB, "s_cube fits s_off");
+    __shared__ int s_last[kSB / kWave];
     __shared__ double s_map[kMapLds];
     // exact block histogram in dynamic LDS sized to the map (hist_slot_bytes)
     extern __shared__ __align__(16) unsigned char s_hist_raw[];
@@ -456,6 +481,7 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
     const int tid = threadIdx.x;
     const int d = st.dim, ni = st.n_intervals;
     const int W = d * ni;
+    auto axis = [d](int k) { return k < MIND || k < d; };
     const HistSlots hs = hist_slots(s_hist_raw, W);
     // the block's histogram values and packed bin ids, kept for pass 2
     double r_jf2[kSPT];
@@ -469,7 +495,10 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
         if (total > st.max_samples) total = st.max_samples;
     }
     const long long s0 = (long long)blockIdx.x * kSB;
-    if (s0 >= total) return;
+    // without a block histogram the runs of kBlock samples are blocks of their own
+    const int j0 = MODE == MODE_FUSED ? 0 : (int)blockIdx.y;
+    constexpr int kRuns = MODE == MODE_FUSED ? kSPT : 1;
+    if (s0 + (long long)j0 * kBlock >= total) return;
     const long long nblocks = (total + kSB - 1) / kSB;
 
     // map tables
@@ -495,24 +524,53 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
         h_lo = s_hrange[0];
         const long long h_hi = s_hrange[1];
         n_off = h_hi - h_lo + 2;  // offsets h_lo .. h_hi+1
-        off_lds = (n_off <= kOffLds);
-        // relative offsets clamped to [-1, kSB + 1]: the search compares them
-        // with s - s0 in [0, kSB), so the clamp changes no comparison
-        if (off_lds)
+        off_lds = n_off <= (MODE == MODE_FUSED ? 0xffff : kOffLds);
+        if (MODE == MODE_FUSED) {
+            for (int i = tid; i < kSB; i += kBlock) s_cube[i] = 0;
+        } else if (off_lds) {
+            // relative offsets clamped to [-1, kSB + 1]: the search compares them
+            // with s - s0 in [0, kSB), so the clamp changes no comparison
             for (long long i = tid; i < n_off; i += kBlock) {
                 long long r = st.offsets[h_lo + i] - s0;
                 r = r < -1 ? -1 : (r > kSB + 1 ? kSB + 1 : r);
                 s_off[i] = (int)r;
             }
+        }
     }
     __syncthreads();
+    // The cube of every sample: the cubes write their index at their first
+    // sample in the block, a running maximum over the samples spreads it (a
+    // binary search per sample was ten dependent LDS reads).
+    int cube[kRuns];
+    if (MODE == MODE_FUSED && off_lds) {
+        for (int i = tid; i < (int)n_off; i += kBlock) {
+            long long r = st.offsets[h_lo + i] - s0;
+            r = r < 0 ? 0 : r;
+            if (r < kSB && (i + 1 == (int)n_off || st.offsets[h_lo + i + 1] - s0 > r)) s_cube[r] = (uint16_t)i;
+        }
+        __syncthreads();
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & (kWave - 1);
+#pragma unroll
+        for (int j = 0; j < kRuns; ++j) {
+            cube[j] = wave_max_scan((int)s_cube[j * kBlock + tid]);
+            if (lane == kWave - 1) s_last[j * kWavesPerBlock + wave] = cube[j];
+        }
+        __syncthreads();
+        const int upto = wave_max_scan(lane < kSB / kWave ? s_last[lane] : 0);
+#pragma unroll
+        for (int j = 0; j < kRuns; ++j) {
+            const int c = j * kWavesPerBlock + wave;
+            const int before = c > 0 ? __builtin_amdgcn_readlane(upto, c - 1) : 0;
+            cube[j] = cube[j] > before ? cube[j] : before;
+        }
+    }
 
     // domain transform (vegas.py:104-112)
     T start[MAXD], size[MAXD];
     T vol = T(1);
 #pragma unroll
     for (int k = 0; k < MAXD; ++k) {
-        if (k < d && MODE != MODE_Y) {
+        if (axis(k) && MODE != MODE_Y) {
             start[k] = A.domain[2 * k];
             size[k] = A.domain[2 * k + 1] - A.domain[2 * k];
             vol = vol * size[k];
@@ -541,12 +599,14 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
     }
 
 #pragma unroll
-    for (int j = 0; j < kSPT; ++j) {
-        const long long s = s0 + (long long)j * kBlock + tid;
+    for (int j = 0; j < kRuns; ++j) {
+        const long long s = s0 + (long long)(j0 + j) * kBlock + tid;
         const bool active = s < total;
         long long h = 0;
         if (active && !A.warmup) {
-            if (off_lds) {
+            if (MODE == MODE_FUSED && off_lds) {
+                h = h_lo + cube[j];
+            } else if (off_lds) {
                 const int sr = (int)(s - s0);
                 int lo = 0, hi = (int)n_off - 1;  // find last i with s_off[i] <= s - s0
                 while (lo < hi) {
@@ -574,7 +634,7 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
         for (int k = 0; k < MAXD; ++k) {
             ids[k] = -1;
             x[k] = T(0);
-            if (k < d) {
+            if (axis(k)) {
                 const T u = (MODE != MODE_FUSED && A.u_in)
                                 ? (active ? A.u_in[s * d + k] : T(0))
                                 : uniform_coord<T>(A.seed, A.offset + (uint64_t)(active ? s : 0), k, blk);
@@ -614,9 +674,12 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
         if (MODE == MODE_Y) continue;
         if (MODE == MODE_POINTS) {
             if (active) {
-                for (int k = 0; k < d; ++k) {
-                    A.x_out[s * d + k] = x[k];
-                    A.ids_out[s * d + k] = ids[k];
+#pragma unroll
+                for (int k = 0; k < MAXD; ++k) {
+                    if (axis(k)) {
+                        A.x_out[s * d + k] = x[k];
+                        A.ids_out[s * d + k] = ids[k];
+                    }
                 }
                 A.jac_out[s] = jac;
             }
@@ -634,19 +697,19 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
                 r_jf2[j] = active ? jf2 : 0.0;
 #pragma unroll
                 for (int k = 0; k < MAXD; k += 2) {
-                    const uint32_t lo = (k < d) ? (uint32_t)ids[k] : 0u;
-                    const uint32_t hi = (k + 1 < d) ? (uint32_t)ids[k + 1] : 0u;
+                    const uint32_t lo = axis(k) ? (uint32_t)ids[k] : 0u;
+                    const uint32_t hi = axis(k + 1) ? (uint32_t)ids[k + 1] : 0u;
                     r_ids[j][k >> 1] = lo | (hi << 16);
                 }
                 if (active) {
 #pragma unroll
                     for (int k = 0; k < MAXD; ++k)
-                        if (k < d) hist_pass1(hs, k * ni + ids[k], jf2);
+                        if (axis(k)) hist_pass1(hs, k * ni + ids[k], jf2);
                 }
             } else {
 #pragma unroll
                 for (int k = 0; k < MAXD; ++k) {
-                    if (k < d) {
+                    if (axis(k)) {
                         const int id = active ? ids[k] : -1;
                         wave_hist_add_global(st.weights, st.counts, k, ni, id, jf2);
                     }
@@ -661,7 +724,7 @@ __global__ __launch_bounds__(kBlock) void k_vegas_sample(SampleArgs<T> A) {
             if (r_jf2[j] == 0.0) continue;
 #pragma unroll
             for (int k = 0; k < MAXD; ++k)
-                if (k < d) hist_pass2(hs, k * ni + (int)((r_ids[j][k >> 1] >> (16 * (k & 1))) & 0xffffu), r_jf2[j]);
+                if (axis(k)) hist_pass2(hs, k * ni + (int)((r_ids[j][k >> 1] >> (16 * (k & 1))) & 0xffffu), r_jf2[j]);
         }
         __syncthreads();
         for (int e = tid; e < W; e += kBlock) {
@@ -1708,6 +1771,30 @@ __global__ void k_zero(double* p, long long n) {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = 0.0;
 }
 
+// One launch of the sample kernel: a grid row of blocks, kSPT rows where a
+// block takes one run of kBlock samples.
+template <typename T, int FAM, int MODE, bool LDS_HIST, int MIND, int MAXD>
+static void launch_sample_dim(const SampleArgs<T>& A, long long nb, size_t lds, hipStream_t s) {
+    hipLaunchKernelGGL((k_vegas_sample<T, FAM, MODE, LDS_HIST, MIND, MAXD>),
+                       dim3((unsigned)nb, MODE == MODE_FUSED ? 1 : kSPT), dim3(kBlock), lds, s, A);
+}
+template <typename T, int FAM, int MODE>
+static void launch_sample(const SampleArgs<T>& A, long long nb, bool lds_hist, size_t lds, hipStream_t s) {
+    const int d = A.st.dim;
+    if constexpr (MODE == MODE_FUSED) {
+        if (!lds_hist) {
+            if (d <= 8) launch_sample_dim<T, FAM, MODE, false, 1, 8>(A, nb, 0, s);
+            else launch_sample_dim<T, FAM, MODE, false, 9, TQ_MAX_DIM>(A, nb, 0, s);
+            return;
+        }
+    }
+    constexpr bool H = MODE == MODE_FUSED;
+    if (d <= 4) launch_sample_dim<T, FAM, MODE, H, 1, 4>(A, nb, lds, s);
+    else if (d <= 6) launch_sample_dim<T, FAM, MODE, H, 5, 6>(A, nb, lds, s);
+    else if (d <= 8) launch_sample_dim<T, FAM, MODE, H, 7, 8>(A, nb, lds, s);
+    else launch_sample_dim<T, FAM, MODE, H, 9, TQ_MAX_DIM>(A, nb, lds, s);
+}
+
 template <typename T>
 static int vegas_iterate(const tq_vegas_state* st, const tq_integrand* f, const void* domain, uint64_t seed,
                          uint64_t offset, int it, int use_grid_improve, int warmup, long long n_warm,
@@ -1737,19 +1824,7 @@ static int vegas_iterate(const tq_vegas_state* st, const tq_integrand* f, const 
     const long long nb = sample_blocks(st, warmup, n_warm);
     // exact block histogram: 64-bit sum, exponent and count per bin
     const size_t hist_lds = (size_t)W * (8 + 4 + 4);
-    TQ_DISPATCH_FAMILY(f->family, {
-        if (lds_hist && st->dim <= 8)
-            hipLaunchKernelGGL((k_vegas_sample<T, FAM, MODE_FUSED, true, 8>), dim3((unsigned)nb), dim3(kBlock),
-                               hist_lds, s, A);
-        else if (lds_hist)
-            hipLaunchKernelGGL((k_vegas_sample<T, FAM, MODE_FUSED, true>), dim3((unsigned)nb), dim3(kBlock), hist_lds,
-                               s, A);
-        else if (st->dim <= 8)
-            hipLaunchKernelGGL((k_vegas_sample<T, FAM, MODE_FUSED, false, 8>), dim3((unsigned)nb), dim3(kBlock), 0,
-                               s, A);
-        else
-            hipLaunchKernelGGL((k_vegas_sample<T, FAM, MODE_FUSED, false>), dim3((unsigned)nb), dim3(kBlock), 0, s, A);
-    });
+    TQ_DISPATCH_FAMILY(f->family, (launch_sample<T, FAM, MODE_FUSED>(A, nb, lds_hist, hist_lds, s)););
     int rc = check_launch("k_vegas_sample");
     if (rc) return rc;
     return launch_iteration_tail(st, it, hist, warmup, n_warm, s);
@@ -1812,13 +1887,11 @@ int tq_vegas_points(const tq_vegas_state* st, const void* domain, uint64_t seed,
     if (st->sample_dtype == TQ_F32) {
         SampleArgs<float> A{*st, (const float*)domain, seed, offset, warmup, n_warm, 0, 0, (float*)x_out, jac_out,
                             ids_out, (float*)y_out, make_params<float>(dummy), (const float*)u_in};
-        hipLaunchKernelGGL((k_vegas_sample<float, TQ_FAM_CONSTANT, MODE_POINTS, false>), dim3((unsigned)nb),
-                           dim3(kBlock), 0, s, A);
+        launch_sample<float, TQ_FAM_CONSTANT, MODE_POINTS>(A, nb, false, 0, s);
     } else {
         SampleArgs<double> A{*st, (const double*)domain, seed, offset, warmup, n_warm, 0, 0, (double*)x_out,
                              jac_out, ids_out, (double*)y_out, make_params<double>(dummy), (const double*)u_in};
-        hipLaunchKernelGGL((k_vegas_sample<double, TQ_FAM_CONSTANT, MODE_POINTS, false>), dim3((unsigned)nb),
-                           dim3(kBlock), 0, s, A);
+        launch_sample<double, TQ_FAM_CONSTANT, MODE_POINTS>(A, nb, false, 0, s);
     }
     return check_launch("k_vegas_sample(points)");
 }
@@ -1945,13 +2018,11 @@ int tq_vegas_strat_y(const tq_vegas_state* st, uint64_t seed, uint64_t offset, c
     if (st->sample_dtype == TQ_F32) {
         SampleArgs<float> A{*st, nullptr, seed, offset, 0, 0, 0, 0, nullptr, nullptr, nullptr, (float*)y_out,
                             make_params<float>(dummy), (const float*)u_in};
-        hipLaunchKernelGGL((k_vegas_sample<float, TQ_FAM_CONSTANT, MODE_Y, false>), dim3((unsigned)nb),
-                           dim3(kBlock), 0, s, A);
+        launch_sample<float, TQ_FAM_CONSTANT, MODE_Y>(A, nb, false, 0, s);
     } else {
         SampleArgs<double> A{*st, nullptr, seed, offset, 0, 0, 0, 0, nullptr, nullptr, nullptr, (double*)y_out,
                              make_params<double>(dummy), (const double*)u_in};
-        hipLaunchKernelGGL((k_vegas_sample<double, TQ_FAM_CONSTANT, MODE_Y, false>), dim3((unsigned)nb),
-                           dim3(kBlock), 0, s, A);
+        launch_sample<double, TQ_FAM_CONSTANT, MODE_Y>(A, nb, false, 0, s);
     }
     return check_launch("k_vegas_sample(y)");
 }
