@@ -266,7 +266,7 @@ def require_device(tensor):
         raise NativeUnavailableError(
             "torchquad_amd computes on a ROCm GPU only and none is visible to torch"
         )
-    if tensor.device.type != "cuda":
+    if not tensor.is_cuda:
         raise NativeUnavailableError(
             "torchquad_amd computes on a ROCm GPU only; the integration domain is on "
             f"{tensor.device}. Call enable_cuda() / set_up_backend('torch') or pass a "
@@ -279,8 +279,7 @@ def require_device(tensor):
 
 def call(name, *args):
     """Call a status-returning entry point and raise NativeError on failure."""
-    fn = getattr(lib(), name)
-    rc = fn(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
         msg = lib().tq_last_error().decode(errors="replace")
         raise NativeError(name, rc, msg)
@@ -299,14 +298,15 @@ def stream_ptr(device=None):
         elif isinstance(device, int):
             idx = device
         else:
-            device = torch.device(device)
+            if not isinstance(device, torch.device):
+                device = torch.device(device)
             idx = device.index if device.index is not None else torch.cuda.current_device()
         return _raw_stream(idx)
     return torch.cuda.current_stream(device).cuda_stream
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def dtype_code(dtype):

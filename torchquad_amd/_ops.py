@@ -7,7 +7,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, autotune
 from ._lib import call, lib, ptr, require_device, stream_ptr, workspace
 
 RULES = {
@@ -19,13 +19,7 @@ RULES = {
 
 
 def grid_desc(rule, dim, n, dtype, gl=None, lane_axes=0, items_per_wave=0):
-    g = _lib.GridDesc()
-    g.dtype = _lib.dtype_code(dtype)
-    g.rule = int(rule)
-    g.dim = int(dim)
-    g.n = int(n)
-    g.lane_axes = int(lane_axes)
-    g.items_per_wave = int(items_per_wave)
+    g = _lib.GridDesc(_lib.dtype_code(dtype), int(rule), int(dim), int(n), int(lane_axes), int(items_per_wave))
     if gl is not None:
         g.gl_nodes = gl[0].data_ptr()
         g.gl_weights = gl[1].data_ptr()
@@ -35,9 +29,7 @@ def grid_desc(rule, dim, n, dtype, gl=None, lane_axes=0, items_per_wave=0):
 def _fused_grid_desc(rule, integrand, dim, n, dtype, gl, lane_axes, items_per_wave):
     desc = integrand.descriptor(dim)
     if items_per_wave == 0 and lane_axes == 0:
-        from .autotune import grid_ipw
-
-        items_per_wave = grid_ipw(rule, desc.family, dim, n, dtype)
+        items_per_wave = autotune.grid_ipw(rule, desc.family, dim, n, dtype)
     return grid_desc(rule, dim, n, dtype, gl, lane_axes, items_per_wave), desc
 
 
@@ -74,7 +66,7 @@ def grid_integrate(rule, integrand, dim, n, domain, gl=None, lane_axes=0, items_
         ws = workspace.get(max(nbytes, 8), domain.device, stream=stream)
     elif ws.numel() < nbytes:
         raise ValueError(f"workspace of {ws.numel()} bytes, {nbytes} needed")
-    out = torch.empty((), dtype=domain.dtype, device=domain.device)
+    out = torch.empty_strided((), (), dtype=domain.dtype, device=domain.device)  # cheaper on the host than empty
     call(
         "tq_grid_integrate",
         ctypes.byref(g),

@@ -107,6 +107,8 @@ _file_tried = False  # grid_ipw looked for TQ_AUTOTUNE_CACHE once
 def grid_ipw(rule, family, dim, n, dtype):
     """Tuned items-per-wave of the fused grid kernel for this geometry, or 0 (automatic)."""
     global _file_tried
+    if not _cache and _file_tried:
+        return 0
     key = _grid_key(rule, family, dim, n, dtype)
     hit = _cache.get(key)
     if hit is None and not _cache and not _file_tried:

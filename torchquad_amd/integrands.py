@@ -59,6 +59,12 @@ def _dim_of(v):
     return 1 if arr.ndim == 0 else int(arr.shape[-1])
 
 
+def _floats(values, n):
+    """The first n parameters as a list (one conversion: indexing a numpy array
+    costs more per element than the whole of it)."""
+    return values[:n].tolist() if isinstance(values, np.ndarray) else [values[k] for k in range(n)]
+
+
 class BuiltinIntegrand:
     """Base class: a family id, a dimension and float64 parameters.
 
@@ -178,9 +184,8 @@ class GaussianPeak(BuiltinIntegrand):
 
     def _fill(self, d, i):
         a, u = self._ax("a", i), self._ax("u", i)
-        for k in range(self.dim):
-            d.a[k] = a[k]
-            d.u[k] = u[k]
+        d.a[: self.dim] = _floats(a, self.dim)
+        d.u[: self.dim] = _floats(u, self.dim)
 
     def torch_eval(self, x):
         a, u = self._t(self.a, x), self._t(self.u, x)
@@ -198,8 +203,7 @@ class Oscillatory(BuiltinIntegrand):
     def _fill(self, d, i):
         d.c1 = self._sc("w", i)
         c = self._ax("c", i)
-        for k in range(self.dim):
-            d.a[k] = c[k]
+        d.a[: self.dim] = _floats(c, self.dim)
 
     def torch_eval(self, x):
         c = self._t(self.c, x)
@@ -218,9 +222,8 @@ class ProductPeak(BuiltinIntegrand):
 
     def _fill(self, d, i):
         a, u = self._ax("a", i), self._ax("u", i)
-        for k in range(self.dim):
-            d.a[k] = a[k]
-            d.u[k] = u[k]
+        d.a[: self.dim] = _floats(a, self.dim)
+        d.u[: self.dim] = _floats(u, self.dim)
 
     def torch_eval(self, x):
         a, u = self._t(self.a, x), self._t(self.u, x)
@@ -238,8 +241,7 @@ class ExpLinear(BuiltinIntegrand):
     def _fill(self, d, i):
         d.c1 = self._sc("c", i)
         a = self._ax("a", i)
-        for k in range(self.dim):
-            d.a[k] = a[k]
+        d.a[: self.dim] = _floats(a, self.dim)
 
     def torch_eval(self, x):
         return torch.exp(self._t(self.c, x) + torch.sum(x * self._t(self.a, x), dim=-1))
@@ -255,9 +257,8 @@ class SinSum(BuiltinIntegrand):
 
     def _fill(self, d, i):
         a, u = self._ax("a", i), self._ax("u", i)
-        for k in range(self.dim):
-            d.a[k] = a[k]
-            d.u[k] = u[k]
+        d.a[: self.dim] = _floats(a, self.dim)
+        d.u[: self.dim] = _floats(u, self.dim)
 
     def torch_eval(self, x):
         return torch.sum(torch.sin(x * self._t(self.a, x) + self._t(self.u, x)), dim=-1)

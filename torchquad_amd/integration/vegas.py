@@ -219,7 +219,8 @@ class VEGAS(BaseIntegrator):
         else:
             total = int(dev.offsets[-1].item())
         dom = self._domain
-        unit = torch.tensor([[0.0, 1.0]] * self._dim, dtype=dom.dtype, device=dom.device)
+        # with domain gradients the kernels sample the unit box (a host-to-device copy otherwise left out)
+        box = torch.tensor([[0.0, 1.0]] * self._dim, dtype=dom.dtype, device=dom.device) if self._grad else dom.detach()
         x = torch.empty((total, self._dim), dtype=dom.dtype, device=dom.device)
         jac = torch.empty((total,), dtype=torch.float64, device=dom.device)
         ids = torch.empty((total, self._dim), dtype=torch.int32, device=dom.device)
@@ -230,25 +231,24 @@ class VEGAS(BaseIntegrator):
         else:
             u = self.rng.uniform(size=[total, self._dim], dtype=dom.dtype).to(dom.device).contiguous()
             first, seed = 0, 0
-        call("tq_vegas_points", dev.struct, ptr(unit if self._grad else dom.detach()), seed, first, 1 if warmup else 0,
+        call("tq_vegas_points", dev.struct, ptr(box), seed, first, 1 if warmup else 0,
              n_samples if warmup else 0, ptr(u), ptr(x), ptr(jac), ptr(ids), None, dev.stream())
-        starts = dom[:, 0]
-        sizes = dom[:, 1] - starts
         if self._grad:
-            x = x * sizes + starts
+            starts = dom[:, 0]
+            x = x * (dom[:, 1] - starts) + starts
         values, num = self.evaluate_integrand(self._fn, x)
         self._nr_of_fevals += num
         values = values.squeeze()
         if values.dim() != 1:
             raise ValueError("VEGAS supports only scalar integrands")
         vals = values.detach().to(dom.dtype).contiguous()
-        call("tq_vegas_consume", dev.struct, ptr(vals), ptr(unit if self._grad else dom.detach()), ptr(jac),
+        call("tq_vegas_consume", dev.struct, ptr(vals), ptr(box), ptr(jac),
              ptr(ids), slot, 1 if self.use_grid_improve else 0, 1 if warmup else 0, n_samples if warmup else 0,
              dev.stream())
         if warmup or not (self._grad or values.requires_grad):
             return None
         # differentiable iteration result: sum_s V/nh(s) * jac_s * vol * f_s
-        volume = torch.prod(sizes)
+        volume = torch.prod(dom[:, 1] - dom[:, 0])
         nh = dev.nh
         per_sample = torch.repeat_interleave(self.strat.V_cubes / nh.to(torch.float64), nh, output_size=total)
         coef = (per_sample * jac).to(values.dtype)
