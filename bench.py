@@ -45,9 +45,9 @@ CLOCK_GHZ = 2.4  # MI355X peak engine clock
 # Algorithmic FLOPs per evaluation of the dim-5 Gaussian peak
 # exp(-sum_i a_i^2 (x_i - u_i)^2) with its quadrature weight: 4d+3 arithmetic
 # (+, -, x = 1, FMA = 2) plus 1 exp = 24.  The fused kernel executes far
-# fewer per point (row and lane partial sums are shared across points), so
-# this count is reported only as an "algorithmic-equivalent" rate; the
-# roofline uses the executed FP32 operations from the committed counter pass.
+# fewer per point (per-axis factors are shared across points), so this count
+# is reported only as an "algorithmic-equivalent" rate; the roofline uses the
+# executed FP32 operations from the committed counter pass.
 DIM_C2A = 5
 FLOPS_PER_EVAL_GRID_GAUSSIAN = 4 * DIM_C2A + 3 + 1
 COPY_BYTES = 256 << 20
@@ -76,7 +76,7 @@ def load_valu():
 def probe_rates(dev):
     """The device's own rates for the fused grid kernel's loop (tq_probe_rates):
     cycles per wave instruction of FP32 FMA and exp2 chains at the nominal
-    clock, and the evaluations/s of the loop body alone."""
+    clock, and the evaluations/s of the loop body alone with 4 and 8 states."""
     import ctypes
 
     import torch
@@ -101,7 +101,9 @@ def probe_rates(dev):
         if kind < 2:
             res["fma_cycles" if kind == 0 else "exp2_cycles"] = sec * CLOCK_GHZ * 1e9 / (waves_per_simd * iters * 32)
         else:
-            res["loop_evals_per_s" if kind == 3 else "loop_weighted_evals_per_s"] = blocks * 256 * iters * 256 / sec
+            states = 4 * (kind - 1)
+            res["loop_evals_per_s" if kind == 3 else "loop_4_states_evals_per_s"] = (
+                blocks * 256 * iters * 256 * states / sec)
     return res
 
 
@@ -772,21 +774,20 @@ def main():
     alg_tflops = FLOPS_PER_EVAL_GRID_GAUSSIAN * evals_per_s / 1e12
     roofline = {
         "bound": "valu",
-        "kernel": "k_grid_fused<float, GAUSSIAN_PEAK, table, rowtab, 8 waves> (one launch per step)",
+        "kernel": "k_grid_product<float, GAUSSIAN_PEAK, 8> (one launch per step)",
         "achieved": None,
         "peak": PEAK_FP32_TFLOPS,
         "unit": "TFLOP/s",
         "frac": None,
         "bound_note": "vector ALU (no HBM stream or matrix product on this path): MI355X's FP32 157.3 TFLOP/s; "
-                      "each evaluation is one add, one exp2 and one FMA, and the exp2 issues at about a quarter "
-                      "of the FMA rate (see attainable), so the kernel is bound by its exp2 issue well below "
-                      "the FMA peak",
+                      "each evaluation multiplies its per-axis factors and adds the value in one FMA; the rest is "
+                      "the factor tables that every workgroup evaluates in FP64 before its loop",
         "traffic": load_traffic(),
         "algorithmic_equivalent": {
             "flops_per_eval": FLOPS_PER_EVAL_GRID_GAUSSIAN,
             "tflops": alg_tflops,
             "note": "4d+3 arithmetic + 1 exp per evaluation at d=5 as if each point were evaluated from "
-                    "scratch; not a hardware rate (the kernel shares row and lane partial sums)",
+                    "scratch; not a hardware rate (the kernel shares the per-axis factors across points)",
         },
     }
     rates = probe_rates(dev)
@@ -795,12 +796,11 @@ def main():
         "frac_of_loop": evals_per_s / rates["loop_evals_per_s"],
         "fma_cycles_per_wave_instruction": rates["fma_cycles"],
         "exp2_cycles_per_wave_instruction": rates["exp2_cycles"],
-        "loop_weighted_evals_per_s": rates["loop_weighted_evals_per_s"],
+        "loop_4_states_evals_per_s": rates["loop_4_states_evals_per_s"],
         "note": "tq_probe_rates on this GPU, cycles at the nominal 2.4 GHz: independent FP32 FMA and exp2 "
-                "chains, and the grid loop's body alone as the kernel runs it for this family (state + "
-                "4-byte LDS table term with the weight folded in, exp2, add, 16 points per trip) with none "
-                "of the kernel's tables, rows, flushes or tail; loop_weighted_evals_per_s: the same body "
-                "with (term, weight) entries and a weighted FMA, the form of the non-folding families",
+                "chains, and the grid loop's body alone as the kernel runs it (a loop factor from LDS, one FMA "
+                "with each of the lane's 8 own factors; 4 in loop_4_states) with none of the kernel's tables, "
+                "rows, flushes or tail",
     }
     if valu:
         flops_eval = valu["executed_fp32_flops_per_eval"]

@@ -309,10 +309,9 @@ int tq_sweep_backward(const tq_grid_desc* g, int32_t family, int64_t B, const vo
  * No counterpart in the reference: a measurement hook for the benchmark,
  * which states the fused grid kernel's rate against the device's own rate
  * for the kernel's inner loop.  kind 0: independent FP32 FMA chains, 32
- * instructions per lane and trip; 1: FP32 exp2 chains, likewise; 2: the
- * grid loop's body with (term, weight) table entries (state + LDS table
- * term, exp2, weighted FMA), 256 points per lane and trip; 3: the body with
- * the weight folded into 4-byte entries (state + term, exp2, add).  Launches
+ * instructions per lane and trip; 1: FP32 exp2 chains, likewise; 2 and 3: the
+ * grid loop's body (a loop factor from LDS, one FMA with each of the lane's
+ * own factors), 4 factors or 8, 1024 or 2048 points per lane and trip.  Launches
  * blocks x 256 threads for iters trips; out: device float[blocks * 256]. */
 int tq_probe_rates(int32_t kind, int64_t blocks, int32_t iters, float* out, void* stream);
 

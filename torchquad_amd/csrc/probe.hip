@@ -8,35 +8,28 @@ namespace tq {
 constexpr int kProbeTable = 256;  // loop-table entries of the point-loop probe
 
 // KIND 0: eight independent v_fma_f32 chains per lane; 1: eight v_exp_f32
-// chains; 2: the grid loop's body per point with an (term, weight) table --
-// the lane's state plus an LDS table term (wave-uniform address), exp2, FMA
-// with the table weight into the lane's partial; 3: the body with the weight
-// folded into the term (4-byte entries, exp2, add), as the kernel runs it for
-// the Gaussian peak.  Each trip is 32 instructions (0, 1) or 256 points (2, 3).
+// chains; 2, 3: the product grid loop's body -- a loop factor from LDS at a
+// wave-uniform address and one multiply-add per point with each of the lane's
+// own factors, four (2) or eight (3) of them.  Each trip is 32 instructions
+// (0, 1), 1024 points (2) or 2048 (3).
 template <int KIND>
 __global__ __launch_bounds__(kBlock) void k_probe(float* out, int iters) {
-    __shared__ float2 tab[kProbeTable];
-    __shared__ float tab1[kProbeTable];
-    for (int j = threadIdx.x; j < kProbeTable; j += kBlock) {
-        tab[j] = make_float2(-0.001f * (float)j, 1.0f / (1.0f + (float)j));
-        tab1[j] = -0.001f * (float)j - log2f(1.0f + (float)j);
-    }
+    __shared__ float tab[kProbeTable];
+    for (int j = threadIdx.x; j < kProbeTable; j += kBlock) tab[j] = 0.001f * (float)(j + 1);
     __syncthreads();
     float a[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) a[k] = 0.1f + 0.01f * (float)((threadIdx.x + k) & 31);
-    const float s_rl = -0.01f * (float)(threadIdx.x & 63);
-    float acc = 0.0f;
+    float acc = 0.0f, sum[8] = {};
     for (int i = 0; i < iters; ++i) {
-        if (KIND == 2) {
-#pragma unroll 16
+        if (KIND >= 2) {
+#pragma unroll 8
             for (int j = 0; j < kProbeTable; ++j) {
-                const float2 e = tab[j];
-                acc = fmaf(e.y, __builtin_amdgcn_exp2f(s_rl + e.x), acc);
+                const float e = tab[j];
+#pragma unroll
+                for (int k = 0; k < 4 * (KIND - 1); ++k) sum[k & 7] = fmaf(a[k & 7], e, sum[k & 7]);
             }
-        } else if (KIND == 3) {
-#pragma unroll 16
-            for (int j = 0; j < kProbeTable; ++j) acc += __builtin_amdgcn_exp2f(s_rl + tab1[j]);
+            asm volatile("" ::: "memory");  // the table is read again on every trip
         } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -47,7 +40,7 @@ __global__ __launch_bounds__(kBlock) void k_probe(float* out, int iters) {
         }
     }
 #pragma unroll
-    for (int k = 0; k < 8; ++k) acc += a[k];
+    for (int k = 0; k < 8; ++k) acc += a[k] + sum[k];
     out[(long long)blockIdx.x * kBlock + threadIdx.x] = acc;
 }
 

@@ -423,22 +423,26 @@ inline bool split_product_axes(int d, int n, int K, int C, int tsize, long long 
                                int lane_axes, size_t lds_max, ProductSplit& S, int max_q = 2) {
     if (d < 2 || n < 2) return false;
     double best = -1.0;
+    double power[TQ_MAX_DIM + 1];  // n^i (the host plans thousands of integrals a batch: no libm calls here)
+    power[0] = 1.0;
+    for (int i = 1; i <= d; ++i) power[i] = power[i - 1] * n;
     for (int q = 1; q <= max_q && q < d; ++q) {
-        const double nl = q == 2 ? (double)n * n : (double)n, groups = std::ceil(nl / kGroup);
-        if (groups * kGroup > (double)max_entries) break;
+        const long long nl = q == 2 ? (long long)n * n : n, groups = (nl + kGroup - 1) / kGroup;
+        if (groups * kGroup > max_entries) break;
         for (int m = 1; m <= d - q; ++m) {
             if (lane_axes > 0 && m != lane_axes) continue;
             for (int outer = 1; outer <= 2 && outer <= m; ++outer) {
-                const double N = outer == 2 ? (double)n * n : (double)n;
-                if (outer == 2 && N > (double)max_outer) break;
-                const double H = std::ceil(N / K), slots = H * std::pow((double)n, m - outer);
-                if (slots > (double)(1 << 30)) break;
+                const long long N = outer == 2 ? (long long)n * n : n;
+                if (outer == 2 && N > max_outer) break;
+                const long long H = (N + K - 1) / K;
+                if ((double)H * power[m - outer] > (double)(1 << 30)) break;
+                const long long slots = H * (long long)power[m - outer], lane_groups = (slots + kWave - 1) / kWave;
                 const int L = d - q - m;
-                const double rows = std::pow((double)n, L);
-                const double row = groups * kGroup * K * C + (L > 0 ? 30 + 8 * L + 2 * K * C : 0) +
-                                   std::ceil(groups / (kFlush / kGroup)) * 8;
-                const double init = 20 + 12 * (m - outer) + K * (5 + 3 * C);
-                const double work = std::ceil(slots / kWave) * (init + std::round(rows) * row);
+                constexpr int kFlushGroups = kFlush / kGroup;
+                const long long row = groups * kGroup * K * C + (L > 0 ? 30 + 8 * L + 2 * K * C : 0) +
+                                      (groups + kFlushGroups - 1) / kFlushGroups * 8;
+                const long long init = 20 + 12 * (m - outer) + K * (5 + 3 * C);
+                const double work = (double)lane_groups * ((double)init + power[L] * (double)row);
                 if (best >= 0.0 && work >= best) continue;
                 ProductSplit X;
                 X.d = d;
@@ -453,7 +457,7 @@ inline bool split_product_axes(int d, int n, int K, int C, int tsize, long long 
                 X.groups = (int)groups;
                 if (product_lds_bytes(X, C, tsize) > lds_max) continue;
                 X.slots = (int)slots;
-                X.lane_groups = (int)std::ceil(slots / kWave);
+                X.lane_groups = (int)lane_groups;
                 long long r;
                 if (ipow_checked(n, L, (1LL << 62) / X.groups, &r) != 0) continue;
                 X.items = r * X.groups;
