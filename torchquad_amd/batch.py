@@ -1,10 +1,10 @@
-"""Batched form: many parameterised integrals in one launch per LDS class.
+"""Batched form: many parameterised integrals in one launch.
 
 A :class:`Batch` takes a list of integrals -- rule, built-in integrand,
 dimension, total point count N (rounded per axis exactly as the reference's
 integrators round it) and domain -- plans them once on the host (C ABI
 ``tq_batch_plan``), keeps the plan on the device and runs all of them with
-one wave per tile (one kernel per LDS class) plus one per-integral
+a wave or a workgroup per tile (one launch for the usual classes) plus one per-integral
 reduction (``tq_batch_run``).  The launches have no host synchronisation and
 no memset, so :meth:`Batch.graph` captures them in a HIP graph for replay.
 
