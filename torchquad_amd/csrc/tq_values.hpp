@@ -355,11 +355,10 @@ inline int plan_values(int d, int n, int rule, const double* glw, long long P, l
     if (d > 0) {
         long long inner = n;
         int m = 1;
-        while (m < d && n > 1 && inner * n <= kInnerMax) {
+        while (m < d && n > 1 && inner * n <= kInnerMax) {  // one node per axis: the other axes stay outer ones
             inner *= n;
             ++m;
         }
-        if (n == 1) m = d;
         w.inner = (uint32_t)inner;
         w.outer_axes = d - m;
         w.by_n = make_fast_div((uint32_t)n);
