@@ -1,0 +1,62 @@
+"""The product form of the fused rules where single points decide the result:
+infinite values, weights of very different sizes, partial sums that need more
+than 24 bits, nodes to the last bit."""
+import ctypes
+from fractions import Fraction
+
+import numpy as np
+import pytest
+import torch
+
+import torchquad_amd as tq
+from torchquad_amd import _lib, _ops
+from torchquad_amd.autograd import product_peak_integrals
+from torchquad_amd.batch import Batch
+
+pytestmark = pytest.mark.gpu
+
+GL = _ops.RULES["gauss_legendre"]
+
+
+def _table(x, w, dev):
+    return torch.tensor(x, dtype=torch.float64, device=dev), torch.tensor(w, dtype=torch.float64, device=dev)
+
+
+def _grid64(fn, d, n, dom, gl=None, rule=GL):
+    out = torch.zeros((), dtype=torch.float64, device=dom.device)
+    _ops.grid_integrate(rule, fn, d, n, dom, gl, out_f64=out)
+    return float(out)
+
+
+# (dim, n) with and without a last group of loop points and a last lane group that are not full
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("d,n", [(3, 9), (3, 17), (4, 13), (5, 5), (3, 65)])
+def test_one_singular_axis_is_infinite(d, n, dtype, dev):
+    """A product peak whose peak on one axis is a pole on a node: +inf, in a
+    grid, in a batch (one and many tiles) and in a sweep; its neighbours keep
+    their values."""
+    big = 1e30 if dtype == torch.float32 else 1e200
+    dom = torch.tensor([[0.0, 1.0]] * d, dtype=dtype, device=dev)
+    items, a_rows = [], []
+    for k in range(d):
+        a = [1.0] * d
+        a[k] = big
+        fn = tq.ProductPeak(a, [0.5] * d)
+        assert _grid64(fn, d, n, dom, rule=_ops.RULES["simpson"]) == float("inf"), k
+        items.append({"rule": "simpson", "fn": fn, "dim": d, "n": n, "domain": [[0.0, 1.0]] * d})
+        a_rows += [a, [1.0] * d]
+    items.append({"rule": "simpson", "fn": tq.ProductPeak([1.0] * d, [0.5] * d), "dim": d, "n": n,
+                  "domain": [[0.0, 1.0]] * d})
+    x = np.linspace(0.0, 1.0, n)
+    w = np.full(n, 2.0)
+    w[1::2], w[0], w[-1] = 4.0, 1.0, 1.0
+    ref = (np.sum(w / (1.0 + (x - 0.5) ** 2)) / (n - 1) / 3.0) ** d
+    bar = 1e-6 if dtype == torch.float32 else 1e-12  # this package's bars for fused grid rules
+    for tile_points in (64, 8192):
+        out = Batch(items, dtype=dtype, device=dev, tile_points=tile_points).run()[1]
+        assert bool(torch.isinf(out[:d]).all()) and bool((out[:d] > 0).all())
+        assert abs(float(out[d]) - ref) <= bar * ref
+    a = torch.tensor(a_rows, dtype=dtype, device=dev)
+    val = product_peak_integrals(a, torch.full_like(a, 0.5), dom.repeat(2 * d, 1, 1), n=n, rule="simpson").double()
+    assert bool((val[0::2] == float("inf")).all())
+    assert float((val[1::2] - ref).abs().max()) <= bar * ref

@@ -235,11 +235,7 @@ __device__ __forceinline__ void product_block(const BatchDev<T>& D, const tq_bat
 #undef TQ_BP
     }
     acc = block_sum(acc, s_red);
-    if (tid == 0) {
-        int exponent = 0;
-        for (int k = 0; k < D.d; ++k) exponent += exp_or_zero(s_exp[k]);
-        *part = ldexp(acc, exponent);
-    }
+    if (tid == 0) *part = scale_back(acc, D.d, s_exp);
 }
 
 // Product tiles alone (big tables; runs without classes).

@@ -72,12 +72,8 @@ __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, 
     if (!sum_over_blocks(acc, A.sums, s_red, &v)) return;
     if (tid == 0) {
         double scale = A.c0;
-        int exponent = 0;
-        for (int k = 0; k < d; ++k) {
-            scale *= s_scale[k];
-            exponent += exp_or_zero(s_exp[k]);
-        }
-        const double r = ldexp(v, exponent) * scale;
+        for (int k = 0; k < d; ++k) scale *= s_scale[k];
+        const double r = scale_back(v, d, s_exp) * scale;
         if (A.out) *A.out = (T)r;
         if (A.out64) *A.out64 = r;
     }

@@ -98,11 +98,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_fwd(SweepUnits 
         acc += sum_items<FAM, T, K>(S, tab, own, t0, t1);
     }
     acc = block_sum(acc, s_red);
-    if (tid == 0) {
-        int exponent = 0;
-        for (int k = 0; k < S.d; ++k) exponent += exp_or_zero(s_exp[k]);
-        partials[b * gridDim.x + blockIdx.x] = ldexp(acc, exponent);
-    }
+    if (tid == 0) partials[b * gridDim.x + blockIdx.x] = scale_back(acc, S.d, s_exp);
 }
 
 // Loop-axis sums kept beside F.
@@ -153,7 +149,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
         if (FAM == TQ_FAM_PRODUCT_PEAK) s_g[e] = (T)(1.0 / fma((double)t, (double)t, (double)s_p.b[k]));
         if (k == 0) s_r[j] = (T)node_r(j, n, U.rule, glx);
     }
-    const ProductTables<T> tab = build_product_tables<FAM, T>(S, U.rule, s_axis, glx, glw, s_p, s_lds, s_exp);
+    const ProductTables<T> tab = build_product_tables<FAM, T, false>(S, U.rule, s_axis, glx, glw, s_p, s_lds, s_exp);
     auto functions = [&](int k, int j, double* h) {
         sweep_functions<FAM>((double)s_t[k * n + j], FAM == TQ_FAM_PRODUCT_PEAK ? (double)s_g[k * n + j] : 0.0,
                              (double)s_r[j], h);

@@ -47,12 +47,27 @@ __device__ inline double factor_exponent(int k, T x, const Params<T>& p) {
     return e > 1e8 ? 1e8 : (e < -1e8 ? -1e8 : e);
 }
 
+// Denominator of the product peak's factor on axis k.
+template <typename T>
+__device__ inline double peak_denominator(int k, T x, const Params<T>& p) {
+    const double t = (double)x - (double)p.u[k];
+    return fma(t, t, (double)p.b[k]);
+}
+
+// A node on which the product peak has a pole (a denominator of zero, or one
+// whose reciprocal may leave the FP64 range).  Stored as it is, the infinite
+// factor would meet the zeros of lanes and loop entries past the end and make
+// NaN of an integral that is infinite; so its axis keeps the signs of the
+// poles' weights alone, everything else on it counting for nothing beside
+// them, and an exponent that takes any sum but 0 out of the range.
+constexpr int kPoleExp = 1 << 27;  // above every other exponent
+__device__ inline bool is_pole(double denominator) { return fabs(denominator) < 0x1.0p-1022; }
+
 // Weighted factor of a family that is not exponential.
 template <int FAM, typename T>
 __device__ inline void factor_comps(int k, T x, double w, const Params<T>& p, double* v) {
     if constexpr (FAM == TQ_FAM_PRODUCT_PEAK) {
-        const double t = (double)x - (double)p.u[k];
-        v[0] = w / fma(t, t, (double)p.b[k]);
+        v[0] = w / peak_denominator(k, x, p);
     } else if constexpr (FAM == TQ_FAM_OSCILLATORY) {
         double s, c;
         double phase = (double)p.a[k] * (double)x;  // FP32: revolutions, FP64: radians
@@ -123,19 +138,33 @@ __device__ inline int exp_or_zero(int e) { return e == -0x7fffffff ? 0 : e; }
 // Exponent that a node's weighted factor does not exceed by more than one,
 // without evaluating the factor: the power of two that its axis is scaled by
 // is the largest of these.
-template <int FAM, typename T>
+template <int FAM, typename T, bool POLES>
 __device__ inline int factor_scale(int k, T x, double w, double ex, const Params<T>& p) {
     const int m = mag_exp(w);
     if (m == -0x7fffffff) return m;
     if constexpr (family_exponential(FAM)) {
         return ex == ex ? m + (int)ceil(ex) : -0x7fffffff;
     } else if constexpr (FAM == TQ_FAM_PRODUCT_PEAK) {
-        const double t = (double)x - (double)p.u[k];
-        const int e = mag_exp(fma(t, t, (double)p.b[k]));
+        const double den = peak_denominator(k, x, p);
+        if (POLES && is_pole(den)) return kPoleExp;
+        const int e = mag_exp(den);
         return e == -0x7fffffff ? e : m - e + 1;
     } else {
         return m;
     }
+}
+
+// A block's sum v with the powers of two put back that were taken out of its
+// axes.  A pole on every axis: NaN, as from a sum over 0 times infinity.
+__device__ inline double scale_back(double v, int d, const int* s_exp) {
+    long long e = 0;
+    int poles = 0;
+    for (int k = 0; k < d; ++k) {
+        e += exp_or_zero(s_exp[k]);
+        poles += s_exp[k] >= kPoleExp ? 1 : 0;
+    }
+    if (poles == d) return __longlong_as_double(0x7ff8000000000000ll);
+    return ldexp(v, (int)(e > (1 << 30) ? (1 << 30) : (e < -(1 << 30) ? -(1 << 30) : e)));
 }
 
 // Axis tables of a whole block: component c of axis k's node j goes to
@@ -145,7 +174,7 @@ __device__ inline int factor_scale(int k, T x, double w, double ex, const Params
 // earlier form, one wave per axis with the factors in registers, left most
 // lanes idle on short axes and evaluated long ones up to three times).  Ends
 // with a barrier.
-template <int FAM, typename T>
+template <int FAM, typename T, bool POLES>
 __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax, const double* glx,
                                           const double* glw, const Params<T>& p, FastDiv by_n, T* axis, int* s_exp) {
     constexpr int C = family_comps(FAM);
@@ -168,7 +197,7 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
         if constexpr (EXP) v.ex = factor_exponent<FAM, T>(v.k, v.x, p);
         return v;
     };
-    auto scale = [&](const Node& v) { atomicMax(&s_exp[v.k], factor_scale<FAM, T>(v.k, v.x, v.w, v.ex, p)); };
+    auto scale = [&](const Node& v) { atomicMax(&s_exp[v.k], factor_scale<FAM, T, POLES>(v.k, v.x, v.w, v.ex, p)); };
     auto store = [&](const Node& nd, int e) {
         const int m = exp_or_zero(s_exp[nd.k]);
         double v[C];
@@ -176,8 +205,13 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
             v[0] = nd.w * exp2(nd.ex - (double)m);
         } else {
             factor_comps<FAM, T>(nd.k, nd.x, nd.w, p, v);
+            if (FAM == TQ_FAM_PRODUCT_PEAK && POLES && m >= kPoleExp) {
+                if (is_pole(peak_denominator(nd.k, nd.x, p))) v[0] = copysign(1.0, v[0]);
+                else if (v[0] == v[0]) v[0] = 0.0;
+            } else {
 #pragma unroll
-            for (int c = 0; c < C; ++c) v[c] = ldexp(v[c], -m);
+                for (int c = 0; c < C; ++c) v[c] = ldexp(v[c], -m);
+            }
         }
 #pragma unroll
         for (int c = 0; c < C; ++c) axis[c * total + e] = (T)v[c];
@@ -324,8 +358,9 @@ __host__ __device__ inline size_t product_lds_bytes(const ProductSplit& S, int C
            (S.outer == 2 ? (size_t)C * S.N * tsize : 0);
 }
 
-// Builds them (all threads of the block; ends with a barrier).
-template <int FAM, typename T>
+// Builds them (all threads of the block; ends with a barrier).  POLES: an
+// infinite factor as the sign of its weight (kPoleExp), for scale_back.
+template <int FAM, typename T, bool POLES = true>
 __device__ inline ProductTables<T> build_product_tables(const ProductSplit& S, int rule, const Axis* ax,
                                                         const double* glx, const double* glw, const Params<T>& p,
                                                         unsigned char* lds, int* s_exp) {
@@ -335,7 +370,7 @@ __device__ inline ProductTables<T> build_product_tables(const ProductSplit& S, i
     t.axis = reinterpret_cast<T*>(lds);
     const size_t a = ((size_t)C * total * sizeof(T) + 15) & ~(size_t)15;
     t.loop = reinterpret_cast<T*>(lds + a);
-    build_axis_factors<FAM, T>(S.d, S.n, rule, ax, glx, glw, p, S.by_n, t.axis, s_exp);
+    build_axis_factors<FAM, T, POLES>(S.d, S.n, rule, ax, glx, glw, p, S.by_n, t.axis, s_exp);
     build_table<FAM, T, true>(t.axis, total, S.n, S.L, S.q, S.nl, entries, S.by_n, t.loop);
     if (S.outer == 2) {
         t.outer = reinterpret_cast<T*>(lds + a + (((size_t)C * entries * sizeof(T) + 15) & ~(size_t)15));
