@@ -60,3 +60,47 @@ def test_one_singular_axis_is_infinite(d, n, dtype, dev):
     val = product_peak_integrals(a, torch.full_like(a, 0.5), dom.repeat(2 * d, 1, 1), n=n, rule="simpson").double()
     assert bool((val[0::2] == float("inf")).all())
     assert float((val[1::2] - ref).abs().max()) <= bar * ref
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("d", [3, 5])
+def test_double_gaussian_weights_far_from_the_centres(d, dtype, dev):
+    """The nodes that carry the integral have weights of 1e-28 (FP64: 1e-60)
+    beside ones of 1 where the peaks have decayed."""
+    x = np.array([-0.9375, 0.0, 0.0625, 0.125, 0.9375])
+    tiny = 1e-28 if dtype == torch.float32 else 1e-60
+    w = np.array([1.0, tiny, 0.5 * tiny, tiny, 0.75])
+    width, centers = (0.09375 if dtype == torch.float32 else 0.0625), (0.0, 0.125)
+    fn = tq.DoubleGaussian(d, width=width, centers=centers)
+    want = 0.5 * (width * np.sqrt(np.pi)) ** -d * sum(np.sum(w * np.exp(-(((x - c) / width) ** 2))) ** d for c in centers)
+    dom = torch.tensor([[-1.0, 1.0]] * d, dtype=dtype, device=dev)
+    # exponents of up to 100 (FP64: 230) octaves carry the rounding of the parameters
+    bar = d * (100 * 2.0**-23 if dtype == torch.float32 else 230 * 2.0**-51)
+    got = _grid64(fn, d, len(x), dom, _table(x, w, dev))
+    assert abs(got - want) <= bar * want
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_double_gaussian_peaks_on_different_axes(dtype, dev):
+    """One component is large on the first axis, the other one on the second."""
+    fn = tq.DoubleGaussian(3, width=0.125, centers=(0.25, 0.75))
+    box = [[0.2, 0.3], [0.7, 0.8], [0.4, 0.6]]
+    n = 9
+    dom = torch.tensor(box, dtype=dtype, device=dev)
+    b = dom.double().cpu().numpy()
+    want = 0.0
+    for c in fn.centers:
+        p = 1.0
+        for lo, hi in b:
+            x = np.linspace(lo, hi, n)
+            w = np.full(n, 2.0)
+            w[0] = w[-1] = 1.0
+            p *= np.sum(w * np.exp(-(((x - c) / 0.125) ** 2))) * (hi - lo) / (n - 1) / 2.0
+        want += 0.5 * (0.125 * np.sqrt(np.pi)) ** -3 * p
+    got = _grid64(fn, 3, n, dom, rule=_ops.RULES["trapezoid"])
+    assert abs(got - want) <= (4e-6 if dtype == torch.float32 else 1e-12) * want  # exponents of up to 30
+
+
+def _whole_weights(n, lo, hi, seed, dev):
+    w = np.random.default_rng(seed).integers(lo, hi + 1, n).astype(np.float64)
+    return _table(np.linspace(-1.0, 1.0, n), w, dev), float(w.sum())

@@ -210,7 +210,7 @@ template <typename T>
 __device__ __forceinline__ void product_block(const BatchDev<T>& D, const tq_batch_tile& tile, Axis* s_ax,
                                               unsigned char* s_lds, const double* glx, const double* glw,
                                               long long gl_len, double* part) {
-    __shared__ int s_exp[TQ_MAX_DIM];
+    __shared__ int s_exp[kExpSlots];
     __shared__ double s_red[kWavesPerBlock];
     const int tid = threadIdx.x;
     if (!gl_in_range(D, glx, glw, gl_len)) {
@@ -235,7 +235,7 @@ __device__ __forceinline__ void product_block(const BatchDev<T>& D, const tq_bat
 #undef TQ_BP
     }
     acc = block_sum(acc, s_red);
-    if (tid == 0) *part = scale_back(acc, D.d, s_exp);
+    if (tid == 0) *part = scale_back(D.fam, acc, D.d, s_exp);
 }
 
 // Product tiles alone (big tables; runs without classes).

@@ -44,7 +44,7 @@ template <typename T, int FAM, int K>
 __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, sizeof(T))) void k_grid_product(ProductArgs<T> A) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ Axis s_axis[TQ_MAX_DIM];
-    __shared__ int s_exp[TQ_MAX_DIM];
+    __shared__ int s_exp[kExpSlots];
     __shared__ double s_red[kProductWaves], s_scale[TQ_MAX_DIM];
     const ProductGeom& g = A.g;
     const int tid = threadIdx.x, d = g.s.d;
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, 
     if (tid == 0) {
         double scale = A.c0;
         for (int k = 0; k < d; ++k) scale *= s_scale[k];
-        const double r = scale_back(v, d, s_exp) * scale;
+        const double r = scale_back(FAM, v, d, s_exp) * scale;
         if (A.out) *A.out = (T)r;
         if (A.out64) *A.out64 = r;
     }

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_fwd(SweepUnits 
     extern __shared__ __align__(16) unsigned char s_lds[];
     __shared__ Params<T> s_p;
     __shared__ Axis s_axis[TQ_MAX_DIM];
-    __shared__ int s_exp[TQ_MAX_DIM];
+    __shared__ int s_exp[kExpSlots];
     __shared__ double s_red[kSweepBlockWaves];
     const ProductSplit& S = U.s;
     const long long b = blockIdx.y;
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_fwd(SweepUnits 
         acc += sum_items<FAM, T, K>(S, tab, own, t0, t1);
     }
     acc = block_sum(acc, s_red);
-    if (tid == 0) partials[b * gridDim.x + blockIdx.x] = scale_back(acc, S.d, s_exp);
+    if (tid == 0) partials[b * gridDim.x + blockIdx.x] = scale_back(FAM, acc, S.d, s_exp);
 }
 
 // Loop-axis sums kept beside F.
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
     extern __shared__ __align__(16) unsigned char s_lds[];
     __shared__ Params<T> s_p;
     __shared__ Axis s_axis[TQ_MAX_DIM];
-    __shared__ int s_exp[TQ_MAX_DIM];
+    __shared__ int s_exp[kExpSlots];
     __shared__ double s_red[kSweepBlockWaves];
     const ProductSplit& S = U.s;
     const int n = S.n, L = S.L, groups = S.groups, entries = groups * kGroup;

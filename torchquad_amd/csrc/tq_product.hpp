@@ -17,16 +17,22 @@
 // The factors are evaluated once per axis node in FP64 (node rounded to T,
 // parameters as T holds them), multiplied by the node's weight, brought to
 // at most 1 in magnitude per axis (an exact power of two, returned as an
-// exponent for the result) and rounded to T once.  With factors of at most 1
-// a partial product can only underflow when the point's own share of the sum
-// is below 2^-126 (2^-1022) of the largest, so the form needs no range check
-// and does not overflow where the sum of exponents did not.
+// exponent for the result) and rounded to T once.  The largest factor of an
+// axis is then in (1/4, 1]: of a family with one positive component and, each
+// component by itself, of the double Gaussian (the smaller component's share
+// goes to the first axis).  A partial product underflows only when the point
+// is below 2^(2d - 126) (FP64: 2^(2d - 1022)) of the largest, so the form
+// needs no range check and does not overflow where the sum of exponents did
+// not.  The oscillatory and the sin-sum factors are scaled by the weights
+// alone, which bound them.
 #pragma once
 #include "tq_grid_tile.hpp"
 
 namespace tq {
 
 constexpr bool family_exponential(int fam) { return fam == TQ_FAM_GAUSSIAN_PEAK || fam == TQ_FAM_EXP_LINEAR; }
+// Exponents that a family's factors have by themselves: one, the double Gaussian one per component.
+constexpr int family_exponents(int fam) { return family_exponential(fam) ? 1 : (fam == TQ_FAM_DOUBLE_GAUSSIAN ? 2 : 0); }
 constexpr int family_comps(int fam) {
     return (fam == TQ_FAM_OSCILLATORY || fam == TQ_FAM_SIN_SUM || fam == TQ_FAM_DOUBLE_GAUSSIAN) ? 2 : 1;
 }
@@ -63,7 +69,17 @@ __device__ inline double peak_denominator(int k, T x, const Params<T>& p) {
 constexpr int kPoleExp = 1 << 27;  // above every other exponent
 __device__ inline bool is_pole(double denominator) { return fabs(denominator) < 0x1.0p-1022; }
 
-// Weighted factor of a family that is not exponential.
+// log2 of the double Gaussian's factors, kept in range as factor_exponent's.
+template <typename T>
+__device__ inline void gauss_exponents(T x, const Params<T>& p, double* ex) {
+    const double t1 = (double)x - (double)p.c1, t2 = (double)x - (double)p.c2, c = -(double)p.c3;
+    ex[0] = c * t1 * t1;
+    ex[1] = c * t2 * t2;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ex[i] = ex[i] > 1e8 ? 1e8 : (ex[i] < -1e8 ? -1e8 : ex[i]);
+}
+
+// Weighted factor of a family without exponents.
 template <int FAM, typename T>
 __device__ inline void factor_comps(int k, T x, double w, const Params<T>& p, double* v) {
     if constexpr (FAM == TQ_FAM_PRODUCT_PEAK) {
@@ -79,10 +95,6 @@ __device__ inline void factor_comps(int k, T x, double w, const Params<T>& p, do
     } else if constexpr (FAM == TQ_FAM_SIN_SUM) {
         v[0] = w;
         v[1] = w * sin(fma((double)p.a[k], (double)x, (double)p.u[k]));
-    } else if constexpr (FAM == TQ_FAM_DOUBLE_GAUSSIAN) {
-        const double t1 = (double)x - (double)p.c1, t2 = (double)x - (double)p.c2, c = -(double)p.c3;
-        v[0] = w * exp2(c * t1 * t1);
-        v[1] = w * exp2(c * t2 * t2);
     } else {
         v[0] = w;
     }
@@ -142,7 +154,7 @@ template <int FAM, typename T, bool POLES>
 __device__ inline int factor_scale(int k, T x, double w, double ex, const Params<T>& p) {
     const int m = mag_exp(w);
     if (m == -0x7fffffff) return m;
-    if constexpr (family_exponential(FAM)) {
+    if constexpr (family_exponents(FAM) > 0) {
         return ex == ex ? m + (int)ceil(ex) : -0x7fffffff;
     } else if constexpr (FAM == TQ_FAM_PRODUCT_PEAK) {
         const double den = peak_denominator(k, x, p);
@@ -154,15 +166,25 @@ __device__ inline int factor_scale(int k, T x, double w, double ex, const Params
     }
 }
 
+// Powers of two taken out of the axes: s_exp[k] of axis k, of the double
+// Gaussian's second component s_exp[TQ_MAX_DIM + k].
+constexpr int kExpSlots = 2 * TQ_MAX_DIM;
+__device__ inline long long sum_exponents(int d, const int* s_exp) {
+    long long e = 0;
+    for (int k = 0; k < d; ++k) e += exp_or_zero(s_exp[k]);
+    return e;
+}
+
 // A block's sum v with the powers of two put back that were taken out of its
 // axes.  A pole on every axis: NaN, as from a sum over 0 times infinity.
-__device__ inline double scale_back(double v, int d, const int* s_exp) {
-    long long e = 0;
-    int poles = 0;
-    for (int k = 0; k < d; ++k) {
-        e += exp_or_zero(s_exp[k]);
-        poles += s_exp[k] >= kPoleExp ? 1 : 0;
+__device__ inline double scale_back(int fam, double v, int d, const int* s_exp) {
+    long long e = sum_exponents(d, s_exp);
+    if (fam == TQ_FAM_DOUBLE_GAUSSIAN) {
+        const long long e2 = sum_exponents(d, s_exp + TQ_MAX_DIM);
+        if (e2 > e) e = e2;
     }
+    int poles = 0;
+    for (int k = 0; k < d; ++k) poles += s_exp[k] >= kPoleExp ? 1 : 0;
     if (poles == d) return __longlong_as_double(0x7ff8000000000000ll);
     return ldexp(v, (int)(e > (1 << 30) ? (1 << 30) : (e < -(1 << 30) ? -(1 << 30) : e)));
 }
@@ -179,13 +201,13 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
                                           const double* glw, const Params<T>& p, FastDiv by_n, T* axis, int* s_exp) {
     constexpr int C = family_comps(FAM);
     const int tid = threadIdx.x, nt = blockDim.x, total = d * n;
-    constexpr bool EXP = family_exponential(FAM);
-    if (tid < d) s_exp[tid] = -0x7fffffff;
+    constexpr int E = family_exponents(FAM);
+    if (tid < kExpSlots) s_exp[tid] = -0x7fffffff;
     __syncthreads();
     struct Node {
         int k;
         T x;
-        double w, ex;
+        double w, ex[2];
     };
     auto node = [&](int e) {
         Node v;
@@ -193,16 +215,27 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
         const int j = e - v.k * n;
         v.x = (T)node_of(ax[v.k], j, n, rule, glx);
         v.w = weight_of(rule, j, n, glw);
-        v.ex = 0.0;
-        if constexpr (EXP) v.ex = factor_exponent<FAM, T>(v.k, v.x, p);
+        v.ex[0] = v.ex[1] = 0.0;
+        if constexpr (E == 1) v.ex[0] = factor_exponent<FAM, T>(v.k, v.x, p);
+        if constexpr (E == 2) gauss_exponents<T>(v.x, p, v.ex);
         return v;
     };
-    auto scale = [&](const Node& v) { atomicMax(&s_exp[v.k], factor_scale<FAM, T, POLES>(v.k, v.x, v.w, v.ex, p)); };
+    auto scale = [&](const Node& v) {
+        atomicMax(&s_exp[v.k], factor_scale<FAM, T, POLES>(v.k, v.x, v.w, v.ex[0], p));
+        if constexpr (E == 2)
+            atomicMax(&s_exp[TQ_MAX_DIM + v.k], factor_scale<FAM, T, POLES>(v.k, v.x, v.w, v.ex[1], p));
+    };
     auto store = [&](const Node& nd, int e) {
         const int m = exp_or_zero(s_exp[nd.k]);
         double v[C];
-        if constexpr (EXP) {
-            v[0] = nd.w * exp2(nd.ex - (double)m);
+        if constexpr (E == 1) {
+            v[0] = nd.w * exp2(nd.ex[0] - (double)m);
+        } else if constexpr (E == 2) {
+            const int m2 = exp_or_zero(s_exp[TQ_MAX_DIM + nd.k]);
+            // the first axis brings the components to the larger one's power of two
+            const double behind = nd.k == 0 ? (double)(sum_exponents(d, s_exp) - sum_exponents(d, s_exp + TQ_MAX_DIM)) : 0.0;
+            v[0] = nd.w * exp2(nd.ex[0] - (double)m + fmin(behind, 0.0));
+            v[1] = nd.w * exp2(nd.ex[1] - (double)m2 - fmax(behind, 0.0));
         } else {
             factor_comps<FAM, T>(nd.k, nd.x, nd.w, p, v);
             if (FAM == TQ_FAM_PRODUCT_PEAK && POLES && m >= kPoleExp) {
