@@ -104,3 +104,32 @@ def test_double_gaussian_peaks_on_different_axes(dtype, dev):
 def _whole_weights(n, lo, hi, seed, dev):
     w = np.random.default_rng(seed).integers(lo, hi + 1, n).astype(np.float64)
     return _table(np.linspace(-1.0, 1.0, n), w, dev), float(w.sum())
+
+
+def test_partial_sums_join_in_64_bits(dev):
+    """Sums of whole numbers: an FP32 partial of up to 128 values stays below
+    2^24, so it is exact, while two or more together are not; every join has
+    to be in FP64 for the result to be exact."""
+    # grid, eight states per lane (1.8e8 points), loops of 2025
+    gl, s = _whole_weights(45, 9, 10, 0, dev)
+    dom = torch.tensor([[-1.0, 1.0]] * 5, dtype=torch.float32, device=dev)
+    assert _grid64(tq.Constant(5), 5, 45, dom, gl) == s**5
+    # batch, four states per lane
+    gl, s = _whole_weights(20, 9, 10, 1, dev)
+    b = Batch([{"rule": "gauss_legendre", "fn": tq.Constant(5), "dim": 5, "n": 20, "domain": [[-1.0, 1.0]] * 5}],
+              dtype=torch.float32, device=dev)
+    out64 = torch.zeros(1, dtype=torch.float64, device=dev)
+    _lib.call("tq_batch_run", b.dt, _lib.ptr(b.desc), 1, _lib.ptr(b.tiles), b.n_tiles, _lib.ptr(b.tile_begin),
+              _lib.ptr(b.tile_count), _lib.ptr(gl[0]), _lib.ptr(gl[1]), None, 20, _lib.ptr(b.tile_part), None,
+              _lib.ptr(out64), None, _lib.stream_ptr(dev))
+    assert float(out64) == s**5
+    # sweep forward, eight states per lane; a = 0 makes the integrand 1
+    gl, s = _whole_weights(16, 9, 10, 2, dev)
+    g = _ops.grid_desc(GL, 5, 16, torch.float32, gl)
+    zero = torch.zeros(3, 5, device=dev)
+    doms = dom.repeat(3, 1, 1).contiguous()
+    ws = torch.empty(_lib.lib().tq_sweep_workspace_size(ctypes.byref(g), 3), dtype=torch.uint8, device=dev)
+    out, out64 = torch.zeros(3, device=dev), torch.zeros(3, dtype=torch.float64, device=dev)
+    _lib.call("tq_sweep_forward", ctypes.byref(g), _lib.FAM_GAUSSIAN_PEAK, 3, _lib.ptr(zero), _lib.ptr(zero),
+              _lib.ptr(doms), _lib.ptr(ws), ws.numel(), _lib.ptr(out), _lib.ptr(out64), _lib.stream_ptr(dev))
+    assert out64.tolist() == [s**5] * 3

@@ -207,45 +207,45 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
             F rf = F::one(true);
             for (int k = 0; k < L; ++k)
                 rf = F::merge(rf, axis_factor<FAM, T>(tab.axis, D * n, k * n + __builtin_amdgcn_readlane(dig, k)));
-            T s[K], all = T(0);
+            T s[K];
 #pragma unroll
-            for (int k = 0; k < K; ++k) {
-                s[k] = own[k].v[0] * rf.v[0];
-                all += s[k];
-            }
+            for (int k = 0; k < K; ++k) s[k] = own[k].v[0] * rf.v[0];
+            const T all = (T)join_states<T, K>(s);
             const int left = groups - gi;
             const int ge = t1 - at < left ? gi + (int)(t1 - at) : groups;
             double Frow = 0.0;
             constexpr int kFlushGroups = kFlush / kGroup;
             for (int gb = gi; gb < ge; gb += kFlushGroups) {
                 const int gend = gb + kFlushGroups < ge ? gb + kFlushGroups : ge;
-                T fa[K], fm[NM];
+                T fa[K];
 #pragma unroll
                 for (int k = 0; k < K; ++k) fa[k] = T(0);
+                // the moments' FP32 partials stand for K points per entry
+                constexpr int kMomentGroups = sizeof(T) == 4 ? kFlushGroups / K : kFlushGroups;
+                for (int gm = gb; gm < gend; gm += kMomentGroups) {
+                    const int gmend = gm + kMomentGroups < gend ? gm + kMomentGroups : gend;
+                    T fm[NM];
 #pragma unroll
-                for (int i = 0; i < NM; ++i) fm[i] = T(0);
-                for (int gq = gb; gq < gend; ++gq) {
-                    EntryGroup<TQ_FAM_CONSTANT, T> e, em[NM];
-                    e.load(tab.loop, entries, gq);
+                    for (int i = 0; i < NM; ++i) fm[i] = T(0);
+                    for (int gq = gm; gq < gmend; ++gq) {
+                        EntryGroup<TQ_FAM_CONSTANT, T> e, em[NM];
+                        e.load(tab.loop, entries, gq);
 #pragma unroll
-                    for (int i = 0; i < NM; ++i) em[i].load(mom + i * entries, entries, gq);
+                        for (int i = 0; i < NM; ++i) em[i].load(mom + i * entries, entries, gq);
 #pragma unroll
-                    for (int x = 0; x < kGroup; ++x) {
+                        for (int x = 0; x < kGroup; ++x) {
 #pragma unroll
-                        for (int k = 0; k < K; ++k) fa[k] = fma(s[k], e.v[0][x], fa[k]);
+                            for (int k = 0; k < K; ++k) fa[k] = fma(s[k], e.v[0][x], fa[k]);
 #pragma unroll
-                        for (int i = 0; i < NM; ++i) fm[i] = fma(all, em[i].v[0][x], fm[i]);
+                            for (int i = 0; i < NM; ++i) fm[i] = fma(all, em[i].v[0][x], fm[i]);
+                        }
                     }
+#pragma unroll
+                    for (int i = 0; i < NM; ++i) M[i] += (double)fm[i];
                 }
 #pragma unroll
                 for (int k = 0; k < K; ++k) Fk[k] += (double)fa[k];
-#pragma unroll
-                for (int i = 0; i < NM; ++i) M[i] += (double)fm[i];
-#pragma unroll
-                for (int v = K / 2; v > 0; v >>= 1)
-#pragma unroll
-                    for (int k = 0; k < v; ++k) fa[k] += fa[k + v];
-                Frow += (double)fa[0];
+                Frow += join_states<T, K>(fa);
             }
             accF += Frow;
             // row axes: uniform nodes

@@ -288,6 +288,20 @@ struct EntryGroup {
     }
 };
 
+// The states' partial sums, joined in FP64 (joined in FP32, one rounding there
+// would stand for 128 K points).
+template <typename T, int K>
+__device__ inline double join_states(const T* fa) {
+    double r[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) r[k] = (double)fa[k];
+#pragma unroll
+    for (int w = K / 2; w > 0; w >>= 1)
+#pragma unroll
+        for (int k = 0; k < w; ++k) r[k] += r[k + w];
+    return r[0];
+}
+
 // Sum over the entries of groups [g0, g1) and the K states of a lane of
 // their values, FP32 partials of at most 128 entries per state added to FP64.
 // K states share each entry that is read from LDS: with one state the four
@@ -314,11 +328,7 @@ __device__ inline double sum_entries(const Factor<FAM, T>* s, const T* tab, int 
 #pragma unroll
                     for (int c = 0; c < C; ++c) fa[k] = fma(s[k].v[c], e.v[c][i], fa[k]);
         }
-#pragma unroll
-        for (int w = K / 2; w > 0; w >>= 1)
-#pragma unroll
-            for (int k = 0; k < w; ++k) fa[k] += fa[k + w];
-        acc += (double)fa[0];
+        acc += join_states<T, K>(fa);
     }
     return acc;
 }
