@@ -133,3 +133,33 @@ def test_partial_sums_join_in_64_bits(dev):
     _lib.call("tq_sweep_forward", ctypes.byref(g), _lib.FAM_GAUSSIAN_PEAK, 3, _lib.ptr(zero), _lib.ptr(zero),
               _lib.ptr(doms), _lib.ptr(ws), ws.numel(), _lib.ptr(out), _lib.ptr(out64), _lib.stream_ptr(dev))
     assert out64.tolist() == [s**5] * 3
+
+
+@pytest.mark.parametrize("rule", ["trapezoid", "simpson", "gauss_legendre"])
+@pytest.mark.parametrize("d,n", [(3, 21), (3, 65), (3, 201), (4, 13), (4, 45), (5, 9), (5, 33), (6, 9), (7, 9)])
+def test_sin_sum_rounding_errors_average_out(d, n, rule, dev):
+    """FP32 sums of sines whose rounding errors are independent stay within
+    half a unit in the last place of sum |w f|; additions that repeat one
+    rounding for many points do not."""
+    from torchquad_amd.gl_nodes import gauss_legendre
+
+    n = min(n, 200) if rule == "gauss_legendre" else n
+    gl = gauss_legendre(n, device=dev) if rule == "gauss_legendre" else None
+    for seed, (lo, hi) in enumerate([(-1.0, 1.0), (0.0, 1.0), (-0.75, 1.5), (-0.5, 0.25)]):
+        rng = np.random.default_rng([seed, n])
+        a = rng.uniform(0.5, 1.5, d).astype(np.float32).astype(np.float64)
+        u = rng.uniform(0.8, 1.0, d).astype(np.float32).astype(np.float64)
+        dom = torch.tensor([[lo, hi]] * d, dtype=torch.float32, device=dev)
+        if gl is not None:
+            x = 0.5 * (hi - lo) * gl[0].cpu().numpy() + 0.5 * (hi + lo)
+            w = 0.5 * (hi - lo) * gl[1].cpu().numpy()
+        else:
+            x, w = np.linspace(lo, hi, n), np.full(n, 2.0)
+            if rule == "simpson":
+                w[1::2] = 4.0
+            w[0] = w[-1] = 1.0
+            w *= (hi - lo) / (n - 1) / (3.0 if rule == "simpson" else 2.0)
+        W = w.sum()
+        ref = sum(np.sum(w * np.sin(a[k] * x + u[k])) for k in range(d)) * W ** (d - 1)
+        got = _grid64(tq.SinSum(d, a, u), d, n, dom, gl, rule=_ops.RULES[rule])
+        assert abs(got - ref) <= 2.0**-24 * d * W**d, (seed, got, ref)

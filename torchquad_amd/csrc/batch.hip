@@ -196,12 +196,14 @@ __device__ __forceinline__ double batch_product_tile(const BatchDev<T>& D, const
     const long long per = (items + parts - 1) / parts;
     double acc = 0.0;
     Factor<FAM, T> own[kBatchStates];
+    double wl[kBatchStates];
     for (int u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < lane_groups * parts; u += kWavesPerBlock) {
         const int lg = u / parts, part = u - lg * parts;
         const long long t0 = tile.t0 + part * per, t1 = t0 + per < tile.t1 ? t0 + per : tile.t1;
         if (t0 >= t1) continue;
-        lane_states<FAM, T, kBatchStates>(S, tab, (tile.lane_wave + lg) * kWave + (int)(threadIdx.x & (kWave - 1)), own);
-        acc += sum_items<FAM, T, kBatchStates>(S, tab, own, t0, t1);
+        lane_states<FAM, T, kBatchStates>(S, tab, (tile.lane_wave + lg) * kWave + (int)(threadIdx.x & (kWave - 1)), own,
+                                          wl);
+        acc += sum_items<FAM, T, kBatchStates>(S, tab, own, wl, t0, t1);
     }
     return acc;
 }

@@ -65,8 +65,9 @@ __global__ __launch_bounds__(kProductWaves * kWave, product_waves_per_simd(FAM, 
         const long long t0 = (long long)chunk * g.ipw;
         const long long t1 = t0 + g.ipw < g.s.items ? t0 + g.ipw : g.s.items;
         Factor<FAM, T> own[K];
-        lane_states<FAM, T, K>(g.s, tab, lg * kWave + (tid & (kWave - 1)), own);
-        acc = sum_items<FAM, T, K>(g.s, tab, own, t0, t1);
+        double wl[K];
+        lane_states<FAM, T, K>(g.s, tab, lg * kWave + (tid & (kWave - 1)), own, wl);
+        acc = sum_items<FAM, T, K>(g.s, tab, own, wl, t0, t1);
     }
     double v;
     if (!sum_over_blocks(acc, A.sums, s_red, &v)) return;

@@ -91,11 +91,12 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_fwd(SweepUnits 
     const int units = S.lane_groups * U.parts, waves = gridDim.x * kSweepBlockWaves;
     double acc = 0.0;
     Factor<FAM, T> own[K];
+    double wl[K];
     for (int w = blockIdx.x * kSweepBlockWaves + __builtin_amdgcn_readfirstlane(tid >> 6); w < units; w += waves) {
         const int lg = w / U.parts, part = w - lg * U.parts;
         const long long t0 = part * U.per, t1 = t0 + U.per < S.items ? t0 + U.per : S.items;
-        lane_states<FAM, T, K>(S, tab, lg * kWave + (tid & (kWave - 1)), own);
-        acc += sum_items<FAM, T, K>(S, tab, own, t0, t1);
+        lane_states<FAM, T, K>(S, tab, lg * kWave + (tid & (kWave - 1)), own, wl);
+        acc += sum_items<FAM, T, K>(S, tab, own, wl, t0, t1);
     }
     acc = block_sum(acc, s_red);
     if (tid == 0) partials[b * gridDim.x + blockIdx.x] = scale_back(FAM, acc, S.d, s_exp);
@@ -190,7 +191,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
         const long long t0 = part * U.per, t1 = t0 + U.per < S.items ? t0 + U.per : S.items;
         const int slot = lg * kWave + lane;
         F own[K];
-        lane_states<FAM, T, K>(S, tab, slot, own);
+        lane_states<FAM, T, K>(S, tab, slot, own, nullptr);
         double Fk[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) Fk[k] = 0.0;

@@ -6,7 +6,7 @@
 //   exp-linear        prod 2^(a_k x_k)                    1
 //   product peak      prod 1 / (a_k^-2 + (x_k - u_k)^2)   1
 //   oscillatory       Re prod e^(i a_k x_k)               2 (complex product)
-//   sin-sum           eps part of prod (1 + eps s_k)      2 (dual numbers)
+//   sin-sum           sum s_k                             2 (weight, sum)
 //   double Gaussian   sum of two products                 2
 //   constant          1                                   1
 // so a point costs one multiply-add per component from tables instead of a
@@ -36,6 +36,16 @@ constexpr int family_exponents(int fam) { return family_exponential(fam) ? 1 : (
 constexpr int family_comps(int fam) {
     return (fam == TQ_FAM_OSCILLATORY || fam == TQ_FAM_SIN_SUM || fam == TQ_FAM_DOUBLE_GAUSSIAN) ? 2 : 1;
 }
+
+// The sin-sum keeps the weights of row and lane axes out of its factors, in
+// FP64, as the point-by-point kernel does; only the loop table carries its
+// weights in T.  Rounded into FP32 factors, the weights of a Gauss-Legendre
+// rule are off alike on every axis (error / sum |w f|, rms over d = 3..7:
+// 3.3e-8 so, 0.7e-8 apart, 0.9e-8 point by point).  The other families'
+// rounding errors differ from axis to axis and stay where the point-by-point
+// kernel's are, and most need the weights inside for their range: weights may
+// fall as fast as the factors rise.
+constexpr bool weights_apart(int fam) { return fam == TQ_FAM_SIN_SUM; }
 
 // log2 of an exponential family's factor; the constant term goes to axis 0.
 // Kept within +-1e8, far outside any result, so that the exponents of 16 axes
@@ -93,8 +103,8 @@ __device__ inline void factor_comps(int k, T x, double w, const Params<T>& p, do
         v[0] = w * c;
         v[1] = w * s;
     } else if constexpr (FAM == TQ_FAM_SIN_SUM) {
-        v[0] = w;
-        v[1] = w * sin(fma((double)p.a[k], (double)x, (double)p.u[k]));
+        v[0] = 1.0;
+        v[1] = sin(fma((double)p.a[k], (double)x, (double)p.u[k]));
     } else {
         v[0] = w;
     }
@@ -119,22 +129,20 @@ struct Factor {
             r.v[0] = fma(a.v[0], b.v[0], -(a.v[1] * b.v[1]));
             r.v[1] = fma(a.v[0], b.v[1], a.v[1] * b.v[0]);
         } else if constexpr (FAM == TQ_FAM_SIN_SUM) {
-            r.v[0] = a.v[0] * b.v[0];
-            r.v[1] = fma(a.v[0], b.v[1], a.v[1] * b.v[0]);
+            r.v[0] = T(1);
+            r.v[1] = a.v[1] + b.v[1];
         } else {
 #pragma unroll
             for (int c = 0; c < C; ++c) r.v[c] = a.v[c] * b.v[c];
         }
         return r;
     }
-    // the form in which an entry meets a state: value(merge(a, b)) = sum_c a.v[c] * b.dual().v[c]
-    __device__ inline Factor dual() const {
+    // the form in which an entry (of weight w, where that is kept apart) meets a state: value(merge(a, b)) =
+    // sum_c a.v[c] * b.entry(w).v[c]; sin-sum: b.entry(w).v[0] * (a.v[1] + b.entry(w).v[1])
+    __device__ inline Factor entry(double w) const {
         Factor r = *this;
         if constexpr (FAM == TQ_FAM_OSCILLATORY) r.v[1] = -v[1];
-        if constexpr (FAM == TQ_FAM_SIN_SUM) {
-            r.v[0] = v[1];
-            r.v[1] = v[0];
-        }
+        if constexpr (FAM == TQ_FAM_SIN_SUM) r.v[0] = (T)w;
         return r;
     }
 };
@@ -189,6 +197,13 @@ __device__ inline double scale_back(int fam, double v, int d, const int* s_exp) 
     return ldexp(v, (int)(e > (1 << 30) ? (1 << 30) : (e < -(1 << 30) ? -(1 << 30) : e)));
 }
 
+// An axis's weights where they are kept apart, in the place of the component
+// that is not stored (n FP64 numbers; d >= 2 axes of n numbers of T).
+template <typename T>
+__device__ inline double* apart_weights(const T* axis) {
+    return const_cast<double*>(reinterpret_cast<const double*>(axis));
+}
+
 // Axis tables of a whole block: component c of axis k's node j goes to
 // axis[c * d * n + k * n + j], the power of two taken out of axis k to
 // s_exp[k].  The d n nodes are spread over the block's threads; the scales
@@ -214,7 +229,7 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
         v.k = (int)by_n.div((uint32_t)e);
         const int j = e - v.k * n;
         v.x = (T)node_of(ax[v.k], j, n, rule, glx);
-        v.w = weight_of(rule, j, n, glw);
+        v.w = weights_apart(FAM) ? 1.0 : weight_of(rule, j, n, glw);
         v.ex[0] = v.ex[1] = 0.0;
         if constexpr (E == 1) v.ex[0] = factor_exponent<FAM, T>(v.k, v.x, p);
         if constexpr (E == 2) gauss_exponents<T>(v.x, p, v.ex);
@@ -247,23 +262,27 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
             }
         }
 #pragma unroll
-        for (int c = 0; c < C; ++c) axis[c * total + e] = (T)v[c];
+        for (int c = FAM == TQ_FAM_SIN_SUM ? 1 : 0; c < C; ++c) axis[c * total + e] = (T)v[c];
     };
     // the thread's first node is kept over the barrier, later ones are formed again
     Node first = node(tid < total ? tid : total - 1);
-    if (tid < total) scale(first);
-    for (int e = tid + nt; e < total; e += nt) scale(node(e));
-    __syncthreads();
+    if constexpr (!weights_apart(FAM)) {
+        if (tid < total) scale(first);
+        for (int e = tid + nt; e < total; e += nt) scale(node(e));
+        __syncthreads();
+    }
     if (tid < total) store(first, tid);
     for (int e = tid + nt; e < total; e += nt) store(node(e), e);
+    if constexpr (weights_apart(FAM))
+        for (int j = tid; j < n; j += nt) apart_weights(axis)[j] = weight_of(rule, j, n, glw);
     __syncthreads();
 }
 
 template <int FAM, typename T>
 __device__ inline Factor<FAM, T> axis_factor(const T* axis, int total, int e) {
-    Factor<FAM, T> f;
+    Factor<FAM, T> f = Factor<FAM, T>::one(true);
 #pragma unroll
-    for (int c = 0; c < Factor<FAM, T>::C; ++c) f.v[c] = axis[c * total + e];
+    for (int c = FAM == TQ_FAM_SIN_SUM ? 1 : 0; c < Factor<FAM, T>::C; ++c) f.v[c] = axis[c * total + e];
     return f;
 }
 
@@ -290,11 +309,12 @@ struct EntryGroup {
 
 // The states' partial sums, joined in FP64 (joined in FP32, one rounding there
 // would stand for 128 K points).
+// w: the states' weights, where they are kept apart.
 template <typename T, int K>
-__device__ inline double join_states(const T* fa) {
+__device__ inline double join_states(const T* fa, const double* w = nullptr) {
     double r[K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) r[k] = (double)fa[k];
+    for (int k = 0; k < K; ++k) r[k] = w ? w[k] * (double)fa[k] : (double)fa[k];
 #pragma unroll
     for (int w = K / 2; w > 0; w >>= 1)
 #pragma unroll
@@ -307,8 +327,13 @@ __device__ inline double join_states(const T* fa) {
 // K states share each entry that is read from LDS: with one state the four
 // SIMDs' reads of a 4-byte entry take 8 cycles of the CU's LDS against 2.7
 // cycles of multiply-add, with four they take less than the arithmetic.
+// Sin-sum: a value is formed before it is added.  As a sum of two products,
+// weight and sine each multiplied through, one component is the same power of
+// two on most entries and repeats one rounding along the loop, so the errors
+// do not average out (FP32 Newton-Cotes rules, as above: 4e-8 so, 0.6e-8 here).
 template <int FAM, typename T, int K>
-__device__ inline double sum_entries(const Factor<FAM, T>* s, const T* tab, int entries, int g0, int g1) {
+__device__ inline double sum_entries(const Factor<FAM, T>* s, const double* wl, const T* tab, int entries, int g0,
+                                     int g1) {
     constexpr int C = Factor<FAM, T>::C;
     constexpr int kFlushGroups = kFlush / kGroup;
     double acc = 0.0;
@@ -324,20 +349,29 @@ __device__ inline double sum_entries(const Factor<FAM, T>* s, const T* tab, int 
 #pragma unroll
             for (int i = 0; i < kGroup; ++i)
 #pragma unroll
-                for (int k = 0; k < K; ++k)
+                for (int k = 0; k < K; ++k) {
+                    if constexpr (FAM == TQ_FAM_SIN_SUM) {
+                        fa[k] = fma(e.v[0][i], s[k].v[1] + e.v[1][i], fa[k]);
+                    } else {
 #pragma unroll
-                    for (int c = 0; c < C; ++c) fa[k] = fma(s[k].v[c], e.v[c][i], fa[k]);
+                        for (int c = 0; c < C; ++c) fa[k] = fma(s[k].v[c], e.v[c][i], fa[k]);
+                    }
+                }
         }
-        acc += join_states<T, K>(fa);
+        if constexpr (weights_apart(FAM)) {
+            acc += join_states<T, K>(fa, wl);
+        } else {
+            acc += join_states<T, K>(fa);
+        }
     }
     return acc;
 }
 
 // Table of the combined factors of axes A .. A + q - 1 (q = 2: entry
-// j1 n + j2), `count` of them, zeros from there to `entries`; DUAL: in the
-// form that meets a state.  Four entries per thread and trip: their reads go
+// j1 n + j2), `count` of them, zeros from there to `entries`; LOOP: in the
+// form that meets a state (Factor::entry).  Four entries per thread and trip: their reads go
 // out together.  The caller's next barrier publishes it.
-template <int FAM, typename T, bool DUAL>
+template <int FAM, typename T, bool LOOP>
 __device__ inline void build_table(const T* axis, int total, int n, int A, int q, int count, int entries, FastDiv by_n,
                                    T* tab) {
     using F = Factor<FAM, T>;
@@ -349,14 +383,17 @@ __device__ inline void build_table(const T* axis, int total, int n, int A, int q
             const int e = e0 + i * nt;
             f[i] = F::one(false);
             if (e < count) {
+                double w = 1.0;
                 if (q == 2) {
                     const int j1 = (int)by_n.div((uint32_t)e);
+                    if (LOOP && weights_apart(FAM)) w = apart_weights(axis)[j1] * apart_weights(axis)[e - j1 * n];
                     f[i] = F::merge(axis_factor<FAM, T>(axis, total, A * n + j1),
                                     axis_factor<FAM, T>(axis, total, (A + 1) * n + e - j1 * n));
                 } else {
+                    if (LOOP && weights_apart(FAM)) w = apart_weights(axis)[e];
                     f[i] = axis_factor<FAM, T>(axis, total, A * n + e);
                 }
-                if (DUAL) f[i] = f[i].dual();
+                if (LOOP) f[i] = f[i].entry(w);
             }
         }
 #pragma unroll
@@ -427,16 +464,21 @@ __device__ inline ProductTables<T> build_product_tables(const ProductSplit& S, i
     return t;
 }
 
-// The K states of lane slot `slot`; zeros where there is no combination.
+// The K states of lane slot `slot`, and their weights where they are kept
+// apart; zeros where there is no combination.
 template <int FAM, typename T, int K>
-__device__ inline void lane_states(const ProductSplit& S, const ProductTables<T>& t, int slot, Factor<FAM, T>* own) {
+__device__ inline void lane_states(const ProductSplit& S, const ProductTables<T>& t, int slot, Factor<FAM, T>* own,
+                                   double* wl) {
     using F = Factor<FAM, T>;
     const bool on = slot < S.slots;
     uint32_t r = on ? (uint32_t)slot : 0u;
     F common = F::one(true);
+    double w = 1.0;
     for (int a = S.d - 1; a >= S.d - S.inner; --a) {
         const uint32_t q = S.by_n.div(r);
-        common = F::merge(common, axis_factor<FAM, T>(t.axis, S.d * S.n, a * S.n + (int)(r - q * S.by_n.n)));
+        const int j = (int)(r - q * S.by_n.n);
+        common = F::merge(common, axis_factor<FAM, T>(t.axis, S.d * S.n, a * S.n + j));
+        if constexpr (weights_apart(FAM)) w *= apart_weights(t.axis)[j];
         r = q;
     }
 #pragma unroll
@@ -447,6 +489,12 @@ __device__ inline void lane_states(const ProductSplit& S, const ProductTables<T>
         o = F::merge(common, o);
 #pragma unroll
         for (int c = 0; c < F::C; ++c) own[k].v[c] = has ? o.v[c] : T(0);
+        if constexpr (weights_apart(FAM)) {
+            const int j1 = S.outer == 2 ? (int)S.by_n.div((uint32_t)(has ? f : 0)) : (has ? f : 0);
+            double wo = apart_weights(t.axis)[j1];
+            if (S.outer == 2) wo *= apart_weights(t.axis)[(has ? f : 0) - j1 * S.n];
+            wl[k] = has ? w * wo : 0.0;
+        }
     }
 }
 
@@ -455,10 +503,10 @@ __device__ inline void lane_states(const ProductSplit& S, const ProductTables<T>
 // the axes [0, L)) is merged into the states.
 template <int FAM, typename T, int K>
 __device__ inline double sum_items(const ProductSplit& S, const ProductTables<T>& t, const Factor<FAM, T>* own,
-                                   long long t0, long long t1) {
+                                   const double* wl, long long t0, long long t1) {
     using F = Factor<FAM, T>;
     const int lane = threadIdx.x & (kWave - 1), n = S.n, L = S.L, groups = S.groups, entries = groups * kGroup;
-    if (L == 0) return sum_entries<FAM, T, K>(own, t.loop, entries, (int)t0, (int)t1);
+    if (L == 0) return sum_entries<FAM, T, K>(own, wl, t.loop, entries, (int)t0, (int)t1);
     // row odometer: lane k of `dig` holds the digit of row axis k
     long long row = t0 / groups;
     int gi = (int)(t0 - row * groups);
@@ -471,14 +519,20 @@ __device__ inline double sum_items(const ProductSplit& S, const ProductTables<T>
     double acc = 0.0;
     for (long long at = t0; at < t1;) {
         F rf = F::one(true);
-        for (int k = 0; k < L; ++k)
-            rf = F::merge(rf, axis_factor<FAM, T>(t.axis, S.d * n, k * n + __builtin_amdgcn_readlane(dig, k)));
+        double rw = 1.0;
+        for (int k = 0; k < L; ++k) {
+            const int j = __builtin_amdgcn_readlane(dig, k);
+            rf = F::merge(rf, axis_factor<FAM, T>(t.axis, S.d * n, k * n + j));
+            if constexpr (weights_apart(FAM)) rw *= apart_weights(t.axis)[j];
+        }
         F s[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) s[k] = F::merge(own[k], rf);
         const int left = groups - gi;
         const int ge = t1 - at < left ? gi + (int)(t1 - at) : groups;
-        acc += sum_entries<FAM, T, K>(s, t.loop, entries, gi, ge);
+        const double part = sum_entries<FAM, T, K>(s, wl, t.loop, entries, gi, ge);
+        if constexpr (weights_apart(FAM)) acc = fma(rw, part, acc);
+        else acc += part;
         at += ge - gi;
         gi = 0;
         for (int k = L - 1; k >= 0; --k) {
