@@ -163,3 +163,18 @@ def test_sin_sum_rounding_errors_average_out(d, n, rule, dev):
         ref = sum(np.sum(w * np.sin(a[k] * x + u[k])) for k in range(d)) * W ** (d - 1)
         got = _grid64(tq.SinSum(d, a, u), d, n, dom, gl, rule=_ops.RULES[rule])
         assert abs(got - ref) <= 2.0**-24 * d * W**d, (seed, got, ref)
+
+
+@pytest.mark.parametrize("rule,c", [("simpson", 3.0), ("boole", 22.5), ("trapezoid", 2.0)])
+@pytest.mark.parametrize("d", [3, 6, 8])
+def test_rule_scale_is_a_division(d, rule, c, dev):
+    """FP64: the scale of an axis is its spacing divided by the rule's
+    constant, to the last bit."""
+    sums = {"simpson": 12.0, "boole": 90.0, "trapezoid": 8.0}[rule]
+    for h in (5.0, 0.7, 1.1, 3.3):
+        dom = torch.tensor([[0.0, 4.0 * h]] * d, dtype=torch.float64, device=dev)
+        width = float(dom[0, 1])
+        scale = 1.0
+        for _ in range(d):
+            scale *= width / 4.0 / c
+        assert _grid64(tq.Constant(d), d, 5, dom, rule=_ops.RULES[rule]) == sums**d * scale

@@ -73,13 +73,14 @@ __device__ __host__ inline double axis_scale(double a, double b, int n, int rule
     }
 }
 
-// axis_scale from an axis's map: the spacing (Newton-Cotes) or half width is
-// already there, so no second division is waited for.
+// axis_scale from an axis's map, whose spacing (Newton-Cotes) or half width
+// is already there.  Divided like there: times the reciprocal of 3 or 22.5 is
+// off by a unit in the last place per axis, in the same direction on all.
 __device__ inline double axis_scale_of(const Axis& ax, int rule) {
     switch (rule) {
-        case TQ_RULE_TRAPEZOID: return ax.h * 0.5;
-        case TQ_RULE_SIMPSON: return ax.h * (1.0 / 3.0);
-        case TQ_RULE_BOOLE: return ax.h * (1.0 / 22.5);
+        case TQ_RULE_TRAPEZOID: return ax.h / 2.0;
+        case TQ_RULE_SIMPSON: return ax.h / 3.0;
+        case TQ_RULE_BOOLE: return ax.h / 22.5;
         default: return ax.a;
     }
 }
