@@ -178,3 +178,25 @@ def test_rule_scale_is_a_division(d, rule, c, dev):
         for _ in range(d):
             scale *= width / 4.0 / c
         assert _grid64(tq.Constant(d), d, 5, dom, rule=_ops.RULES[rule]) == sums**d * scale
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_one_axis_nodes_to_the_last_bit(batch, dev):
+    """FP64: node j of a Newton-Cotes axis is a + j h rounded once.  The phase
+    2^40 x makes a neighbouring node a different value."""
+    lo, hi, n = 0.5, 0.9, 4097
+    h = (hi - lo) / (n - 1)
+    x = np.array([float(Fraction(lo) + j * Fraction(h)) for j in range(n)])
+    x[-1] = hi
+    w = np.full(n, 2.0)
+    w[0] = w[-1] = 1.0
+    ref = float(np.sum(w * np.cos(2.0**40 * x))) * h / 2.0
+    fn = tq.Oscillatory([2.0**40], 0.0)
+    if batch:
+        got = float(Batch([{"rule": "trapezoid", "fn": fn, "dim": 1, "n": n, "domain": [[lo, hi]]}],
+                          dtype=torch.float64, device=dev).run()[1][0])
+    else:
+        dom = torch.tensor([[lo, hi]], dtype=torch.float64, device=dev)
+        got = _grid64(fn, 1, n, dom, rule=_ops.RULES["trapezoid"])
+    # sines and cosines to a few units in the last place
+    assert abs(got - ref) <= 1e-13 * (hi - lo)

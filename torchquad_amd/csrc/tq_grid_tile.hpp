@@ -312,15 +312,19 @@ __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule,
                 const double row_step = kWave * a0.h;
                 for (long long tb = ib; tb < ie; tb += kFlush) {
                     const long long te = (tb + kFlush < ie) ? (tb + kFlush) : ie;
-                    // four rows per trip: one FP64 product for their nodes, then an addition each
+                    // four rows per trip: one conversion of the index.  FP32: one FP64 product for their nodes, then
+                    // an addition each; FP64: the nodes rounded once, like everywhere else.
                     T fa = T(0);
                     long long t = tb;
                     constexpr int U = FAM == TQ_FAM_SIN_SUM ? 1 : 4;
                     for (; t + U <= te; t += U) {
-                        const double x0 = fma((double)(t * kWave + lane), a0.h, a0.a);
+                        const double j0 = (double)(t * kWave + lane), x0 = fma(j0, a0.h, a0.a);
 #pragma unroll
-                        for (int u = 0; u < U; ++u)
-                            fa += F::finish(F::fold_c(s0, ac0, (T)(u ? x0 + u * row_step : x0), p), p);
+                        for (int u = 0; u < U; ++u) {
+                            double x = x0;
+                            if (u) x = sizeof(T) == 4 ? x0 + u * row_step : fma(j0 + u * kWave, a0.h, a0.a);
+                            fa += F::finish(F::fold_c(s0, ac0, (T)x, p), p);
+                        }
                     }
                     for (; t < te; ++t)
                         fa += F::finish(F::fold_c(s0, ac0, (T)fma((double)(t * kWave + lane), a0.h, a0.a), p), p);
