@@ -36,3 +36,25 @@ def test_one_gauss_node_per_axis(d, S, dtype, dev):
     _lib.call("tq_grid_reduce_backward", ctypes.byref(desc), _lib.ptr(dom), None, 0, _lib.ptr(g), S, _lib.ptr(other),
               _lib.stream_ptr(dev))
     assert bool(((other.double() - ref[0]).abs() <= eps * ref[0]).all())
+
+
+@pytest.mark.parametrize("rule", ["trapezoid", "gauss_legendre"])
+@pytest.mark.parametrize("d,n", [(1, 1001), (2, 31), (1, 3001)])
+def test_points_backward_at_the_upper_end(d, n, rule, dev):
+    """d/d lower bound takes g (1 - t) of every point: values 1e15 times as
+    large at t = 1 do not blur it (Newton-Cotes: t is 1 there exactly)."""
+    if rule == "gauss_legendre":
+        t = torch.linspace(0.0, 1.0, n, dtype=torch.float64, device=dev)
+        gl = (2.0 * t - 1.0, torch.ones_like(t))
+    else:
+        t, gl = torch.arange(n, dtype=torch.float64, device=dev) / (n - 1), None
+    dom = torch.tensor([[-0.5, 1.0]] * d, dtype=torch.float64, device=dev)
+    g = torch.ones([n] * d + [d], dtype=torch.float64, device=dev)
+    for k in range(d):
+        g.select(k, n - 1)[..., k] = 1e15
+    got = _ops.grid_points_backward(_ops.RULES[rule], d, n, dom, g.reshape(-1, d).contiguous(), gl)
+    for k in range(d):
+        rows = g[..., k].sum(dim=[q for q in range(d) if q != k]) if d > 1 else g[..., 0]
+        ref = float(torch.sum(rows * (1.0 - t)))
+        # a sum of n^d terms of one sign, t to half a unit in the last place
+        assert abs(float(got[k, 0]) - ref) <= (n**d + 4) * 2.0**-53 * ref

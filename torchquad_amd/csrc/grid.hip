@@ -668,22 +668,19 @@ __global__ __launch_bounds__(kBlock) void k_grid_points_backward(int d, int n, i
             if (r >= per32) r -= per32;
             return TABLE ? s_t[j] : node_fraction(j, n, rule, glx);
         };
+        // (sum g - sum g t would lose the first where the gradients sit at the upper end)
+        auto add = [&](double g, double t) {
+            acc = fma(g, 1.0 - t, acc);
+            acc_t = fma(g, t, acc_t);
+        };
         for (; p + (long long)(U - 1) * step < p1; p += (long long)U * step, src += U * row) {
             T x[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) x[u] = src[u * row];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const double g = (double)x[u];
-                acc += g;
-                acc_t = fma(g, fraction(p + (long long)u * step), acc_t);
-            }
+            for (int u = 0; u < U; ++u) add((double)x[u], fraction(p + (long long)u * step));
         }
-        for (; p < p1; p += step, src += row) {
-            const double g = (double)*src;
-            acc += g;
-            acc_t = fma(g, fraction(p), acc_t);
-        }
+        for (; p < p1; p += step, src += row) add((double)*src, fraction(p));
     }
     s_a[threadIdx.x] = acc;
     s_b[threadIdx.x] = acc_t;
@@ -695,7 +692,7 @@ __global__ __launch_bounds__(kBlock) void k_grid_points_backward(int d, int n, i
                 va += s_a[q * kWave + i];
                 vb += s_b[q * kWave + i];
             }
-        partials[((long long)blockIdx.x * d + threadIdx.x) * 2] = va - vb;
+        partials[((long long)blockIdx.x * d + threadIdx.x) * 2] = va;
         partials[((long long)blockIdx.x * d + threadIdx.x) * 2 + 1] = vb;
     }
 }
