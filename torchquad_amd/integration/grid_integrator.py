@@ -162,7 +162,7 @@ class GridIntegrator(BaseIntegrator):
         if self._tq_standard():
             # user callable: HIP points -> fn -> HIP weighted reduction with the
             # rule's own weights (no [N] weight tensor is built)
-            if type(self).calculate_grid is GridIntegrator.calculate_grid:
+            if type(self).calculate_grid is GridIntegrator.calculate_grid and "calculate_grid" not in vars(self):
                 # Gaussian rules scale by the domain, and so do Newton-Cotes rules whose domain carries
                 # a gradient (h = width / (n - 1) there too): neither forms the mesh widths
                 gauss = self._tq_rule == _ops.RULES["gauss_legendre"]
