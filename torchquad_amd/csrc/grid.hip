@@ -398,13 +398,15 @@ static void launch_points_staged(const tq_grid_desc* g, const void* domain, long
                                  hipStream_t st) {
     const FastDiv by_n = make_fast_div((uint32_t)g->n);
     const size_t nodes = (size_t)g->dim * g->n * sizeof(T);
-    const bool table = nodes <= kNodeTableMax;
-    const size_t lds = stage_bytes(g->dim, sizeof(T)) * kWavesPerBlock + (table ? nodes : 0);
     const uint32_t chunks = (uint32_t)((P + kWave * PPL - 1) / (kWave * PPL));
     // as many blocks as there is work for, at most 8 per CU: each builds the
     // node table once and then walks its chunks
     long long blocks = ((long long)chunks + kWavesPerBlock - 1) / kWavesPerBlock;
     if (blocks > 2048) blocks = 2048;
+    // the node table where a block uses a node twice or more: 4000 points of
+    // one axis took 4.5 us with it, 2.5 us without
+    const bool table = nodes <= kNodeTableMax && P >= 2 * blocks * g->n;
+    const size_t lds = stage_bytes(g->dim, sizeof(T), PPL) * kWavesPerBlock + (table ? nodes : 0);
     if (table)
         hipLaunchKernelGGL((k_grid_points_staged<T, true, PPL>), dim3((unsigned)blocks), dim3(kBlock), lds, st,
                            (const T*)domain, g->dim, by_n, g->rule, g->gl_nodes, (uint32_t)P, chunks, (T*)points,
@@ -418,8 +420,9 @@ static void launch_points_staged(const tq_grid_desc* g, const void* domain, long
 template <typename T>
 static int launch_points(const tq_grid_desc* g, const void* domain, long long P, void* points, void* h,
                          hipStream_t st) {
-    if (P <= 0x7fffffffLL && stage_fits(g->dim, sizeof(T), points)) {
-        if (stage_ppl(g->dim, sizeof(T)) > 1)
+    const int ppl = stage_ppl(g->dim, sizeof(T), P, 2048);
+    if (P <= 0x7fffffffLL && stage_fits(g->dim, sizeof(T), ppl, points)) {
+        if (ppl > 1)
             launch_points_staged<T, 16 / (int)sizeof(T)>(g, domain, P, points, h, st);
         else
             launch_points_staged<T, 1>(g, domain, P, points, h, st);
@@ -509,18 +512,24 @@ __global__ __launch_bounds__(kBlock) void k_grid_reduce_backward(PointWeights w,
     if (tid == 0) s_scale = scale();
     const WeightTables tab = build_weights<MODE>(w, s_w);
     __syncthreads();
+    const double sc = s_scale;
     const long long wave = (long long)blockIdx.x * kWavesPerBlock + __builtin_amdgcn_readfirstlane(tid >> 6);
     const long long e0 = wave * span;
     if (e0 >= total) return;
     const uint32_t len = (uint32_t)(total - e0 < span ? total - e0 : span);
-    const long long pt0 = S == 1 ? e0 : e0 / S;
-    const uint32_t sub0 = S == 1 ? 0u : (uint32_t)(e0 - pt0 * S);
-    uint32_t row0 = 0, in0 = (uint32_t)pt0;
-    if (MODE != kUnitWeights && w.outer_axes > 0) {
-        row0 = (uint32_t)(pt0 / w.inner);
-        in0 = (uint32_t)(pt0 - (long long)row0 * w.inner);
+    uint32_t sub0 = 0, row0 = 0, in0 = 0;
+    if (total <= 0x7fffffffLL) {  // every index fits the 32-bit divisions below
+        if (S == 1) in0 = (uint32_t)e0;
+        else sub0 = (uint32_t)e0;
+    } else {
+        const long long pt0 = S == 1 ? e0 : e0 / S;
+        sub0 = S == 1 ? 0u : (uint32_t)(e0 - pt0 * S);
+        in0 = (uint32_t)pt0;
+        if (MODE != kUnitWeights && w.outer_axes > 0) {
+            row0 = (uint32_t)(pt0 / w.inner);
+            in0 = (uint32_t)(pt0 - (long long)row0 * w.inner);
+        }
     }
-    const double sc = s_scale;
     const double g0 = S == 1 ? (double)grad_out[0] : 0.0;
     T* dst = grad_f + e0;
     auto values = [&](uint32_t off, T* x, int count) {
@@ -572,6 +581,14 @@ __global__ __launch_bounds__(kBlock) void k_grid_reduce_backward(PointWeights w,
     for (off += lane; off < len; off += kWave) values(off, dst + off, 1);
 }
 
+// Below kSmallBackward values a lane writes one, with the weights formed where
+// they are used: the tables that a block would build first, and waves of 1024
+// values on a few CUs, took longer than the launch (1.5e4 values, d=4, FP64:
+// 6.7 us, now 3.5; 1e6 values, d=6, FP32: 6.4 us with tables, 9.7 without).
+// Up to kMidBackward values waves of 256 still leave enough of them (7e5
+// values, FP32: 4.0 us, 6.5 with 1024; 3e6: 10.2 and 9.5).
+constexpr long long kSmallBackward = 1LL << 19, kMidBackward = 1LL << 21;
+
 template <typename T>
 static int launch_reduce_backward(const tq_grid_desc* g, const void* domain, const void* hs, int unit,
                                   const void* grad_out, long long S, void* grad_f, const void* out, void* grad_domain,
@@ -581,15 +598,18 @@ static int launch_reduce_backward(const tq_grid_desc* g, const void* domain, con
     int rc = plan_reduce(g, 1, unit, V);
     if (rc) return rc;
     const long long total = V.P * S;
+    const bool small = total < kSmallBackward;
+    if (small && V.w.mode != kUnitWeights) direct_weights(g->dim, V);
     const GridScale<T> scale{(const T*)domain, (const T*)hs, g->dim, g->n, g->rule, unit};
     long long span = (total + 8191) / 8192;
-    if (span < 1024) span = 1024;
+    if (span < 1024) span = total < kMidBackward ? 256 : 1024;
     span = (span + kWave * VEC - 1) / (kWave * VEC) * (kWave * VEC);
+    if (small) span = kWave;
     if (span > (1LL << 30)) return fail(TQ_E_ARG, "too many values for one launch");
     const long long per_block = span * kWavesPerBlock;
     const long long blocks = (grad_f ? (total + per_block - 1) / per_block : 0) + (grad_domain ? 1 : 0);
     if (blocks == 0) return TQ_OK;
-    const bool vec = ((uintptr_t)grad_f & 15) == 0 &&
+    const bool vec = !small && ((uintptr_t)grad_f & 15) == 0 &&
                      (V.w.mode == kUnitWeights || S > 1 || V.w.inner >= (uint32_t)VEC);
     const FastDiv by_S = make_fast_div((uint32_t)S);
 #define TQ_RB(VV, MODE)                                                                                             \
@@ -708,9 +728,9 @@ __global__ __launch_bounds__(kBlock) void k_grid_points_backward_finalize(const 
     if (threadIdx.x == 0) grad_domain[e] = (T)v;
 }
 
-// Points per wave: at most about 4096 waves, at least 2048 values each.
+// Points per wave: at most about 4096 waves, at least 512 values each.
 static void points_backward_shape(int d, long long P, long long* span, long long* nb) {
-    const long long least = (2048 + d - 1) / d;
+    const long long least = (512 + d - 1) / d;
     long long s = (P + 4095) / 4096;
     if (s < least) s = least;
     *span = s;

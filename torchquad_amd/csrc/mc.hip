@@ -170,7 +170,8 @@ __global__ __launch_bounds__(kBlock) void k_mc_points(const T* domain, int d, lo
     }
 }
 
-// Unaligned outputs: one sample per thread, stored coordinate by coordinate.
+// Unaligned outputs and few samples of one or two axes: one sample per
+// thread, stored coordinate by coordinate.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_mc_points_any(const T* domain, int d, long long N, uint64_t seed,
                                                           uint64_t offset, T* pts) {
@@ -192,16 +193,17 @@ __global__ __launch_bounds__(kBlock) void k_mc_points_any(const T* domain, int d
 template <typename T>
 static int launch_mc_points(const tq_mc_desc* m, const void* domain, void* points, hipStream_t st) {
     long long blocks = (m->N + kBlock - 1) / kBlock;
-    if (!stage_fits(m->dim, sizeof(T), points)) {
+    const int ppl = stage_ppl(m->dim, sizeof(T), m->N, 1024);
+    // one point per lane of one or two coordinates is as good as contiguous (1000 points, FP32: 2.3 us, staged 2.5)
+    if ((ppl == 1 && m->dim <= 2) || !stage_fits(m->dim, sizeof(T), ppl, points)) {
         if (blocks > 65536) blocks = 65536;
         hipLaunchKernelGGL((k_mc_points_any<T>), dim3((unsigned)blocks), dim3(kBlock), 0, st, (const T*)domain,
                            m->dim, m->N, m->seed, m->offset, (T*)points);
         return check_launch("k_mc_points_any");
     }
-    const int ppl = stage_ppl(m->dim, sizeof(T));
     blocks = (blocks + ppl - 1) / ppl;
     if (blocks > 4096) blocks = 4096;
-    const size_t lds = stage_bytes(m->dim, sizeof(T)) * kWavesPerBlock;
+    const size_t lds = stage_bytes(m->dim, sizeof(T), ppl) * kWavesPerBlock;
 #define TQ_MC_POINTS(MAXD)                                                                                        \
     hipLaunchKernelGGL((k_mc_points<T, MAXD>), dim3((unsigned)blocks), dim3(kBlock), lds, st, (const T*)domain,   \
                        m->dim, (long long)m->N, m->seed, m->offset, ppl, (T*)points)

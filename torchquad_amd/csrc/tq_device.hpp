@@ -71,15 +71,23 @@ __device__ inline void wave_lds_fence() {
 // coordinates itself would touch 64 separate d-element rows per store
 // instruction.  Instead each wave puts a chunk of 64 ppl points into its own
 // LDS slice and writes the slice out in 16-byte pieces, consecutive lanes at
-// consecutive addresses (5 axes, 6.9e7 FP32 points: 530 us with lane-strided
+// consecutive addresses (5 axes of 37, 6.9e7 FP32 points: 530 us with lane-strided
 // 4-byte stores and 64-bit index divisions, 237 us or 5.8 TB/s of writes so).
 constexpr size_t kStageMax = 40 * 1024;  // LDS of a block's slices
 
-// Points per lane and chunk: 16 bytes of each coordinate while four slices stay small, else one point.
-inline int stage_ppl(int d, int tsize) { return d <= 8 ? 16 / tsize : 1; }
-inline size_t stage_bytes(int d, int tsize) { return (size_t)kWave * stage_ppl(d, tsize) * d * tsize; }
-inline bool stage_fits(int d, int tsize, const void* out) {
-    return stage_bytes(d, tsize) * kWavesPerBlock <= kStageMax && ((uintptr_t)out & 15) == 0;
+// Points per lane and chunk: 16 bytes of each coordinate while four slices
+// stay small and the chunks still make `waves` waves; else one point.  Eight
+// waves per CU for grids, four for Monte Carlo, whose points cost more to
+// make (FP32, one and four points per lane: grid d=8 n=5 5.9 and 7.1 us;
+// Monte Carlo d=2, 65000 points 2.6 and 3.2 us, 400000 points 4.4
+// and 3.9 us).
+inline int stage_ppl(int d, int tsize, long long points, int waves) {
+    const int ppl = d <= 8 ? 16 / tsize : 1;
+    return points >= (long long)waves * kWave * ppl ? ppl : 1;
+}
+inline size_t stage_bytes(int d, int tsize, int ppl) { return (size_t)kWave * ppl * d * tsize; }
+inline bool stage_fits(int d, int tsize, int ppl, const void* out) {
+    return stage_bytes(d, tsize, ppl) * kWavesPerBlock <= kStageMax && ((uintptr_t)out & 15) == 0;
 }
 
 // Writes the wave's slice (`points` rows of d values) to out + first * d.  first is a multiple of

@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kBlock) void k_values_narrow(PointWeights w, const 
             in0 = (uint32_t)(p0 - (long long)row0 * w.inner);
         }
         const T* base = fv + p0 * S + lane;
-        constexpr int U = 4;
+        constexpr int U = MODE == kUnitWeights ? 8 : 4;  // loads in flight; with weights, 4 take fewer registers
         uint32_t off = po;
         const uint32_t row = step * (uint32_t)S;  // values per step
         long long at = 0;
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(kFinalBlock) void k_values_final(const double* part
     if (S < kWave) {
         const long long s = blockIdx.x;
         double v = 0.0;
-        for (long long b = threadIdx.x; b < blocks; b += kFinalBlock) v += partials[b * S + s];
+        for (long long b = threadIdx.x; b < blocks; b += blockDim.x) v += partials[b * S + s];
         v = block_sum(v, s_red);
         if (threadIdx.x == 0) out[s] = (T)(v * scale());
         return;
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kFinalBlock) void k_values_final(const double* part
 
 // Plan for f[P, S] of the data type's size; d = 0: unit weights over P
 // points.  Waves: at most about 8192 (32 per CU), each with at least 1024
-// values, so small inputs still spread over the chip and the final sum
+// values (512 of several components below 2^20 of them), so small inputs still spread over the chip and the final sum
 // stays short.  The block count does not depend on the buffer's alignment.
 inline int plan_values(int d, int n, int rule, const double* glw, long long P, long long S, int tsize, ValuePlan& V) {
     V.P = P;
@@ -372,7 +372,8 @@ inline int plan_values(int d, int n, int rule, const double* glw, long long P, l
     const long long groups = S < kWave ? 1 : (S + kWave - 1) / kWave;
     const long long waves = 8192 / groups > 4 ? 8192 / groups : 4;
     long long span = (P + waves - 1) / waves;
-    const long long least = S < kWave ? 1024 / S : 16;  // points per wave
+    // points per wave
+    const long long least = S == 1 ? 1024 : S < kWave ? (P * S < (1LL << 20) ? 512 : 1024) / S : 16;
     if (span < least) span = least;
     const long long round = S == 1 ? kWave * vec : 1;  // of the data type, whatever the weights allow
     span = (span + round - 1) / round * round;
@@ -380,6 +381,15 @@ inline int plan_values(int d, int n, int rule, const double* glw, long long P, l
     V.span = span;
     V.blocks = (P + span * kWavesPerBlock - 1) / (span * kWavesPerBlock);
     return TQ_OK;
+}
+
+// The plan's weights without tables: one inner axis, the others outer ones.
+inline void direct_weights(int d, ValuePlan& V) {
+    V.w.mode = kDirectWeights;
+    V.w.inner = (uint32_t)V.w.n;
+    V.w.outer_axes = d - 1;
+    V.w.by_inner = V.w.by_n;
+    V.lds = 0;
 }
 
 inline size_t values_workspace(const ValuePlan& V) { return (size_t)(V.blocks * V.S) * sizeof(double); }
@@ -412,7 +422,9 @@ static int launch_values(const ValuePlan& V, const T* fv, double* partials, SCAL
     const int rc = check_launch("k_values");
     if (rc) return rc;
     const long long fb = V.S < kWave ? V.S : (V.S + kWave - 1) / kWave;
-    hipLaunchKernelGGL((k_values_final<T, SCALE>), dim3((unsigned)fb), dim3(kFinalBlock), 0, st, partials, V.blocks,
+    // (few partials: four waves start and meet sooner than sixteen)
+    const int threads = V.S < kWave && V.blocks <= kBlock ? kBlock : kFinalBlock;
+    hipLaunchKernelGGL((k_values_final<T, SCALE>), dim3((unsigned)fb), dim3(threads), 0, st, partials, V.blocks,
                        V.S, scale, out);
     return check_launch("k_values_final");
 }
