@@ -209,8 +209,7 @@ __device__ inline double gl_pair_rows(int n, const Params<float>& p, const Axis&
             fa = fmaf(e.y, value(fmaf(sa, e.x, sh)), fa);
             fa = fmaf(e.y, value(fmaf(-sa, e.x, sh)), fa);
         };
-        // (one row where the sine's argument reduction would be repeated eightfold: 132 registers)
-        constexpr int U = FAM == TQ_FAM_SIN_SUM ? 1 : 4;
+        constexpr int U = 4;
         long long t = tb;
         for (; t + U <= tf; t += U) {
             const float2* row = pairs + t * kWave;
@@ -316,7 +315,7 @@ __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule,
                     // an addition each; FP64: the nodes rounded once, like everywhere else.
                     T fa = T(0);
                     long long t = tb;
-                    constexpr int U = FAM == TQ_FAM_SIN_SUM ? 1 : 4;
+                    constexpr int U = 4;
                     for (; t + U <= te; t += U) {
                         const double j0 = (double)(t * kWave + lane), x0 = fma(j0, a0.h, a0.a);
 #pragma unroll
