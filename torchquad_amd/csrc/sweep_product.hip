@@ -14,13 +14,19 @@
 // 1024 Gaussian peaks of 32^4 FP32 points: forward 122 -> 32 us, backward
 // 332 -> 70 us against one exponential per point (grad.hip, which keeps one
 // axis, axes too long for the tables and the oscillatory backward).
+#include "tq_grid_launch.hpp"
 #include "tq_product.hpp"
 #include "tq_sweep.hpp"
 
 namespace tq {
 
+// Waves of a block: at most, and for integrals of P points.  A block builds its
+// tables and sums its waves; small integrals in waves that have next to nothing
+// to do paid for both (1000 Gaussian peaks of 14^3 FP32 points: forward 12.3
+// us with eight waves, 10.1 with four; backward 30 and 15.5).
 constexpr int kSweepBlockWaves = 8;
 constexpr int kSweepThreads = kSweepBlockWaves * kWave;
+static int sweep_block_waves(long long P) { return P <= 1024 ? 1 : P <= 2048 ? 2 : P <= 4096 ? 4 : kSweepBlockWaves; }
 constexpr size_t kSweepLdsMax = 60 * 1024;
 // States per lane: the backward reads a loop entry's three or four tables per
 // point from LDS, which eight FP32 states share.
@@ -32,6 +38,7 @@ struct SweepUnits {
     ProductSplit s;
     int rule;
     int parts;
+    int block_waves;
     long long per;  // items per part
 };
 
@@ -47,7 +54,10 @@ static bool plan_sweep_product(const tq_grid_desc* g, int C, int tsize, bool bac
                             kSweepLdsMax - extra, U.s, backward ? 1 : 2))
         return false;
     U.rule = g->rule;
-    const long long waves = blocks * kSweepBlockWaves;
+    long long P;
+    ipow_checked(n, d, 1LL << 62, &P);
+    U.block_waves = sweep_block_waves(P);
+    const long long waves = blocks * U.block_waves;
     long long parts = waves / U.s.lane_groups;
     if (parts < 1) parts = 1;
     if (parts > U.s.items) parts = U.s.items;
@@ -88,11 +98,11 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_fwd(SweepUnits 
     load_sweep_params<T, FAM>(S.d, S.n, U.rule, b, a, u, dom, &s_p, s_axis);
     __syncthreads();
     const ProductTables<T> tab = build_product_tables<FAM, T>(S, U.rule, s_axis, glx, glw, s_p, s_lds, s_exp);
-    const int units = S.lane_groups * U.parts, waves = gridDim.x * kSweepBlockWaves;
+    const int units = S.lane_groups * U.parts, waves = gridDim.x * U.block_waves;
     double acc = 0.0;
     Factor<FAM, T> own[K];
     double wl[K];
-    for (int w = blockIdx.x * kSweepBlockWaves + __builtin_amdgcn_readfirstlane(tid >> 6); w < units; w += waves) {
+    for (int w = blockIdx.x * U.block_waves + __builtin_amdgcn_readfirstlane(tid >> 6); w < units; w += waves) {
         const int lg = w / U.parts, part = w - lg * U.parts;
         const long long t0 = part * U.per, t1 = t0 + U.per < S.items ? t0 + U.per : S.items;
         lane_states<FAM, T, K>(S, tab, lg * kWave + (tid & (kWave - 1)), own, wl);
@@ -131,7 +141,6 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
     __shared__ Params<T> s_p;
     __shared__ Axis s_axis[TQ_MAX_DIM];
     __shared__ int s_exp[kExpSlots];
-    __shared__ double s_red[kSweepBlockWaves];
     const ProductSplit& S = U.s;
     const int n = S.n, L = S.L, groups = S.groups, entries = groups * kGroup;
     const long long b = blockIdx.y;
@@ -143,7 +152,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
     T* s_t = mom + NM * entries;
     T* s_g = s_t + D * n;
     T* s_r = s_g + (FAM == TQ_FAM_PRODUCT_PEAK ? D * n : 0);
-    for (int e = tid; e < D * n; e += kSweepThreads) {
+    for (int e = tid; e < D * n; e += blockDim.x) {
         const int k = (int)S.by_n.div((uint32_t)e), j = e - k * n;
         const T t = (T)node_of(s_axis[k], j, n, U.rule, glx) - s_p.u[k];
         s_t[e] = t;
@@ -155,7 +164,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
         sweep_functions<FAM>((double)s_t[k * n + j], FAM == TQ_FAM_PRODUCT_PEAK ? (double)s_g[k * n + j] : 0.0,
                              (double)s_r[j], h);
     };
-    for (int e = tid; e < entries; e += kSweepThreads) {
+    for (int e = tid; e < entries; e += blockDim.x) {
         double h[3] = {0.0, 0.0, 0.0};
         const double v = (double)tab.loop[e];  // zero past the last node
         const int j = e < n ? e : 0;
@@ -185,8 +194,8 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
             for (int i = 0; i < 3; ++i) acc[i][k] = fma(h[i], fk, acc[i][k]);
         }
     };
-    const int units = S.lane_groups * U.parts, waves = gridDim.x * kSweepBlockWaves;
-    for (int w = blockIdx.x * kSweepBlockWaves + __builtin_amdgcn_readfirstlane(tid >> 6); w < units; w += waves) {
+    const int units = S.lane_groups * U.parts, waves = gridDim.x * U.block_waves;
+    for (int w = blockIdx.x * U.block_waves + __builtin_amdgcn_readfirstlane(tid >> 6); w < units; w += waves) {
         const int lg = w / U.parts, part = w - lg * U.parts;
         const long long t0 = part * U.per, t1 = t0 + U.per < S.items ? t0 + U.per : S.items;
         const int slot = lg * kWave + lane;
@@ -311,18 +320,28 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
         const double h[3] = {M[0], M[1], M[NM - 1]};
         add(L, h, 1.0);
     }
-    int exponent = 0;
-    for (int k = 0; k < D; ++k) exponent += exp_or_zero(s_exp[k]);
-    double* out = partials + (b * gridDim.x + blockIdx.x) * (1 + 3 * D);
-    double v = block_sum(accF, s_red);
-    if (tid == 0) out[0] = ldexp(v, exponent);
+    // the waves' sums meet in LDS once, then a thread adds each value's (block sums one after the other: two barriers
+    // and twelve LDS permutes for each of the 1 + 3 D)
+    constexpr int V = 1 + 3 * D;
+    __shared__ double s_sum[kSweepBlockWaves][V];
+    const int wb = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto put = [&](int i, double x) {
+        x = wave_sum_last(x);
+        if (lane == kWave - 1) s_sum[wb][i] = x;
+    };
+    put(0, accF);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int k = 0; k < D; ++k) {
-            v = block_sum(acc[i][k], s_red);
-            if (tid == 0) out[1 + i * D + k] = ldexp(v, exponent);
-        }
+        for (int k = 0; k < D; ++k) put(1 + i * D + k, acc[i][k]);
+    __syncthreads();
+    if (tid < V) {
+        int exponent = 0;
+        for (int k = 0; k < D; ++k) exponent += exp_or_zero(s_exp[k]);
+        double x = 0.0;
+        for (int q = 0; q < U.block_waves; ++q) x += s_sum[q][tid];
+        partials[(b * gridDim.x + blockIdx.x) * V + tid] = ldexp(x, exponent);
+    }
 }
 
 template <typename T, int FAM>
@@ -332,7 +351,7 @@ int launch_sweep_product_fwd(const tq_grid_desc* g, int64_t B, const void* a, co
     const int C = family_comps(FAM);
     if (!plan_sweep_product(g, C, (int)sizeof(T), false, blocks, U)) return fail(TQ_E_ARG, "no product plan for the sweep");
     hipLaunchKernelGGL((k_sweep_product_fwd<T, FAM, kSweepStates<T>>), dim3((unsigned)blocks, (unsigned)B),
-                       dim3(kSweepThreads), product_lds_bytes(U.s, C, (int)sizeof(T)), s, U, (const T*)a, (const T*)u,
+                       dim3(U.block_waves * kWave), product_lds_bytes(U.s, C, (int)sizeof(T)), s, U, (const T*)a, (const T*)u,
                        (const T*)dom, g->gl_nodes, g->gl_weights, partials);
     return check_launch("k_sweep_product_fwd");
 }
@@ -344,7 +363,7 @@ static void launch_bwd(const SweepUnits& U, const tq_grid_desc* g, int64_t B, co
     const size_t lds = product_lds_bytes(U.s, 1, (int)sizeof(T)) + 16 +
                        ((size_t)sweep_moments(FAM) * entries + (size_t)2 * D * n + n) * sizeof(T);
     hipLaunchKernelGGL((k_sweep_product_bwd<T, FAM, kSweepStates<T>, D>), dim3((unsigned)blocks, (unsigned)B),
-                       dim3(kSweepThreads), lds, s, U, (const T*)a, (const T*)u, (const T*)dom, g->gl_nodes,
+                       dim3(U.block_waves * kWave), lds, s, U, (const T*)a, (const T*)u, (const T*)dom, g->gl_nodes,
                        g->gl_weights, partials);
 }
 
