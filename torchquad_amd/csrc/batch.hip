@@ -22,7 +22,7 @@ namespace tq {
 
 template <typename T>
 struct BatchDev {
-    int rule, fam, d, n, m, L, q, nl, lane_count, lane_waves;
+    int rule, fam, d, n, m, L, nl, lane_count, lane_waves;
     int product;      // 1: `split` and the product kernel, 0: the fields above and grid_tile
     ProductSplit split;
     long long items;
@@ -376,7 +376,6 @@ static bool plan_product_item(const tq_batch_item& it, int tsize, long long tile
     G.rule = it.rule;
     G.m = S.outer + S.inner;
     G.L = S.L;
-    G.q = S.q;
     G.nl = S.nl;
     G.lane_count = S.slots;
     G.lane_waves = S.lane_groups;
@@ -447,7 +446,6 @@ static int plan_batch(const tq_batch_item* items, long long count, long long til
             D.n = it.n;
             D.m = G.m;
             D.L = G.L;
-            D.q = G.q;
             D.nl = G.nl;
             D.lane_count = G.lane_count;
             D.lane_waves = G.lane_waves;

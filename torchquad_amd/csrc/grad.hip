@@ -34,8 +34,7 @@ constexpr long long kSweepWaves = 16384;
 static int sweep_geom(const tq_grid_desc* gd, long long B, SweepGeom& S) {
     const long long per_integral = B > 0 ? (kSweepWaves + B - 1) / B : kSweepWaves;
     // the backward's one-axis rows walk every node, so the forward does too
-    int rc = plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, per_integral, S.g, 0, false,
-                       false);
+    int rc = plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, per_integral, S.g, false);
     if (rc) return rc;
     S.blocks_x = (S.g.num_waves + kWavesPerBlock - 1) / kWavesPerBlock;
     return TQ_OK;

@@ -73,10 +73,10 @@ static int check_gl_tables(const tq_grid_desc* g) {
     return TQ_OK;
 }
 
-// merge_cap 1024: the plan that workspaces are sized by (at least as many
-// workgroups as any launch takes).
-static int make_geom(const tq_grid_desc* gd, GridGeom& G, long long merge_cap = 1024) {
-    return plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, 16384, G, merge_cap);
+// The point-by-point kernel's plan, which workspaces are sized by; the product
+// kernel keeps its workgroups within the workspace it is given.
+static int make_geom(const tq_grid_desc* gd, GridGeom& G) {
+    return plan_geom(gd->dim, gd->n, gd->rule, gd->lane_axes, gd->items_per_wave, 16384, G);
 }
 
 // ---------------------------------------------------------------------------
@@ -268,10 +268,6 @@ static int launch_grid(const tq_grid_desc* gd, const tq_integrand* f, const void
     bool taken = false;
     rc = launch_grid_product<T>(gd, f, domain, ws, ws_bytes, out, out64, st, &taken);
     if (rc || taken) return rc;
-    // one loop axis: the integrals that could merge two take the product kernel
-    rc = make_geom(gd, G, 0);
-    if (rc) return rc;
-    if (ws_bytes < kWsHeader + (size_t)G.blocks * sizeof(double)) return fail(TQ_E_WORKSPACE, "grid workspace too small");
     GridArgs<T> A;
     A.g = G;
     A.domain = (const T*)domain;

@@ -453,8 +453,8 @@ __device__ inline double grid_tile(int d, int n, int nl, int m, int L, int rule,
 
 // ---- host-side planning ---------------------------------------------------
 struct GridGeom {
-    int d, n, m, L;       // L: row axes [0, L), loop axes [L, L + q)
-    int q, nl;            // loop axes (1 or 2) and loop length n^q
+    int d, n, m, L;       // L: row axes [0, L), loop axis L
+    int nl;               // loop length (n; batched product tiles: n or n^2)
     int rule;
     int lane_count;       // n^m
     int lane_waves;       // ceil(lane_count / 64)
@@ -477,26 +477,15 @@ inline int ipow_checked(long long base, int e, long long limit, long long* out) 
     return 0;
 }
 
-// Largest n for which the planner gives up a lane axis to merge two loop
-// axes (the choice of lane axes, and so the launch size, then does not
-// depend on merge caps of 1024 or more).
-constexpr int kMergeMaxN = 32;
-
 // Splits the n^d index space of one integral (see grid_tile).  lane_axes /
-// items_per_wave override the automatic choice (0 = automatic).  When
-// merge_cap > 0 and n^2 <= merge_cap, the loop is planned over the last two
-// non-lane axes: no kernel walks such a plan (those integrals take the factor
-// tables of tq_product.hpp), but the sizes of the plain path's workspace, and
-// so the grids that fit a given one, are those of this plan.
-// trade_lane_axis = false keeps the lane axes of the unmerged plan.  gl_fold:
-// a one-axis (m == 0) Gauss-Legendre plan covers half the table (grid_tile's
+// items_per_wave override the automatic choice (0 = automatic).  gl_fold: a
+// one-axis (m == 0) Gauss-Legendre plan covers half the table (grid_tile's
 // GL_FOLD).
 inline int plan_geom(int d, int n, int rule, int lane_axes, long long items_per_wave, long long target_waves,
-                     GridGeom& G, long long merge_cap = 0, bool trade_lane_axis = true, bool gl_fold = true) {
+                     GridGeom& G, bool gl_fold = true) {
     G.d = d;
     G.n = n;
     G.rule = rule;
-    G.q = 1;
     G.nl = n;
     G.gl_fold = 0;
     int m = 0;
@@ -526,16 +515,6 @@ inline int plan_geom(int d, int n, int rule, int lane_axes, long long items_per_
             }
         }
         if (d == 1) m = 1;
-        // One lane axis fewer when that lets the loop run over two short
-        // axes (n^2 points per row instead of n) and the lanes still fill
-        // three quarters of their waves.
-        if (trade_lane_axis && merge_cap > 0 && d >= 3 && d - m == 1 && m >= 2 && n <= kMergeMaxN &&
-            (long long)n * n <= merge_cap) {
-            long long c1 = 1;
-            for (int k = 0; k < m - 1; ++k) c1 *= n;
-            const double util = (double)c1 / (double)(((c1 + kWave - 1) / kWave) * kWave);
-            if (util >= 0.75) m -= 1;
-        }
     }
     long long items = 1;
     if (m == 0) {
@@ -554,14 +533,9 @@ inline int plan_geom(int d, int n, int rule, int lane_axes, long long items_per_
         G.lane_waves = (int)((lc + kWave - 1) / kWave);
         G.L = d - m - 1;
         if (G.L >= 0) ipow_checked(n, d - m, 1LL << 62, &items);
-        if (merge_cap > 0 && G.L >= 1 && (long long)n * n <= merge_cap) {
-            G.q = 2;
-            G.nl = n * n;
-            G.L -= 1;
-        }
     }
     G.items = items;
-    G.use_table = (G.m > 0 && G.L >= 0 && (G.nl <= kLoopTable || G.q == 2)) ? 1 : 0;
+    G.use_table = (G.m > 0 && G.L >= 0 && G.nl <= kLoopTable) ? 1 : 0;
     long long ipw = items_per_wave;
     if (ipw <= 0) {
         const long long work = items * (long long)G.lane_waves;
