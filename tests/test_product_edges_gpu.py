@@ -200,3 +200,24 @@ def test_one_axis_nodes_to_the_last_bit(batch, dev):
         got = _grid64(fn, 1, n, dom, rule=_ops.RULES["trapezoid"])
     # sines and cosines to a few units in the last place
     assert abs(got - ref) <= 1e-13 * (hi - lo)
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_exponents_that_cancel_between_axes(batch, dev):
+    """FP64 exp-linear with exponents of 7e8 octaves on two axes whose sum is
+    small: the integrand's change over the box (5 octaves each) counts."""
+    n, hi = 9, 0.5 + 2.0**-28
+    a = [1e9, -1e9, 1.0]
+    fn = tq.ExpLinear(3, a, 0.0)
+    x = np.longdouble(0.5) + np.arange(n) * np.longdouble(2.0) ** -31
+    w = np.full(n, 2.0)
+    w[0] = w[-1] = 1.0
+    ref = float(np.exp(np.longdouble(0.5)) * np.prod([np.sum(w * np.exp(np.longdouble(c) * (x - 0.5))) for c in a])) * 2.0**-96
+    if batch:
+        got = float(Batch([{"rule": "trapezoid", "fn": fn, "dim": 3, "n": n, "domain": [[0.5, hi]] * 3}],
+                          dtype=torch.float64, device=dev).run()[1][0])
+    else:
+        dom = torch.tensor([[0.5, hi]] * 3, dtype=torch.float64, device=dev)
+        got = _grid64(fn, 3, n, dom, rule=_ops.RULES["trapezoid"])
+    # an exponent of 2^30 is known to 2^-23
+    assert abs(got - ref) <= 4 * 2.0**-23 * ref

@@ -336,11 +336,9 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
         for (int k = 0; k < D; ++k) put(1 + i * D + k, acc[i][k]);
     __syncthreads();
     if (tid < V) {
-        int exponent = 0;
-        for (int k = 0; k < D; ++k) exponent += exp_or_zero(s_exp[k]);
         double x = 0.0;
         for (int q = 0; q < U.block_waves; ++q) x += s_sum[q][tid];
-        partials[(b * gridDim.x + blockIdx.x) * V + tid] = ldexp(x, exponent);
+        partials[(b * gridDim.x + blockIdx.x) * V + tid] = scale_by(x, sum_exponents(D, s_exp));
     }
 }
 

@@ -48,8 +48,10 @@ constexpr int family_comps(int fam) {
 constexpr bool weights_apart(int fam) { return fam == TQ_FAM_SIN_SUM; }
 
 // log2 of an exponential family's factor; the constant term goes to axis 0.
-// Kept within +-1e8, far outside any result, so that the exponents of 16 axes
-// add up in 32 bits and overflow to infinity only in the result (NaN stays).
+// Kept within a 32-bit integer, far outside any result, so that exponents
+// that cancel between axes do and overflow to infinity happens only in the
+// result (NaN stays).
+__device__ inline double bound_exponent(double e) { return e > 2e9 ? 2e9 : (e < -2e9 ? -2e9 : e); }
 template <int FAM, typename T>
 __device__ inline double factor_exponent(int k, T x, const Params<T>& p) {
     double e;
@@ -60,7 +62,7 @@ __device__ inline double factor_exponent(int k, T x, const Params<T>& p) {
         e = (double)p.a[k] * (double)x;
         if (k == 0) e += (double)p.c1;
     }
-    return e > 1e8 ? 1e8 : (e < -1e8 ? -1e8 : e);
+    return bound_exponent(e);
 }
 
 // Denominator of the product peak's factor on axis k.
@@ -76,17 +78,15 @@ __device__ inline double peak_denominator(int k, T x, const Params<T>& p) {
 // NaN of an integral that is infinite; so its axis keeps the signs of the
 // poles' weights alone, everything else on it counting for nothing beside
 // them, and an exponent that takes any sum but 0 out of the range.
-constexpr int kPoleExp = 1 << 27;  // above every other exponent
+constexpr int kPoleExp = 1 << 27;  // above the product peak's other exponents
 __device__ inline bool is_pole(double denominator) { return fabs(denominator) < 0x1.0p-1022; }
 
 // log2 of the double Gaussian's factors, kept in range as factor_exponent's.
 template <typename T>
 __device__ inline void gauss_exponents(T x, const Params<T>& p, double* ex) {
     const double t1 = (double)x - (double)p.c1, t2 = (double)x - (double)p.c2, c = -(double)p.c3;
-    ex[0] = c * t1 * t1;
-    ex[1] = c * t2 * t2;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) ex[i] = ex[i] > 1e8 ? 1e8 : (ex[i] < -1e8 ? -1e8 : ex[i]);
+    ex[0] = bound_exponent(c * t1 * t1);
+    ex[1] = bound_exponent(c * t2 * t2);
 }
 
 // Weighted factor of a family without exponents.
@@ -182,6 +182,9 @@ __device__ inline long long sum_exponents(int d, const int* s_exp) {
     for (int k = 0; k < d; ++k) e += exp_or_zero(s_exp[k]);
     return e;
 }
+__device__ inline double scale_by(double v, long long e) {
+    return ldexp(v, (int)(e > (1 << 30) ? (1 << 30) : (e < -(1 << 30) ? -(1 << 30) : e)));
+}
 
 // A block's sum v with the powers of two put back that were taken out of its
 // axes.  A pole on every axis: NaN, as from a sum over 0 times infinity.
@@ -191,10 +194,12 @@ __device__ inline double scale_back(int fam, double v, int d, const int* s_exp) 
         const long long e2 = sum_exponents(d, s_exp + TQ_MAX_DIM);
         if (e2 > e) e = e2;
     }
-    int poles = 0;
-    for (int k = 0; k < d; ++k) poles += s_exp[k] >= kPoleExp ? 1 : 0;
-    if (poles == d) return __longlong_as_double(0x7ff8000000000000ll);
-    return ldexp(v, (int)(e > (1 << 30) ? (1 << 30) : (e < -(1 << 30) ? -(1 << 30) : e)));
+    if (fam == TQ_FAM_PRODUCT_PEAK) {
+        int poles = 0;
+        for (int k = 0; k < d; ++k) poles += s_exp[k] >= kPoleExp ? 1 : 0;
+        if (poles == d) return __longlong_as_double(0x7ff8000000000000ll);
+    }
+    return scale_by(v, e);
 }
 
 // An axis's weights where they are kept apart, in the place of the component
