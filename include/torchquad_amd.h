@@ -241,7 +241,7 @@ typedef struct tq_batch_tile {
 } tq_batch_tile;
 
 /* Host-side plan sizes: bytes of the device descriptor array and tile count
- * for tiles of about tile_points points (16 times as many where a workgroup
+ * for tiles of about tile_points points (64 times as many where a workgroup
  * takes a tile). */
 int tq_batch_plan_sizes(const tq_batch_item* items, int64_t count, int32_t dtype, int64_t tile_points,
                         int64_t* desc_bytes, int64_t* n_tiles);
