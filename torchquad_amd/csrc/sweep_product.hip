@@ -12,7 +12,7 @@
 // W r^2, from which the three follow (t = alpha r + gamma on an axis).
 //
 // 1024 Gaussian peaks of 32^4 FP32 points: forward 122 -> 32 us, backward
-// 332 -> 70 us against one exponential per point (grad.hip, which keeps one
+// 332 -> 62 us against one exponential per point (grad.hip, which keeps one
 // axis, axes too long for the tables and the oscillatory backward).
 #include "tq_grid_launch.hpp"
 #include "tq_product.hpp"
@@ -145,6 +145,9 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
     const int n = S.n, L = S.L, groups = S.groups, entries = groups * kGroup;
     const long long b = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    // not blockDim.x, with which the kernel holds 25 more registers (D = 4
+    // product peak, FP32: 134 against 107, three waves per SIMD in place of four)
+    const int stride = U.block_waves * kWave;
     load_sweep_params<T, FAM>(D, n, U.rule, b, a, u, dom, &s_p, s_axis);
     __syncthreads();
     // node tables and the loop axis's moment tables, after the split's own tables
@@ -152,7 +155,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
     T* s_t = mom + NM * entries;
     T* s_g = s_t + D * n;
     T* s_r = s_g + (FAM == TQ_FAM_PRODUCT_PEAK ? D * n : 0);
-    for (int e = tid; e < D * n; e += blockDim.x) {
+    for (int e = tid; e < D * n; e += stride) {
         const int k = (int)S.by_n.div((uint32_t)e), j = e - k * n;
         const T t = (T)node_of(s_axis[k], j, n, U.rule, glx) - s_p.u[k];
         s_t[e] = t;
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
         sweep_functions<FAM>((double)s_t[k * n + j], FAM == TQ_FAM_PRODUCT_PEAK ? (double)s_g[k * n + j] : 0.0,
                              (double)s_r[j], h);
     };
-    for (int e = tid; e < entries; e += blockDim.x) {
+    for (int e = tid; e < entries; e += stride) {
         double h[3] = {0.0, 0.0, 0.0};
         const double v = (double)tab.loop[e];  // zero past the last node
         const int j = e < n ? e : 0;
