@@ -341,7 +341,7 @@ __global__ __launch_bounds__(kSweepThreads) void k_sweep_product_bwd(SweepUnits 
     if (tid < V) {
         double x = 0.0;
         for (int q = 0; q < U.block_waves; ++q) x += s_sum[q][tid];
-        partials[(b * gridDim.x + blockIdx.x) * V + tid] = scale_by(x, sum_exponents(D, s_exp));
+        partials[(b * gridDim.x + blockIdx.x) * V + tid] = scale_by(x, sum_exponents(s_exp));
     }
 }
 

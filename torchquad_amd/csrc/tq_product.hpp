@@ -175,11 +175,14 @@ __device__ inline int factor_scale(int k, T x, double w, double ex, const Params
 }
 
 // Powers of two taken out of the axes: s_exp[k] of axis k, of the double
-// Gaussian's second component s_exp[TQ_MAX_DIM + k].
+// Gaussian's second component s_exp[TQ_MAX_DIM + k]; slots without an axis
+// count as 0, so that a sum reads them all at once (axis by axis it waits for
+// LDS d times: double Gaussian, 13^7 FP32 points, 16.2 us, 15.4 so).
 constexpr int kExpSlots = 2 * TQ_MAX_DIM;
-__device__ inline long long sum_exponents(int d, const int* s_exp) {
+__device__ inline long long sum_exponents(const int* s_exp) {
     long long e = 0;
-    for (int k = 0; k < d; ++k) e += exp_or_zero(s_exp[k]);
+#pragma unroll
+    for (int k = 0; k < TQ_MAX_DIM; ++k) e += exp_or_zero(s_exp[k]);
     return e;
 }
 __device__ inline double scale_by(double v, long long e) {
@@ -189,14 +192,15 @@ __device__ inline double scale_by(double v, long long e) {
 // A block's sum v with the powers of two put back that were taken out of its
 // axes.  A pole on every axis: NaN, as from a sum over 0 times infinity.
 __device__ inline double scale_back(int fam, double v, int d, const int* s_exp) {
-    long long e = sum_exponents(d, s_exp);
+    long long e = sum_exponents(s_exp);
     if (fam == TQ_FAM_DOUBLE_GAUSSIAN) {
-        const long long e2 = sum_exponents(d, s_exp + TQ_MAX_DIM);
+        const long long e2 = sum_exponents(s_exp + TQ_MAX_DIM);
         if (e2 > e) e = e2;
     }
     if (fam == TQ_FAM_PRODUCT_PEAK) {
         int poles = 0;
-        for (int k = 0; k < d; ++k) poles += s_exp[k] >= kPoleExp ? 1 : 0;
+#pragma unroll
+        for (int k = 0; k < TQ_MAX_DIM; ++k) poles += s_exp[k] >= kPoleExp ? 1 : 0;
         if (poles == d) return __longlong_as_double(0x7ff8000000000000ll);
     }
     return scale_by(v, e);
@@ -253,7 +257,7 @@ __device__ inline void build_axis_factors(int d, int n, int rule, const Axis* ax
         } else if constexpr (E == 2) {
             const int m2 = exp_or_zero(s_exp[TQ_MAX_DIM + nd.k]);
             // the first axis brings the components to the larger one's power of two
-            const double behind = nd.k == 0 ? (double)(sum_exponents(d, s_exp) - sum_exponents(d, s_exp + TQ_MAX_DIM)) : 0.0;
+            const double behind = nd.k == 0 ? (double)(sum_exponents(s_exp) - sum_exponents(s_exp + TQ_MAX_DIM)) : 0.0;
             v[0] = nd.w * exp2(nd.ex[0] - (double)m + fmin(behind, 0.0));
             v[1] = nd.w * exp2(nd.ex[1] - (double)m2 - fmax(behind, 0.0));
         } else {
