@@ -484,7 +484,7 @@ static int plan_reduce(const tq_grid_desc* g, long long S, int unit, ValuePlan& 
 // W(p), a stream of writes.  Waves write contiguous ranges of `span` values
 // (a multiple of 64 VEC), VEC per lane and store; a lane's values mostly
 // share their point, so its weight is formed when the point changes (1e6
-// values, d=4: 10.2 -> 7.6 us; [N, S] values were written one component at a
+// values, d=4: 10.2 -> 5.4 us; [N, S] values were written one component at a
 // time with lanes S elements apart).  One
 // more block (when grad_domain is asked for) forms d/d domain, which only
 // the scale depends on: -+ sum_s grad_out[s] out[s] / (b_k - a_k).

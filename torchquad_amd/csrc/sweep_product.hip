@@ -11,7 +11,7 @@
 // and the sum meets the tables of W h_i -- for the Gaussian peak of W r and
 // W r^2, from which the three follow (t = alpha r + gamma on an axis).
 //
-// 1024 Gaussian peaks of 32^4 FP32 points: forward 122 -> 32 us, backward
+// 1024 Gaussian peaks of 32^4 FP32 points: forward 122 -> 31 us, backward
 // 332 -> 62 us against one exponential per point (grad.hip, which keeps one
 // axis, axes too long for the tables and the oscillatory backward).
 #include "tq_grid_launch.hpp"
